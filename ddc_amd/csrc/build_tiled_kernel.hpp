@@ -33,7 +33,7 @@ using namespace tiled;
 // TMODE: 0 row table read from global memory (L2), 1 staged in LDS whole,
 // 2 staged in LDS one sweep's fields at a time (tables too large for 1)
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int TMODE, bool IC>
-__global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildView bv,
+__global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, BuildView bv,
                                                            const double* __restrict__ vals, Layout vl,
                                                            const double* __restrict__ dl,
                                                            const double* __restrict__ dr, Layout dlay,
@@ -46,6 +46,7 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
     constexpr int RSF = KF + (FDIV ? 1 : 0), RSB = KB + 1; // split records
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
+    __shared__ double b2s[kNbMax][LB];
     __shared__ double x2s[kNbMax][LB];
     __shared__ BorderLds bl;
     extern __shared__ double rt_lds[];
@@ -71,12 +72,12 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
     uint32_t const clo = uint32_t(cb - lay(cl, 0, line0));
     uint32_t const vrs = uint32_t(vl.rs), crs = uint32_t(cl.rs);
 
-    // dynamic LDS: the row table and the padded Q^-1 gamma blocks (TLDS),
+    // dynamic LDS: the row table and the Q^-1 gamma blocks (TLDS),
     // then the staging area, LB x stage_pitch(K * L) doubles, and the per-line
     // offsets of vals and coef (IC)
     int const tab = TMODE == 2 ? K * L * (RSF > RSB ? RSF : RSB) : K * L * RS; // doubles of the table region
     double* gpad = rt_lds + tab;
-    double* stg = rt_lds + (TLDS ? tab + tv.ngb * L * kNbMax : 0);
+    double* stg = rt_lds + (TLDS ? tab + tv.ngb * L * tv.nb : 0);
     uint32_t* loff = reinterpret_cast<uint32_t*>(stg + LB * SP);
     int const nl = int(min<int64_t>(LB, nbatch - line0));
 
@@ -124,20 +125,12 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
         }
     }
 
-    // the border rows' right-hand side does not depend on the sweeps: segment
-    // 0 loads it now, with the tile, and parks it in x2s (which it overwrites
-    // with the border solution later), so the border step does not wait on
-    // memory while the other waves wait at its barrier
-    if (tv.nb > 0 && seg == 0) {
-        int64_t const db = lay(dlay, 0, lc);
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k)
-            if (k < tv.nb)
-                x2s[k][ln] = active ? rhs_src(bv, vals, vl, vb, dl, dr, dlay, db, k < tv.top ? k : tv.nq + k) : 0.0;
-    }
-
-    // the segment's Q^-1 gamma block (-1: none), read before it is needed
-    int const gblk = tv.nb > 0 ? tv.gseg[seg] : -1;
+    // the border rows' right-hand side and the segment's part of the border
+    // step do not depend on the sweeps: read now, with the tile
+    double b2 = 0.0;
+    if (seg < tv.nb && active)
+        b2 = rhs_src(bv, vals, vl, vb, dl, dr, dlay, lay(dlay, 0, lc), seg < tv.top ? seg : tv.nq + seg);
+    SegBorder const sb = tv.seg[seg];
 
     // per-row table and border data: staged in LDS when they fit (one copy
     // per workgroup)
@@ -146,6 +139,7 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
         // backward sweep's, in the same LDS region
         stage_half<NT, KF, KB, FDIV, true>(tv.rt, RS, K * L, rt_lds, tid);
         stage_border<NT, true>(tv, bl, gpad, tid);
+        if (seg < tv.nb) b2s[seg][ln] = b2;
         __syncthreads();
         tiled_forward<LB, K, L, KF, FDIV, 0, KF>(y, rt_lds + r0 * RSF, RSF, tv, ex, seg, ln);
         stage_half<NT, KF, KB, FDIV, false>(tv.rt, RS, K * L, rt_lds, tid);
@@ -160,10 +154,12 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
             double2* dst = reinterpret_cast<double2*>(rt_lds);
             for (int idx = tid; idx < n2; idx += NT) dst[idx] = src[idx];
             stage_border<NT, true>(tv, bl, gpad, tid);
+            if (seg < tv.nb) b2s[seg][ln] = b2;
             __syncthreads();
             T = rt_lds + r0 * RS;
         } else {
-            stage_border<NT, false>(tv, bl, gpad, tid); // couplings only
+            stage_border<NT, false>(tv, bl, gpad, tid); // without the Q^-1 gamma blocks
+            if (seg < tv.nb) b2s[seg][ln] = b2;
             __syncthreads();
             T = tv.rt + size_t(r0) * RS;
         }
@@ -175,65 +171,25 @@ __global__ void __launch_bounds__(LB* K) build_tiled_kernel(TiledView tv, BuildV
     int const off = bv.offset;
     int const nbas = bv.nbasis;
     if (nb > 0) {
-        for (int z = 0; z < tv.bl_nnz; ++z) {
-            int const c = bl.c[z];
-            if (c >= r0 && c < r0 + L) {
-                double v = 0.0;
-#pragma unroll
-                for (int i = 0; i < L; ++i)
-                    if (r0 + i == c) v = y[i];
-                lamx[z][ln] = v;
-            }
-        }
+        gather_coupled<LB, L>(y, sb, lamx, ln);
         __syncthreads();
-        if (seg == 0) {
-            double b2[kNbMax];
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) b2[k] = k < nb ? x2s[k][ln] : 0.0;
-            for (int z = 0; z < tv.bl_nnz; ++z) {
-                int const r = bl.r[z];
-                double const v = bl.v[z] * lamx[z][ln];
-#pragma unroll
-                for (int k = 0; k < kNbMax; ++k)
-                    if (k == r) b2[k] -= v;
-            }
-            getrs_small(nb, tv.s_lu, tv.s_ipiv, b2);
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) {
-                if (k < nb) {
-                    x2s[k][ln] = b2[k];
-                    if (active) {
-                        int const prow = k < tv.top ? k : nq + k;
-                        coef[cb + int64_t(prow + off) * cl.rs] = b2[k];
-                        if (bv.periodic) {
-                            int const j0 = prow + off - nbas;
-                            if (j0 >= 0) coef[cb + int64_t(j0) * cl.rs] = b2[k];
-                            int const j2 = prow + off + nbas;
-                            if (j2 < nbas + bv.degree) coef[cb + int64_t(j2) * cl.rs] = b2[k];
-                        }
-                    }
+        if (seg < nb) {
+            double const x2 = border_row<LB>(tv, bl, b2s, lamx, seg, ln);
+            x2s[seg][ln] = x2;
+            if (active) {
+                int const j = (seg < tv.top ? seg : nq + seg) + off;
+                coef[cb + int64_t(j) * cl.rs] = x2;
+                if (bv.periodic) {
+                    if (j - nbas >= 0) coef[cb + int64_t(j - nbas) * cl.rs] = x2;
+                    if (j + nbas < nbas + bv.degree) coef[cb + int64_t(j + nbas) * cl.rs] = x2;
                 }
             }
         }
         __syncthreads();
-        if (gblk >= 0) { // Q^-1 gamma is nonzero only in the segments near the block ends
-            double x2[kNbMax];
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) x2[k] = k < nb ? x2s[k][ln] : 0.0;
-            if constexpr (TLDS) {
-                apply_gamma<L>(y, gpad + gblk * L * kNbMax, x2);
-            } else {
-                const double* Gb = tv.Gblk + size_t(gblk) * L * nb;
-#pragma unroll
-                for (int i = 0; i < L; ++i) {
-                    double t = y[i];
-#pragma unroll
-                    for (int k = 0; k < kNbMax; ++k)
-                        if (k < nb) t = fma(-Gb[i * nb + k], x2[k], t);
-                    y[i] = t;
-                    chunk_fence(i);
-                }
-            }
+        // Q^-1 gamma is nonzero only in the segments near the block ends
+        if (sb.gblk >= 0) {
+            if constexpr (TLDS) apply_gamma<LB>(y, gpad + sb.gblk * L * nb, nb, x2s, ln);
+            else apply_gamma<LB>(y, tv.Gblk + size_t(sb.gblk) * L * nb, nb, x2s, ln);
         }
     }
 
@@ -309,7 +265,7 @@ void launch_cfg(BuilderPlan const& p, double* coef, Layout cl, const double* val
     constexpr int LB = NT / K;
     constexpr int KE = KF > KB ? KF : KB;
     constexpr size_t static_lds =
-        size_t(KE * K * LB + kLamMax * LB + kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+        size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     bool const ic = vl.rs == 1 && cl.rs == 1;
     size_t const stage = ic ? size_t(LB) * stage_pitch(K * L) * sizeof(double) + 2 * LB * sizeof(uint32_t) : 0;
     constexpr int RSH = (KF + (FDIV ? 1 : 0)) > (KB + 1) ? (KF + (FDIV ? 1 : 0)) : (KB + 1);

@@ -7,8 +7,8 @@
 //      folded gradient of the border rows;
 //   2. b2 -= (Q^-1 gamma)^T y: partial sums of the segments that hold Q^-1
 //      gamma blocks, combined in segment order by one thread per line;
-//   3. b2 = S^-T b2 (Schur complement LU, transposed);
-//   4. y -= lambda^T b2;
+//   3. x2 = S^-T b2 (the inverse of the Schur complement, transposed);
+//   4. y -= lambda^T x2;
 //   5. y = Q^-T y with the tiled sweeps (transposed tables);
 //   6. the rows back to the value and Hermite-derivative gradients.
 #include "tiled_common.hpp"
@@ -19,47 +19,22 @@ namespace {
 
 using namespace tiled;
 
-// dgetrs('T') on an nb x nb LU (nb <= kNbMax) held in registers
-__device__ __forceinline__ void getrs_trans_small(int nb, const double* a, const int* ipiv, double* b)
+// One segment's part of (Q^-1 gamma)^T y, a column of the block G per row of
+// part (the loops as in apply_gamma).
+template <int LB, int L>
+__device__ __forceinline__ void gamma_trans(double const (&y)[L], const double* G, int nb, double (*part)[LB], int ln)
 {
+    for (int k = 0; k < nb; ++k) {
+        const double* g = G + k * L;
+        double acc = 0.0;
 #pragma unroll
-    for (int j = 0; j < kNbMax; ++j) {
-        if (j < nb) {
-            double t = b[j];
-#pragma unroll
-            for (int i = 0; i < j; ++i) t = t - a[i * nb + j] * b[i];
-            b[j] = t / a[j * nb + j];
-        }
-    }
-#pragma unroll
-    for (int j = kNbMax - 1; j >= 0; --j) {
-        if (j < nb) {
-            double t = b[j];
-#pragma unroll
-            for (int i = j + 1; i < kNbMax; ++i)
-                if (i < nb) t = t - a[i * nb + j] * b[i];
-            b[j] = t;
-        }
-    }
-#pragma unroll
-    for (int j = kNbMax - 1; j >= 0; --j) {
-        if (j < nb) {
-            int const p = ipiv[j];
-            double bp = 0.0;
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k)
-                if (k == p) bp = b[k];
-            double const bj = b[j];
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k)
-                if (k == p) b[k] = bj;
-            b[j] = bp;
-        }
+        for (int i = 0; i < L; ++i) acc = fma(g[i], y[i], acc);
+        part[k][ln] = acc;
     }
 }
 
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, bool TLDS, bool IC>
-__global__ void __launch_bounds__(LB* K) build_vjp_tiled_kernel(TiledView tv, BuildView bv,
+__global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv, BuildView bv,
                                                                const double* __restrict__ gcoef, Layout cl,
                                                                double* __restrict__ gvals, Layout vl,
                                                                double* __restrict__ gdl, double* __restrict__ gdr,
@@ -70,6 +45,7 @@ __global__ void __launch_bounds__(LB* K) build_vjp_tiled_kernel(TiledView tv, Bu
     constexpr int SR = stage_rows(K * L), SP = stage_pitch(K * L); // staging chunk rows, pitch (IC)
     __shared__ double ex[KE][K][LB];
     __shared__ double part[kMaxGBlocksVjp][kNbMax][LB];
+    __shared__ double b2s[kNbMax][LB];
     __shared__ double x2s[kNbMax][LB];
     __shared__ BorderLds bl;
     extern __shared__ double rt_lds[];
@@ -93,11 +69,11 @@ __global__ void __launch_bounds__(LB* K) build_vjp_tiled_kernel(TiledView tv, Bu
     uint32_t const vlo = uint32_t(vb - lay(vl, 0, line0)) + uint32_t(tv.q0 + r0) * uint32_t(vl.rs);
     uint32_t const crs = uint32_t(cl.rs), vrs = uint32_t(vl.rs);
 
-    // dynamic LDS: the row table and the padded Q^-1 gamma blocks (TLDS),
+    // dynamic LDS: the row table and the Q^-1 gamma blocks (TLDS),
     // then the staging area (IC), LB x stage_pitch(K * L) doubles, and the per-line
     // offsets of gcoef and gvals
     double* gpad = rt_lds + K * L * RS;
-    double* stg = rt_lds + (TLDS ? K * L * RS + tv.ngb * L * kNbMax : 0);
+    double* stg = rt_lds + (TLDS ? K * L * RS + tv.ngb * L * nb : 0);
     uint32_t* loff = reinterpret_cast<uint32_t*>(stg + LB * SP);
     int const nl = int(min<int64_t>(LB, nbatch - line0));
     if constexpr (IC) {
@@ -161,25 +137,19 @@ __global__ void __launch_bounds__(LB* K) build_vjp_tiled_kernel(TiledView tv, Bu
         }
     }
 
-    // the border rows' incoming gradient (folded like the main rows), read
-    // now and parked in x2s, which segment 0 overwrites with x2 later
-    if (nb > 0 && seg == 0) {
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k) {
-            if (k < nb) {
-                int const j1 = (k < top ? k : nq + k) + off;
-                double v = active ? gcoef[cb + int64_t(j1) * cl.rs] : 0.0;
-                if (active && bv.periodic) {
-                    if (j1 - nbas >= 0) v += gcoef[cb + int64_t(j1 - nbas) * cl.rs];
-                    if (j1 + nbas < nsz) v += gcoef[cb + int64_t(j1 + nbas) * cl.rs];
-                }
-                x2s[k][ln] = v;
-            }
+    // the border rows' incoming gradient, folded like the main rows
+    double b2 = 0.0;
+    if (seg < nb && active) {
+        int const j1 = (seg < top ? seg : nq + seg) + off;
+        b2 = gcoef[cb + int64_t(j1) * cl.rs];
+        if (bv.periodic) {
+            if (j1 - nbas >= 0) b2 += gcoef[cb + int64_t(j1 - nbas) * cl.rs];
+            if (j1 + nbas < nsz) b2 += gcoef[cb + int64_t(j1 + nbas) * cl.rs];
         }
     }
+    SegBorder const sb = tv.seg[seg];
 
     // per-row table and border data in LDS when they fit
-    int const gblk = nb > 0 ? tv.gseg[seg] : -1;
     const double* T;
     if constexpr (TLDS) {
         int const n2 = (K * L * RS) / 2;
@@ -190,87 +160,56 @@ __global__ void __launch_bounds__(LB* K) build_vjp_tiled_kernel(TiledView tv, Bu
         __syncthreads();
         T = rt_lds + r0 * RS;
     } else {
-        stage_border<NT, false>(tv, bl, gpad, tid); // couplings only
+        stage_border<NT, false>(tv, bl, gpad, tid); // without the Q^-1 gamma blocks
         T = tv.rt + size_t(r0) * RS;
     }
 
     // 2. partial sums of (Q^-1 gamma)^T y over this segment's rows
-    if (gblk >= 0) {
-        if constexpr (TLDS) {
-            // padded columns (k >= nb) sum to zero and are never read
-            const double* Gb = gpad + gblk * L * kNbMax;
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) {
-                double acc = 0.0;
-#pragma unroll
-                for (int i = 0; i < L; ++i) acc = fma(Gb[i * kNbMax + k], y[i], acc);
-                part[gblk][k][ln] = acc;
-            }
-        } else {
-            const double* Gb = tv.Gblk + size_t(gblk) * L * nb;
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) {
-                if (k < nb) {
-                    double acc = 0.0;
-#pragma unroll
-                    for (int i = 0; i < L; ++i) acc = fma(Gb[i * nb + k], y[i], acc);
-                    part[gblk][k][ln] = acc;
-                }
-            }
-        }
+    if (sb.gblk >= 0) {
+        if constexpr (TLDS) gamma_trans<LB>(y, gpad + sb.gblk * L * nb, nb, part[sb.gblk], ln);
+        else gamma_trans<LB>(y, tv.Gblk + size_t(sb.gblk) * L * nb, nb, part[sb.gblk], ln);
     }
+    if (seg < nb) b2s[seg][ln] = b2;
     __syncthreads();
 
-    // 3. the border: b2 -= sum of the partials (segment order), b2 = S^-T b2
-    if (seg == 0) {
-        double b2[kNbMax];
-        int const nblk = tv.ngb;
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k) {
-            if (k < nb) {
-                double v = x2s[k][ln];
-                for (int g = 0; g < nblk; ++g) v -= part[g][k][ln];
-                b2[k] = v;
-            } else {
-                b2[k] = 0.0;
-            }
+    // 3. the border: b2 -= sum of the partials (segment order), x2 = S^-T b2;
+    // every border row's thread sums the whole right-hand side for its own
+    // row of the product
+    if (seg < nb) {
+        double x2 = 0.0;
+        for (int j = 0; j < nb; ++j) {
+            double v = b2s[j][ln];
+            for (int g = 0; g < tv.ngb; ++g) v -= part[g][j][ln];
+            x2 = fma(bl.sinv[seg * nb + j], v, x2);
         }
-        if (nb > 0) getrs_trans_small(nb, tv.s_lu, tv.s_ipiv, b2);
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k)
-            if (k < nb) x2s[k][ln] = b2[k];
+        x2s[seg][ln] = x2;
         // 6 (border part). rows back to the gradients they came from
         if (active) {
             int64_t const db = lay(dlay, 0, lc);
             int const nv_end = nbas - bv.nbe_r;
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) {
-                if (k < nb) {
-                    int const i = k < top ? k : nq + k;
-                    if (bv.periodic) {
-                        gvals[vb + int64_t(i) * vl.rs] = b2[k];
-                    } else if (i < bv.nbe_l) {
-                        if (bv.bcl == DDCX_HERMITE) gdl[db + int64_t(i) * dlay.rs] = b2[k] * bv.dxpow[i + bv.odd];
-                    } else if (i < nv_end) {
-                        gvals[vb + int64_t(i - bv.nbe_l) * vl.rs] = b2[k];
-                    } else if (bv.bcu == DDCX_HERMITE) {
-                        gdr[db + int64_t(i - nv_end) * dlay.rs] = b2[k] * bv.dxpow[i - nv_end + bv.odd];
-                    }
-                }
+            int const i = seg < top ? seg : nq + seg;
+            if (bv.periodic) {
+                gvals[vb + int64_t(i) * vl.rs] = x2;
+            } else if (i < bv.nbe_l) {
+                if (bv.bcl == DDCX_HERMITE) gdl[db + int64_t(i) * dlay.rs] = x2 * bv.dxpow[i + bv.odd];
+            } else if (i < nv_end) {
+                gvals[vb + int64_t(i - bv.nbe_l) * vl.rs] = x2;
+            } else if (bv.bcu == DDCX_HERMITE) {
+                gdr[db + int64_t(i - nv_end) * dlay.rs] = x2 * bv.dxpow[i - nv_end + bv.odd];
             }
         }
     }
     __syncthreads();
 
-    // 4. y -= lambda^T x2
-    for (int z = 0; z < tv.bl_nnz; ++z) {
-        int const c = bl.c[z];
-        if (c >= r0 && c < r0 + L) {
-            double const v = bl.v[z] * x2s[bl.r[z]][ln];
+    // 4. y -= lambda^T x2, in the segments that hold coupled rows
+    if (sb.mask != 0) {
 #pragma unroll
-            for (int i = 0; i < L; ++i)
-                if (r0 + i == c) y[i] -= v;
-        }
+        for (int i = 0; i < L; ++i)
+            if ((sb.mask >> i) & 1u) {
+                int const g = sb.slot0 + __popc(sb.mask & ((1u << i) - 1u));
+                int const z1 = bl.p[g + 1];
+                for (int z = bl.p[g]; z < z1; ++z) y[i] = fma(-bl.v[z], x2s[bl.i[z]][ln], y[i]);
+            }
     }
 
     // 5. y = Q^-T y
@@ -316,7 +255,7 @@ void launch_cfg(BuilderPlan const& p, const double* gcoef, Layout cl, double* gv
     constexpr int LB = NT / K;
     constexpr int KE = KF > KB ? KF : KB;
     constexpr size_t static_lds =
-        size_t(KE * K * LB + kMaxGBlocksVjp * kNbMax * LB + kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+        size_t(KE * K * LB + kMaxGBlocksVjp * kNbMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     size_t const table = (size_t(K) * L * p.tiled_t.rs + gamma_lds_doubles(p.tview_t)) * sizeof(double);
     bool const ic = vl.rs == 1 && cl.rs == 1;
     size_t const stage = ic ? size_t(LB) * stage_pitch(K * L) * sizeof(double) + 2 * LB * sizeof(uint32_t) : 0;

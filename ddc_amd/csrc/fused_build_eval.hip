@@ -16,7 +16,7 @@ namespace {
 using namespace tiled;
 
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int D>
-__global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, BuildView bv, BSplinesView b,
+__global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv, BuildView bv, BSplinesView b,
                                                                 Rules1D rules, const double* __restrict__ vals,
                                                                 Layout vl, const double* __restrict__ dl,
                                                                 const double* __restrict__ dr, Layout dlay,
@@ -33,9 +33,10 @@ __global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, B
     constexpr int U = 8;
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
+    __shared__ double b2s[kNbMax][LB];
     __shared__ double x2s[kNbMax][LB];
     __shared__ BorderLds bl;
-    // row table and padded Q^-1 gamma blocks during the build, coefficient
+    // row table and Q^-1 gamma blocks during the build, coefficient
     // tile (size x LB) after
     extern __shared__ double dyn[];
 
@@ -69,16 +70,12 @@ __global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, B
             y[i] = r0 + i < nq ? v : 0.0;
         }
     }
-    // the border rows' right-hand side, loaded with the tile and parked in
-    // x2s (segment 0 overwrites it with the border solution later)
-    if (tv.nb > 0 && seg == 0) {
-        int64_t const db = lay(dlay, 0, lc);
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k)
-            if (k < tv.nb)
-                x2s[k][ln] = active ? rhs_src(bv, vals, vl, vb, dl, dr, dlay, db, k < tv.top ? k : nq + k) : 0.0;
-    }
-    int const gblk = tv.nb > 0 ? tv.gseg[seg] : -1; // Q^-1 gamma block (-1: none)
+    // the border rows' right-hand side and the segment's part of the border
+    // step, read with the tile
+    double b2 = 0.0;
+    if (seg < tv.nb && active)
+        b2 = rhs_src(bv, vals, vl, vb, dl, dr, dlay, lay(dlay, 0, lc), seg < tv.top ? seg : tv.nq + seg);
+    SegBorder const sb = tv.seg[seg];
     double* const gpad = dyn + K * L * RS;
     {
         int const n2 = (K * L * RS) / 2;
@@ -86,6 +83,7 @@ __global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, B
         double2* dst = reinterpret_cast<double2*>(dyn);
         for (int idx = tid; idx < n2; idx += NT) dst[idx] = src[idx];
         stage_border<NT, true>(tv, bl, gpad, tid);
+        if (seg < tv.nb) b2s[seg][ln] = b2;
         __syncthreads();
     }
     tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, dyn + r0 * RS, RS, tv, ex, seg, ln);
@@ -94,40 +92,11 @@ __global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, B
     int const off = bv.offset;
     int const nbas = bv.nbasis;
     if (nb > 0) {
-        for (int z = 0; z < tv.bl_nnz; ++z) {
-            int const c = bl.c[z];
-            if (c >= r0 && c < r0 + L) {
-                double v = 0.0;
-#pragma unroll
-                for (int i = 0; i < L; ++i)
-                    if (r0 + i == c) v = y[i];
-                lamx[z][ln] = v;
-            }
-        }
+        gather_coupled<LB, L>(y, sb, lamx, ln);
         __syncthreads();
-        if (seg == 0) {
-            double b2[kNbMax];
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) b2[k] = k < nb ? x2s[k][ln] : 0.0;
-            for (int z = 0; z < tv.bl_nnz; ++z) {
-                int const r = bl.r[z];
-                double const v = bl.v[z] * lamx[z][ln];
-#pragma unroll
-                for (int k = 0; k < kNbMax; ++k)
-                    if (k == r) b2[k] -= v;
-            }
-            getrs_small(nb, tv.s_lu, tv.s_ipiv, b2);
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k)
-                if (k < nb) x2s[k][ln] = b2[k];
-        }
+        if (seg < nb) x2s[seg][ln] = border_row<LB>(tv, bl, b2s, lamx, seg, ln);
         __syncthreads();
-        if (gblk >= 0) {
-            double x2[kNbMax];
-#pragma unroll
-            for (int k = 0; k < kNbMax; ++k) x2[k] = k < nb ? x2s[k][ln] : 0.0;
-            apply_gamma<L>(y, gpad + gblk * L * kNbMax, x2);
-        }
+        if (sb.gblk >= 0) apply_gamma<LB>(y, gpad + sb.gblk * L * nb, nb, x2s, ln);
     }
     __syncthreads(); // the row table is dead from here on
 
@@ -148,18 +117,13 @@ __global__ void __launch_bounds__(LB* K) fused_build_eval_kernel(TiledView tv, B
             }
         }
     }
-    if (seg == 0) {
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k) {
-            if (k < nb) {
-                double const v = x2s[k][ln];
-                int const prow = k < tv.top ? k : nq + k;
-                put(prow + off, v);
-                if (bv.periodic) {
-                    if (prow + off - nbas >= 0) put(prow + off - nbas, v);
-                    if (prow + off + nbas < nbas + bv.degree) put(prow + off + nbas, v);
-                }
-            }
+    if (seg < nb) {
+        double const v = x2s[seg][ln];
+        int const j = (seg < tv.top ? seg : nq + seg) + off;
+        put(j, v);
+        if (bv.periodic) {
+            if (j - nbas >= 0) put(j - nbas, v);
+            if (j + nbas < nbas + bv.degree) put(j + nbas, v);
         }
     }
     __syncthreads();
@@ -277,7 +241,7 @@ bool launch_build_eval_fused(BuilderPlan const& p, BSplinesPlan const& bs, Rules
     TiledHost const& t = p.tiled_f;
     if (!t.ok || p.bs.get() != &bs) return false;
     if (feet_shift && npts != int64_t(p.points.size())) return false;
-    const double* const fpts = feet_shift ? p.d_points.as<double>() : nullptr;
+    const double* const fpts = feet_shift ? p.d_points : nullptr;
     if (vl.rs == 1 || pl.rs == 1 || (coef && cl.rs == 1)) return false; // batch-contiguous layouts only
     int const K = t.K, L = t.L, LB = 1024 / K;
     if (L != 16 || (K != 64 && K != 128)) return false;
@@ -288,7 +252,7 @@ bool launch_build_eval_fused(BuilderPlan const& p, BSplinesPlan const& bs, Rules
     size_t const tile = size_t(bs.size()) * LB * sizeof(double);
     size_t const lds = std::max(table, tile);
     int const KE = std::max(t.kf, t.kb);
-    size_t const stat = size_t(KE * K * LB + kLamMax * LB + kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+    size_t const stat = size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     if (lds + stat > size_t(160 * 1024)) return false;
     BSplinesView const b = bs.device_view();
     if (K == 64)

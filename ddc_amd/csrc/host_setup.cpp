@@ -618,26 +618,20 @@ void SolveBuffers::upload(HostProblem const& pr, SolveView& sv)
     sv.top = pr.top;
     sv.tr_nnz = int(pr.tr_v.size());
     sv.bl_nnz = int(pr.bl_v.size());
-    q.upload(pr.q.q);
-    ipiv.upload(pr.q.ipiv);
-    slu.upload(pr.schur.q);
-    sipiv.upload(pr.schur.ipiv);
-    trr.upload(pr.tr_r);
-    trc.upload(pr.tr_c);
-    trv.upload(pr.tr_v);
-    blr.upload(pr.bl_r);
-    blc.upload(pr.bl_c);
-    blv.upload(pr.bl_v);
-    sv.q = q.as<double>();
-    sv.ipiv = ipiv.as<int>();
-    sv.s_lu = slu.as<double>();
-    sv.s_ipiv = sipiv.as<int>();
-    sv.tr_r = trr.as<int>();
-    sv.tr_c = trc.as<int>();
-    sv.tr_v = trv.as<double>();
-    sv.bl_r = blr.as<int>();
-    sv.bl_c = blc.as<int>();
-    sv.bl_v = blv.as<double>();
+    size_t const q = pack.add(pr.q.q), ipiv = pack.add(pr.q.ipiv), slu = pack.add(pr.schur.q),
+                 sipiv = pack.add(pr.schur.ipiv), trr = pack.add(pr.tr_r), trc = pack.add(pr.tr_c),
+                 trv = pack.add(pr.tr_v), blr = pack.add(pr.bl_r), blc = pack.add(pr.bl_c), blv = pack.add(pr.bl_v);
+    pack.upload();
+    sv.q = pack.at<double>(q);
+    sv.ipiv = pack.at<int>(ipiv);
+    sv.s_lu = pack.at<double>(slu);
+    sv.s_ipiv = pack.at<int>(sipiv);
+    sv.tr_r = pack.at<int>(trr);
+    sv.tr_c = pack.at<int>(trc);
+    sv.tr_v = pack.at<double>(trv);
+    sv.bl_r = pack.at<int>(blr);
+    sv.bl_c = pack.at<int>(blc);
+    sv.bl_v = pack.at<double>(blv);
 }
 
 void BuilderPlan::ensure_device() const
@@ -648,151 +642,95 @@ void BuilderPlan::ensure_device() const
 
 void BuilderPlan::upload()
 {
-    {
-        d_solve.upload(prob, view.sv);
-        d_points.upload(points);
-        SolveView& sv = view.sv;
-        if (tiled.ok) {
-            t_Mf.upload(tiled.Mf);
-            t_Mb.upload(tiled.Mb);
-            t_rt.upload(tiled.rt);
-            t_gseg.upload(tiled.gseg);
-            t_Gblk.upload(tiled.Gblk);
-            TiledView& tv = tview;
-            tv.K = tiled.K;
-            tv.L = tiled.L;
-            tv.kf = tiled.kf;
-            tv.kb = tiled.kb;
-            tv.wf = tiled.wf;
-            tv.wb = tiled.wb;
-            tv.nq = prob.q.n;
-            tv.nb = prob.nb();
-            tv.top = prob.top;
-            tv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
-            tv.bl_nnz = int(prob.bl_v.size());
-            tv.rs = tiled.rs;
-            tv.ngb = tv.nb > 0 ? int(tiled.Gblk.size() / (size_t(tiled.L) * tv.nb)) : 0;
-            tv.rt = t_rt.as<double>();
-            tv.Mf = t_Mf.as<double>();
-            tv.Mb = t_Mb.as<double>();
-            tv.gseg = t_gseg.as<int>();
-            tv.Gblk = t_Gblk.as<double>();
-            tv.bl_r = sv.bl_r;
-            tv.bl_c = sv.bl_c;
-            tv.bl_v = sv.bl_v;
-            tv.s_lu = sv.s_lu;
-            tv.s_ipiv = sv.s_ipiv;
-        }
-        auto view_of = [&](TiledHost const& th, DeviceBuffer& mf, DeviceBuffer& mb, DeviceBuffer& rt,
-                           DeviceBuffer& gs, DeviceBuffer& gb, TiledView& tv) {
-            mf.upload(th.Mf);
-            mb.upload(th.Mb);
-            rt.upload(th.rt);
-            gs.upload(th.gseg);
-            gb.upload(th.Gblk);
-            tv.K = th.K;
-            tv.L = th.L;
-            tv.kf = th.kf;
-            tv.kb = th.kb;
-            tv.wf = th.wf;
-            tv.wb = th.wb;
-            tv.nq = prob.q.n;
-            tv.nb = prob.nb();
-            tv.top = prob.top;
-            tv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
-            tv.bl_nnz = int(prob.bl_v.size());
-            tv.rs = th.rs;
-            tv.ngb = tv.nb > 0 ? int(th.Gblk.size() / (size_t(th.L) * tv.nb)) : 0;
-            tv.rt = rt.as<double>();
-            tv.Mf = mf.as<double>();
-            tv.Mb = mb.as<double>();
-            tv.gseg = gs.as<int>();
-            tv.Gblk = gb.as<double>();
-            tv.bl_r = sv.bl_r;
-            tv.bl_c = sv.bl_c;
-            tv.bl_v = sv.bl_v;
-            tv.s_lu = sv.s_lu;
-            tv.s_ipiv = sv.s_ipiv;
-        };
-        if (tiled_f.ok) view_of(tiled_f, tf_Mf, tf_Mb, tf_rt, tf_gseg, tf_Gblk, tview_f);
-        if (tiled_t.ok) {
-            tt_Mf.upload(tiled_t.Mf);
-            tt_Mb.upload(tiled_t.Mb);
-            tt_rt.upload(tiled_t.rt);
-            tt_gseg.upload(tiled_t.gseg);
-            tt_Gblk.upload(tiled_t.Gblk);
-            TiledView& tv = tview_t;
-            tv = tview; // sizes and border data are those of the solve
-            tv.K = tiled_t.K;
-            tv.L = tiled_t.L;
-            tv.kf = tiled_t.kf;
-            tv.kb = tiled_t.kb;
-            tv.wf = tiled_t.wf;
-            tv.wb = tiled_t.wb;
-            tv.nq = prob.q.n;
-            tv.nb = prob.nb();
-            tv.top = prob.top;
-            tv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
-            tv.bl_nnz = int(prob.bl_v.size());
-            tv.rs = tiled_t.rs;
-            tv.ngb = tv.nb > 0 ? int(tiled_t.Gblk.size() / (size_t(tiled_t.L) * tv.nb)) : 0;
-            tv.rt = tt_rt.as<double>();
-            tv.Mf = tt_Mf.as<double>();
-            tv.Mb = tt_Mb.as<double>();
-            tv.gseg = tt_gseg.as<int>();
-            tv.Gblk = tt_Gblk.as<double>();
-            tv.bl_r = sv.bl_r;
-            tv.bl_c = sv.bl_c;
-            tv.bl_v = sv.bl_v;
-            tv.s_lu = sv.s_lu;
-            tv.s_ipiv = sv.s_ipiv;
-        }
-        if (refine.ok) {
-            RefineHost const& R = refine;
-            r_rt.upload(R.rt32);
-            r_Mf.upload(R.Mf32);
-            r_Mb.upload(R.Mb32);
-            r_gseg_blk.upload(R.t.gseg);
-            r_Gblk.upload(R.Gblk32);
-            r_rq.upload(R.rq);
-            r_gr.upload(R.gam_r);
-            r_gc.upload(R.gam_c);
-            r_gv.upload(R.gam_v);
-            r_gamseg.upload(R.gam_seg);
-            r_delta.upload(R.delta);
-            RefineView& rv = rview;
-            rv.K = R.t.K;
-            rv.L = R.t.L;
-            rv.kf = R.t.kf;
-            rv.kb = R.t.kb;
-            rv.wf = R.t.wf;
-            rv.wb = R.t.wb;
-            rv.nq = prob.q.n;
-            rv.nb = prob.nb();
-            rv.top = prob.top;
-            rv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
-            rv.bl_nnz = int(prob.bl_v.size());
-            rv.rs = R.rs;
-            rv.kq = R.kq;
-            rv.steps = R.steps;
-            rv.shift = R.shift;
-            rv.rt = r_rt.as<float>();
-            rv.Mf = r_Mf.as<float>();
-            rv.Mb = r_Mb.as<float>();
-            rv.gseg = r_gseg_blk.as<int>();
-            rv.Gblk = r_Gblk.as<float>();
-            rv.rq = r_rq.as<double>();
-            rv.gam_r = r_gr.as<int>();
-            rv.gam_c = r_gc.as<int>();
-            rv.gam_v = r_gv.as<double>();
-            rv.gam_seg = r_gamseg.as<int>();
-            rv.delta = r_delta.as<double>();
-            rv.bl_r = sv.bl_r;
-            rv.bl_c = sv.bl_c;
-            rv.bl_v = sv.bl_v;
-            rv.s_lu = sv.s_lu;
-            rv.s_ipiv = sv.s_ipiv;
-        }
+    d_solve.upload(prob, view.sv);
+    SolveView const& sv = view.sv;
+    int const nb = prob.nb();
+    size_t const at_points = pack.add(points);
+    size_t const slot = pack.add(border.slot), rowp = pack.add(border.rowp), val = pack.add(border.val),
+                 crow = pack.add(border.crow), colp = pack.add(border.colp), cval = pack.add(border.cval),
+                 sinv = pack.add(border.sinv), sinvt = pack.add(border.sinvt);
+    struct Places {
+        size_t Mf, Mb, rt, seg, Gblk;
+    };
+    auto add_tiled = [&](TiledHost const& th) {
+        if (!th.ok) return Places{};
+        // the Q^-1 gamma blocks column by column
+        std::vector<double> cols(th.Gblk.size());
+        for (size_t r = 0; r * nb < th.Gblk.size(); ++r)
+            for (int c = 0; c < nb; ++c) cols[(r / th.L * nb + c) * th.L + r % th.L] = th.Gblk[r * nb + c];
+        return Places{pack.add(th.Mf), pack.add(th.Mb), pack.add(th.rt), pack.add(segment_borders(th, border)),
+                      pack.add(cols)};
+    };
+    Places const p = add_tiled(tiled), p_f = add_tiled(tiled_f), p_t = add_tiled(tiled_t);
+    RefineHost const& R = refine;
+    size_t const r_rt = pack.add(R.rt32), r_Mf = pack.add(R.Mf32), r_Mb = pack.add(R.Mb32),
+                 r_gseg = pack.add(R.t.gseg), r_Gblk = pack.add(R.Gblk32), r_rq = pack.add(R.rq),
+                 r_gr = pack.add(R.gam_r), r_gc = pack.add(R.gam_c), r_gv = pack.add(R.gam_v),
+                 r_gamseg = pack.add(R.gam_seg), r_delta = pack.add(R.delta);
+    pack.upload();
+    d_points = pack.at<double>(at_points);
+    auto view_of = [&](TiledHost const& th, Places const& at, bool transpose, TiledView& tv) {
+        if (!th.ok) return;
+        tv.K = th.K;
+        tv.L = th.L;
+        tv.kf = th.kf;
+        tv.kb = th.kb;
+        tv.wf = th.wf;
+        tv.wb = th.wb;
+        tv.nq = prob.q.n;
+        tv.nb = nb;
+        tv.top = prob.top;
+        tv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
+        tv.rs = th.rs;
+        tv.ngb = nb > 0 ? int(th.Gblk.size() / (size_t(th.L) * nb)) : 0;
+        tv.rt = pack.at<double>(at.rt);
+        tv.Mf = pack.at<double>(at.Mf);
+        tv.Mb = pack.at<double>(at.Mb);
+        tv.seg = pack.at<SegBorder>(at.seg);
+        tv.Gblk = pack.at<double>(at.Gblk);
+        tv.nnz = int(border.val.size());
+        tv.ngroup = transpose ? int(border.cols.size()) : nb;
+        tv.bi = pack.at<int>(transpose ? crow : slot);
+        tv.bv = pack.at<double>(transpose ? cval : val);
+        tv.bp = pack.at<int>(transpose ? colp : rowp);
+        tv.sinv = pack.at<double>(transpose ? sinvt : sinv);
+    };
+    view_of(tiled, p, false, tview);
+    view_of(tiled_f, p_f, false, tview_f);
+    view_of(tiled_t, p_t, true, tview_t);
+    if (refine.ok) {
+        RefineView& rv = rview;
+        rv.K = R.t.K;
+        rv.L = R.t.L;
+        rv.kf = R.t.kf;
+        rv.kb = R.t.kb;
+        rv.wf = R.t.wf;
+        rv.wb = R.t.wb;
+        rv.nq = prob.q.n;
+        rv.nb = nb;
+        rv.top = prob.top;
+        rv.q0 = bs->view.periodic ? 0 : prob.top - nbe_l;
+        rv.bl_nnz = int(prob.bl_v.size());
+        rv.rs = R.rs;
+        rv.kq = R.kq;
+        rv.steps = R.steps;
+        rv.shift = R.shift;
+        rv.rt = pack.at<float>(r_rt);
+        rv.Mf = pack.at<float>(r_Mf);
+        rv.Mb = pack.at<float>(r_Mb);
+        rv.gseg = pack.at<int>(r_gseg);
+        rv.Gblk = pack.at<float>(r_Gblk);
+        rv.rq = pack.at<double>(r_rq);
+        rv.gam_r = pack.at<int>(r_gr);
+        rv.gam_c = pack.at<int>(r_gc);
+        rv.gam_v = pack.at<double>(r_gv);
+        rv.gam_seg = pack.at<int>(r_gamseg);
+        rv.delta = pack.at<double>(r_delta);
+        rv.bl_r = sv.bl_r;
+        rv.bl_c = sv.bl_c;
+        rv.bl_v = sv.bl_v;
+        rv.s_lu = sv.s_lu;
+        rv.s_ipiv = sv.s_ipiv;
     }
     on_device = true;
 }

@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -43,6 +44,32 @@ struct DeviceBuffer {
     T* as() const
     {
         return static_cast<T*>(ptr);
+    }
+};
+
+// Host arrays gathered into one device allocation, each 256-byte aligned: a
+// plan's tables cost one allocation and one copy instead of one of each per
+// array.  add() returns the array's place, valid in at() after upload().
+struct DevicePack {
+    DeviceBuffer buf;
+    std::vector<char> host;
+    template <class T>
+    size_t add(std::vector<T> const& v)
+    {
+        size_t const at = (host.size() + 255) / 256 * 256;
+        host.resize(at + v.size() * sizeof(T));
+        if (!v.empty()) std::memcpy(host.data() + at, v.data(), v.size() * sizeof(T));
+        return at;
+    }
+    void upload()
+    {
+        buf.upload(host.data(), host.size());
+        host = {};
+    }
+    template <class T>
+    T* at(size_t place) const
+    {
+        return reinterpret_cast<T*>(static_cast<char*>(buf.ptr) + place);
     }
 };
 
@@ -160,7 +187,7 @@ void make_dense_block_problem(HostProblem& pr, int n, int bottom, int top);
 // Device copy of a factored HostProblem.  upload() fills every field of the
 // SolveView: sizes, and pointers into these buffers.
 struct SolveBuffers {
-    DeviceBuffer q, ipiv, slu, sipiv, trr, trc, trv, blr, blc, blv;
+    DevicePack pack;
     void upload(HostProblem const& pr, SolveView& sv);
 };
 
@@ -217,19 +244,34 @@ struct TiledHost {
     std::vector<double> Gblk;
 };
 
+// What a segment of a tiling has to do with the border: the index of its
+// Q^-1 gamma block (-1: none), the rows (bit i: row i) that are columns of
+// lambda couplings, and the slot of the first of them.  Slots number the
+// distinct coupled columns in increasing order.
+struct SegBorder {
+    int gblk;
+    uint32_t mask;
+    int slot0;
+    int pad;
+};
+
 struct TiledView {
-    int K, L, kf, kb, wf, wb, nq, nb, top, q0, bl_nnz, rs;
-    int ngb; // number of L x nb blocks in Gblk
+    int K, L, kf, kb, wf, wb, nq, nb, top, q0, rs;
+    int ngb; // number of blocks in Gblk, each nb columns of L rows
     const double* rt;
     const double* Mf;
     const double* Mb;
-    const int* gseg;
+    const SegBorder* seg; // K
     const double* Gblk;
-    const int* bl_r;
-    const int* bl_c;
-    const double* bl_v;
-    const double* s_lu;
-    const int* s_ipiv;
+    // the lambda couplings grouped for the border step: group g holds
+    // couplings bp[g] .. bp[g + 1] - 1.  The solve groups them by border row
+    // (ngroup = nb; bi = slot of the coupled column), the adjoint by coupled
+    // column (ngroup = number of slots; bi = border row).
+    int nnz, ngroup;
+    const int* bi;
+    const double* bv;
+    const int* bp;
+    const double* sinv; // inverse of the Schur complement (transposed for the adjoint), nb x nb
 };
 
 // Plan of the mixed-precision build (build_refine_kernel.hpp): the tiled sweeps run
@@ -281,6 +323,18 @@ struct RefineView {
     const int* s_ipiv;
 };
 
+// The border data of the tiled kernels that does not depend on the tiling.
+// The Schur systems are nb x nb with nb <= 8: x2 = S^-1 b2 as a product with
+// the inverse (columns solved with the LU factors at plan creation) has no
+// serial chain and no division, unlike the substitutions.
+struct BorderHost {
+    std::vector<int> cols;              // distinct coupled columns of lambda, increasing
+    std::vector<int> slot, rowp;        // couplings by border row: slot of the column, row starts
+    std::vector<int> crow, colp;        // couplings by column: border row, column starts
+    std::vector<double> val, cval;      // values in either order
+    std::vector<double> sinv, sinvt;    // S^-1 and its transpose, row-major
+};
+
 struct BuilderPlan {
     std::shared_ptr<BSplinesPlan> bs;
     ddcx_closure bcl, bcu;
@@ -293,21 +347,16 @@ struct BuilderPlan {
     std::vector<double> points;
     HostProblem prob;
     SolveBuffers d_solve;
-    DeviceBuffer d_points; // the interpolation points, for the in-kernel feet of ddcx_advect
+    DevicePack pack; // every device table below
+    const double* d_points = nullptr; // the interpolation points, for the in-kernel feet of ddcx_advect
     BuildView view{}; // device pointers filled by upload()
-    TiledHost tiled;
-    DeviceBuffer t_Mf, t_Mb, t_rt, t_gseg, t_Gblk;
-    TiledView tview{};
-    // tables of the fused build + eval kernel (fused_build_eval.hip)
-    TiledHost tiled_f;
-    DeviceBuffer tf_Mf, tf_Mb, tf_rt, tf_gseg, tf_Gblk;
-    TiledView tview_f{};
-    // tables of the transposed solve (build_vjp_tiled.hip)
-    TiledHost tiled_t;
-    DeviceBuffer tt_Mf, tt_Mb, tt_rt, tt_gseg, tt_Gblk;
-    TiledView tview_t{};
+    // tables of the tiled build (build_tiled_kernel.hpp), of the fused build +
+    // eval kernel (fused_build_eval.hip) and of the transposed solve
+    // (build_vjp_tiled.hip)
+    TiledHost tiled, tiled_f, tiled_t;
+    TiledView tview{}, tview_f{}, tview_t{};
+    BorderHost border;
     RefineHost refine;
-    DeviceBuffer r_rt, r_Mf, r_Mb, r_gseg_blk, r_Gblk, r_rq, r_gr, r_gc, r_gv, r_gamseg, r_delta;
     RefineView rview{};
     bool on_device = false;
     void upload();
@@ -318,6 +367,8 @@ struct BuilderPlan {
 constexpr int kMaxGBlocksVjp = 8;
 
 void make_tiled(BuilderPlan& p);
+// per segment of a tiling, its part of the border step
+std::vector<SegBorder> segment_borders(TiledHost const& t, BorderHost const& b);
 void make_refine(BuilderPlan& p);
 
 // Batched layout: element (row r, line l) at r*rs + (l % inner)*is + (l / inner)*os.

@@ -22,53 +22,86 @@ __device__ __forceinline__ void chunk_fence(int i)
     if (i % M == M - 1) __builtin_amdgcn_sched_barrier(0);
 }
 
-// The border data a workgroup reads after its sweeps, copied to LDS in its
-// prologue so that the border step waits on no global load:
-// - the lambda couplings (row, column, value);
-// - the Q^-1 gamma blocks with each row padded to kNbMax columns (zeros past
-//   nb), so that the correction is kNbMax unconditional FMAs per row (an
-//   FMA with a zero entry and a zero x2 leaves the row exactly as it was).
+// The border data that a workgroup reads after its sweeps, copied to LDS in
+// its prologue so that the border step waits on no global load: the lambda
+// couplings in their groups, the inverse of the Schur complement, and (in
+// dynamic LDS) the Q^-1 gamma blocks.
 struct BorderLds {
-    int c[kLamMax];
-    int r[kLamMax];
+    int i[kLamMax];
+    int p[kLamMax + 1];
     double v[kLamMax];
+    double sinv[kNbMax * kNbMax];
 };
 
-// NT threads (NT >= kLamMax); GAMMA: also the padded Q^-1 gamma blocks
 template <int NT, bool GAMMA>
 __device__ __forceinline__ void stage_border(TiledView const& tv, BorderLds& bl, double* gpad, int tid)
 {
-    static_assert(NT >= kLamMax, "one coupling per thread");
-    if (tid < tv.bl_nnz) {
-        bl.c[tid] = tv.bl_c[tid];
-        bl.r[tid] = tv.bl_r[tid];
-        bl.v[tid] = tv.bl_v[tid];
+    for (int k = tid; k < tv.nnz; k += NT) {
+        bl.i[k] = tv.bi[k];
+        bl.v[k] = tv.bv[k];
     }
+    for (int k = tid; k < tv.ngroup + 1; k += NT) bl.p[k] = tv.bp[k];
+    for (int k = tid; k < tv.nb * tv.nb; k += NT) bl.sinv[k] = tv.sinv[k];
     if constexpr (GAMMA) {
-        int const n = tv.ngb * tv.L * kNbMax;
-        for (int idx = tid; idx < n; idx += NT) {
-            int const k = idx % kNbMax;
-            gpad[idx] = k < tv.nb ? tv.Gblk[(idx / kNbMax) * tv.nb + k] : 0.0;
+        int const n = tv.ngb * tv.L * tv.nb;
+        for (int k = tid; k < n; k += NT) gpad[k] = tv.Gblk[k];
+    }
+}
+
+// The rows of a segment that lambda couples to the border, to their slots in
+// LDS.  A static row loop with a bit test per row, entered only by the one or
+// two segments that hold such rows: no register indexing, no scan of the
+// couplings.
+template <int LB, int L>
+__device__ __forceinline__ void gather_coupled(double const (&y)[L], SegBorder const& sb, double (*lamx)[LB], int ln)
+{
+    static_assert(L <= 32, "one mask bit per row");
+    if (sb.mask != 0) {
+#pragma unroll
+        for (int i = 0; i < L; ++i)
+            if ((sb.mask >> i) & 1u) lamx[sb.slot0 + __popc(sb.mask & ((1u << i) - 1u))][ln] = y[i];
+    }
+}
+
+// Row k of x2 = S^-1 (b2 - lambda y) for one line: every border row's thread
+// computes the whole right-hand side (nb <= 8 rows of a few couplings, from
+// LDS) and its own row of the product, so the rows need no exchange.
+template <int LB>
+__device__ __forceinline__ double border_row(TiledView const& tv, BorderLds const& bl, double const (*b2)[LB],
+                                             double const (*lamx)[LB], int k, int ln)
+{
+    double x = 0.0;
+    for (int j = 0; j < tv.nb; ++j) {
+        double v = b2[j][ln];
+        int const z1 = bl.p[j + 1];
+        for (int z = bl.p[j]; z < z1; ++z) v = fma(-bl.v[z], lamx[bl.i[z]][ln], v);
+        x = fma(bl.sinv[k * tv.nb + j], v, x);
+    }
+    return x;
+}
+
+// y -= G x2 for one segment's block G, stored column by column (nb columns of
+// L rows).  A run-time loop over the columns around a static one over the
+// rows: with the kNbMax columns unrolled a uniform cubic spline (nb = 1) spent
+// eight times the multiply-adds, in the segments that the whole workgroup
+// waits for; variants by column count made the compiler keep several copies
+// of y (164 to 179 registers instead of 109 to 125, and spills at 128).
+template <int LB, int L>
+__device__ __forceinline__ void apply_gamma(double (&y)[L], const double* G, int nb, double const (*x2s)[LB], int ln)
+{
+    for (int k = 0; k < nb; ++k) {
+        double const x = x2s[k][ln];
+        const double* g = G + k * L;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            y[i] = fma(-g[i], x, y[i]);
+            chunk_fence(i);
         }
     }
 }
 
-// y -= G x2 for one segment's L x kNbMax padded block G
-template <int L>
-__device__ __forceinline__ void apply_gamma(double (&y)[L], const double* G, double const (&x2)[kNbMax])
-{
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-        double t = y[i];
-#pragma unroll
-        for (int k = 0; k < kNbMax; ++k) t = fma(-G[i * kNbMax + k], x2[k], t);
-        y[i] = t;
-        chunk_fence(i);
-    }
-}
-
-// doubles of LDS that stage_border's padded Q^-1 gamma blocks take
-inline size_t gamma_lds_doubles(TiledView const& tv) { return size_t(tv.ngb) * tv.L * kNbMax; }
+// doubles of LDS that stage_border's Q^-1 gamma blocks take
+inline size_t gamma_lds_doubles(TiledView const& tv) { return size_t(tv.ngb) * tv.L * tv.nb; }
 
 __device__ __forceinline__ int64_t lay(Layout const& L, int64_t r, int64_t l)
 {

@@ -254,10 +254,61 @@ void tile_tables(HostProblem const& pr, int K, int L, double tol, TiledHost& t, 
     t.ok = true;
 }
 
+BorderHost make_border(HostProblem const& pr)
+{
+    BorderHost b;
+    int const nb = pr.nb(), nnz = int(pr.bl_v.size());
+    b.cols = pr.bl_c;
+    std::sort(b.cols.begin(), b.cols.end());
+    b.cols.erase(std::unique(b.cols.begin(), b.cols.end()), b.cols.end());
+    b.rowp.assign(nb + 1, 0);
+    b.colp.assign(b.cols.size() + 1, 0);
+    // the COO copy is sorted by row; by column the rows stay in order
+    for (int z = 0; z < nnz; ++z) {
+        int const s = int(std::lower_bound(b.cols.begin(), b.cols.end(), pr.bl_c[z]) - b.cols.begin());
+        b.slot.push_back(s);
+        b.val.push_back(pr.bl_v[z]);
+        ++b.rowp[pr.bl_r[z] + 1];
+        ++b.colp[s + 1];
+    }
+    for (int k = 0; k < nb; ++k) b.rowp[k + 1] += b.rowp[k];
+    for (size_t s = 0; s < b.cols.size(); ++s) b.colp[s + 1] += b.colp[s];
+    b.crow.resize(nnz);
+    b.cval.resize(nnz);
+    std::vector<int> next(b.colp.begin(), b.colp.end());
+    for (int z = 0; z < nnz; ++z) {
+        int const at = next[b.slot[z]]++;
+        b.crow[at] = pr.bl_r[z];
+        b.cval[at] = pr.bl_v[z];
+    }
+    b.sinv.assign(size_t(nb) * nb, 0.0);
+    b.sinvt.assign(size_t(nb) * nb, 0.0);
+    for (int j = 0; j < nb; ++j) {
+        std::vector<double> e(nb, 0.0);
+        e[j] = 1.0;
+        pr.schur.solve(e.data(), 1, false);
+        for (int i = 0; i < nb; ++i) b.sinv[size_t(i) * nb + j] = b.sinvt[size_t(j) * nb + i] = e[i];
+    }
+    return b;
+}
+
 } // namespace
+
+std::vector<SegBorder> segment_borders(TiledHost const& t, BorderHost const& b)
+{
+    std::vector<SegBorder> out(t.K);
+    for (int s = 0; s < t.K; ++s) {
+        auto const lo = std::lower_bound(b.cols.begin(), b.cols.end(), s * t.L);
+        out[s] = SegBorder{t.gseg[s], 0u, int(lo - b.cols.begin()), 0};
+        for (auto c = lo; c != b.cols.end() && *c < (s + 1) * t.L; ++c) out[s].mask |= 1u << (*c - s * t.L);
+    }
+    return out;
+}
 
 void make_tiled(BuilderPlan& p)
 {
+    if (p.prob.blocked && p.prob.nb() <= kMaxBorderTiled && int(p.prob.bl_v.size()) <= kMaxLambda)
+        p.border = make_border(p.prob);
     // K segments of L rows (K*L >= nq) on 1024 threads, LB = 1024/K lines
     // (32 lines give 256-byte rows in batch-contiguous layouts)
     int const nq = p.prob.q.n;
