@@ -6,7 +6,7 @@ namespace ddcx {
 bool launch_build_tiled_k64(BuilderPlan const& p, double* coef, Layout cl, const double* vals, Layout vl,
                             const double* dl, const double* dr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
-    return tiled_build::launch_K<64, 32>(p, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
+    return tiled_build::launch_K<64, 32>(p, p.tiled, p.tview, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
 }
 
 } // namespace ddcx

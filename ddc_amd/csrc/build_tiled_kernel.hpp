@@ -41,8 +41,9 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
 {
     constexpr int KE = KF > KB ? KF : KB;
     constexpr int NT = LB * K;
-    constexpr int SR = stage_rows(K * L), SP = stage_pitch(K * L); // staging chunk rows, pitch (IC)
+    constexpr int SR = stage_rows(K * L, LB), SP = stage_pitch(K * L, LB); // staging chunk rows, pitch (IC)
     constexpr bool TLDS = TMODE != 0;
+    constexpr bool MLDS = TMODE == 1 && transfer_in_lds(LB);
     constexpr int RSF = KF + (FDIV ? 1 : 0), RSB = KB + 1; // split records
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
@@ -54,7 +55,8 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     int const tid = threadIdx.x;
     int const ln = tid % LB;
     int const seg = tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
     int64_t const lc = active ? line : line0;
@@ -72,13 +74,17 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     uint32_t const clo = uint32_t(cb - lay(cl, 0, line0));
     uint32_t const vrs = uint32_t(vl.rs), crs = uint32_t(cl.rs);
 
-    // dynamic LDS: the row table and the Q^-1 gamma blocks (TLDS),
-    // then the staging area, LB x stage_pitch(K * L) doubles, and the per-line
-    // offsets of vals and coef (IC)
+    // dynamic LDS: the row table (TLDS) in the space of the staging area (IC,
+    // LB x stage_pitch doubles, in use before the table is loaded and after its
+    // last read), the Q^-1 gamma blocks (TLDS), the segment transfer products
+    // (MLDS) and the per-line offsets of vals and coef (IC)
     int const tab = TMODE == 2 ? K * L * (RSF > RSB ? RSF : RSB) : K * L * RS; // doubles of the table region
-    double* gpad = rt_lds + tab;
-    double* stg = rt_lds + (TLDS ? tab + tv.ngb * L * tv.nb : 0);
-    uint32_t* loff = reinterpret_cast<uint32_t*>(stg + LB * SP);
+    int const area = IC ? max(TLDS ? tab : 0, LB * SP) : TLDS ? tab : 0;
+    double* gpad = rt_lds + area;
+    double* mtr = gpad + tv.ngb * L * tv.nb;
+    double* stg = rt_lds;
+    uint32_t* loff = reinterpret_cast<uint32_t*>(
+        (TLDS ? mtr : gpad) + (MLDS ? K * (tv.wf * KF * KF + tv.wb * KB * KB) : 0));
     int const nl = int(min<int64_t>(LB, nbatch - line0));
 
     double y[L];
@@ -141,18 +147,15 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
         stage_border<NT, true>(tv, bl, gpad, tid);
         if (seg < tv.nb) b2s[seg][ln] = b2;
         __syncthreads();
-        tiled_forward<LB, K, L, KF, FDIV, 0, KF>(y, rt_lds + r0 * RSF, RSF, tv, ex, seg, ln);
+        tiled_forward<LB, K, L, KF, FDIV, 0, KF>(y, rt_lds + r0 * RSF, RSF, tv.Mf, tv.wf, ex, seg, ln);
         stage_half<NT, KF, KB, FDIV, false>(tv.rt, RS, K * L, rt_lds, tid);
         __syncthreads();
-        tiled_backward<LB, K, L, KB, BDIVF, 0, KB>(y, rt_lds + r0 * RSB, RSB, tv, ex, seg, ln);
+        tiled_backward<LB, K, L, KB, BDIVF, 0, KB>(y, rt_lds + r0 * RSB, RSB, tv.Mb, tv.wb, ex, seg, ln);
     } else {
         const double* T;
         if constexpr (TLDS) {
-            // a few double2 per thread (RS <= 10 doubles per row, K * L <= 2 * NT rows)
-            int const n2 = (K * L * RS) / 2;
-            const double2* src = reinterpret_cast<const double2*>(tv.rt);
-            double2* dst = reinterpret_cast<double2*>(rt_lds);
-            for (int idx = tid; idx < n2; idx += NT) dst[idx] = src[idx];
+            stage_table<NT, K * L, RS>(tv.rt, rt_lds, tid);
+            if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
             stage_border<NT, true>(tv, bl, gpad, tid);
             if (seg < tv.nb) b2s[seg][ln] = b2;
             __syncthreads();
@@ -163,7 +166,9 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
             __syncthreads();
             T = tv.rt + size_t(r0) * RS;
         }
-        tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, T, RS, tv, ex, seg, ln);
+        const double* const Mf = MLDS ? mtr : tv.Mf;
+        const double* const Mb = MLDS ? mtr + K * tv.wf * KF * KF : tv.Mb;
+        tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, T, RS, Mf, tv.wf, Mb, tv.wb, ex, seg, ln);
     }
 
     // ---------------- border (2x2 blocks) ----------------
@@ -196,6 +201,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     // ---------------- store ----------------
     if constexpr (IC) {
         constexpr int PER = LB * SR / NT;
+        __syncthreads(); // the staging area holds the row table until here
         for (int rbase = 0; rbase < K * L; rbase += SR) {
             if (r0 >= rbase && r0 < rbase + SR) {
 #pragma unroll
@@ -241,7 +247,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
 }
 
 template <int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int TMODE, bool IC, int NT>
-void launch_one(BuilderPlan const& p, size_t lds, double* coef, Layout cl, const double* vals, Layout vl,
+void launch_one(BuilderPlan const& p, TiledView const& tv, size_t lds, double* coef, Layout cl, const double* vals, Layout vl,
                 const double* dl, const double* dr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
     constexpr int LB = NT / K;
@@ -250,36 +256,42 @@ void launch_one(BuilderPlan const& p, size_t lds, double* coef, Layout cl, const
         hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       int(lds)),
                   "hipFuncSetAttribute");
-    int64_t const blocks = (nbatch + LB - 1) / LB;
-    hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, p.tview, p.view, vals, vl, dl, dr, dlay,
+    hipLaunchKernelGGL(kern, dim3(tile_grid<LB>(nbatch)), dim3(NT), lds, stream, tv, p.view, vals, vl, dl, dr, dlay,
                        coef, cl, nbatch);
     hip_check(hipGetLastError(), "build_tiled_kernel launch");
 }
 
 template <int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int NT>
-void launch_cfg(BuilderPlan const& p, double* coef, Layout cl, const double* vals, Layout vl, const double* dl,
+bool launch_cfg(BuilderPlan const& p, TiledView const& tv, double* coef, Layout cl, const double* vals, Layout vl, const double* dl,
                 const double* dr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
-    if (p.tiled.rs != KF + KB + 1 + (FDIV ? 1 : 0))
+    if (tv.rs != KF + KB + 1 + (FDIV ? 1 : 0))
         throw Error(DDCX_ERR_INVALID, "row table record length does not match the band shape");
     constexpr int LB = NT / K;
     constexpr int KE = KF > KB ? KF : KB;
     constexpr size_t static_lds =
         size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     bool const ic = vl.rs == 1 && cl.rs == 1;
-    size_t const stage = ic ? size_t(LB) * stage_pitch(K * L) * sizeof(double) + 2 * LB * sizeof(uint32_t) : 0;
+    size_t const stage = ic ? size_t(LB) * stage_pitch(K * L, LB) * sizeof(double) : 0;
+    size_t const off = ic ? 2 * LB * sizeof(uint32_t) : 0;
     constexpr int RSH = (KF + (FDIV ? 1 : 0)) > (KB + 1) ? (KF + (FDIV ? 1 : 0)) : (KB + 1);
-    size_t const gam = gamma_lds_doubles(p.tview) * sizeof(double);
-    size_t const table = size_t(K) * L * p.tiled.rs * sizeof(double) + gam;
-    size_t const half = size_t(K) * L * RSH * sizeof(double) + gam;
+    size_t const gam = gamma_lds_doubles(tv) * sizeof(double) +
+                       (transfer_in_lds(LB) ? transfer_doubles(tv) * sizeof(double) : 0);
+    size_t const table = std::max(size_t(K) * L * tv.rs * sizeof(double), stage) + gam + off;
+    size_t const half = std::max(size_t(K) * L * RSH * sizeof(double), stage) + gam + off;
     size_t constexpr budget = 160 * 1024;
-    int const mode = (static_lds + table + stage <= budget && p.tiled.rs <= 10) ? 1
-                     : (static_lds + half + stage <= budget)                   ? 2
-                                                                               : 0;
-    size_t const lds = (mode == 1 ? table : mode == 2 ? half : 0) + stage;
+    int const mode = (static_lds + table <= budget && tv.rs <= 10) ? 1 : static_lds + half <= budget ? 2 : 0;
+    size_t const lds = mode == 1 ? table : mode == 2 ? half : stage + off;
     auto go = [&]<int TM, bool I>() {
-        launch_one<K, L, KF, KB, FDIV, BDIVF, TM, I, NT>(p, lds, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
+        launch_one<K, L, KF, KB, FDIV, BDIVF, TM, I, NT>(p, tv, lds, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
     };
+    // the small-batch tiles exist with the whole table in LDS only
+    if constexpr (transfer_in_lds(LB)) {
+        if (mode != 1) return false;
+        if (ic) go.template operator()<1, true>();
+        else go.template operator()<1, false>();
+        return true;
+    }
     auto pick = [&]<bool I>() {
         if (mode == 1) go.template operator()<1, I>();
         else if (mode == 2) go.template operator()<2, I>();
@@ -287,17 +299,17 @@ void launch_cfg(BuilderPlan const& p, double* coef, Layout cl, const double* val
     };
     if (ic) pick.template operator()<true>();
     else pick.template operator()<false>();
+    return true;
 }
 
-// NT threads per workgroup: NT / K lines of K segments of L rows
+// NT threads per workgroup: NT / K lines of K segments of L rows, the tables
+// t and their device view tv on that tiling
 template <int K, int L, int NT = 1024>
-bool launch_K(BuilderPlan const& p, double* coef, Layout cl, const double* vals, Layout vl, const double* dl,
+bool launch_K(BuilderPlan const& p, TiledHost const& t, TiledView const& tv, double* coef, Layout cl, const double* vals, Layout vl, const double* dl,
               const double* dr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
-    TiledHost const& t = p.tiled;
     auto go = [&]<int KF, int KB, bool FD, bool BD>() {
-        launch_cfg<K, L, KF, KB, FD, BD, NT>(p, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
-        return true;
+        return launch_cfg<K, L, KF, KB, FD, BD, NT>(p, tv, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
     };
     if (t.bwd_divfirst) {
         if (t.kf == 1 && t.kb == 1 && !t.fwd_div) return go.template operator()<1, 1, false, true>();

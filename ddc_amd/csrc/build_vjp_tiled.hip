@@ -42,9 +42,8 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
 {
     constexpr int KE = KF > KB ? KF : KB;
     constexpr int NT = LB * K;
-    constexpr int SR = stage_rows(K * L), SP = stage_pitch(K * L); // staging chunk rows, pitch (IC)
+    constexpr int SR = stage_rows(K * L, LB), SP = stage_pitch(K * L, LB); // staging chunk rows, pitch (IC)
     __shared__ double ex[KE][K][LB];
-    __shared__ double part[kMaxGBlocksVjp][kNbMax][LB];
     __shared__ double b2s[kNbMax][LB];
     __shared__ double x2s[kNbMax][LB];
     __shared__ BorderLds bl;
@@ -53,7 +52,8 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     int const tid = threadIdx.x;
     int const ln = tid % LB;
     int const seg = tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
     int64_t const lc = active ? line : line0;
@@ -69,12 +69,18 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     uint32_t const vlo = uint32_t(vb - lay(vl, 0, line0)) + uint32_t(tv.q0 + r0) * uint32_t(vl.rs);
     uint32_t const crs = uint32_t(cl.rs), vrs = uint32_t(vl.rs);
 
-    // dynamic LDS: the row table and the Q^-1 gamma blocks (TLDS),
-    // then the staging area (IC), LB x stage_pitch(K * L) doubles, and the per-line
-    // offsets of gcoef and gvals
-    double* gpad = rt_lds + K * L * RS;
-    double* stg = rt_lds + (TLDS ? K * L * RS + tv.ngb * L * nb : 0);
-    uint32_t* loff = reinterpret_cast<uint32_t*>(stg + LB * SP);
+    // dynamic LDS: the row table (TLDS) in the space of the staging area (IC,
+    // as in the build), the Q^-1 gamma blocks (TLDS), the segment transfer
+    // products (MLDS), the partial sums of the border step (ngb * nb rows of LB)
+    // and the per-line offsets of gcoef and gvals (IC)
+    constexpr bool MLDS = TLDS && transfer_in_lds(LB);
+    int const tab = TLDS ? K * L * RS : 0;
+    double* stg = rt_lds;
+    double* gpad = rt_lds + (IC ? max(tab, LB * SP) : tab);
+    double* mtr = gpad + (TLDS ? tv.ngb * L * nb : 0);
+    double* partp = mtr + (MLDS ? K * (tv.wf * KF * KF + tv.wb * KB * KB) : 0);
+    double(*part)[LB] = reinterpret_cast<double(*)[LB]>(partp);
+    uint32_t* loff = reinterpret_cast<uint32_t*>(partp + tv.ngb * nb * LB);
     int const nl = int(min<int64_t>(LB, nbatch - line0));
     if constexpr (IC) {
         if (tid < LB) {
@@ -152,10 +158,8 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     // per-row table and border data in LDS when they fit
     const double* T;
     if constexpr (TLDS) {
-        int const n2 = (K * L * RS) / 2;
-        const double2* src = reinterpret_cast<const double2*>(tv.rt);
-        double2* dst = reinterpret_cast<double2*>(rt_lds);
-        for (int idx = tid; idx < n2; idx += NT) dst[idx] = src[idx];
+        stage_table<NT, K * L, RS>(tv.rt, rt_lds, tid);
+        if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
         stage_border<NT, true>(tv, bl, gpad, tid);
         __syncthreads();
         T = rt_lds + r0 * RS;
@@ -166,8 +170,8 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
 
     // 2. partial sums of (Q^-1 gamma)^T y over this segment's rows
     if (sb.gblk >= 0) {
-        if constexpr (TLDS) gamma_trans<LB>(y, gpad + sb.gblk * L * nb, nb, part[sb.gblk], ln);
-        else gamma_trans<LB>(y, tv.Gblk + size_t(sb.gblk) * L * nb, nb, part[sb.gblk], ln);
+        if constexpr (TLDS) gamma_trans<LB>(y, gpad + sb.gblk * L * nb, nb, part + sb.gblk * nb, ln);
+        else gamma_trans<LB>(y, tv.Gblk + size_t(sb.gblk) * L * nb, nb, part + sb.gblk * nb, ln);
     }
     if (seg < nb) b2s[seg][ln] = b2;
     __syncthreads();
@@ -179,7 +183,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
         double x2 = 0.0;
         for (int j = 0; j < nb; ++j) {
             double v = b2s[j][ln];
-            for (int g = 0; g < tv.ngb; ++g) v -= part[g][j][ln];
+            for (int g = 0; g < tv.ngb; ++g) v -= part[g * nb + j][ln];
             x2 = fma(bl.sinv[seg * nb + j], v, x2);
         }
         x2s[seg][ln] = x2;
@@ -213,10 +217,12 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     }
 
     // 5. y = Q^-T y
-    tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, T, RS, tv, ex, seg, ln);
+    tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, T, RS, MLDS ? mtr : tv.Mf, tv.wf,
+                                                    MLDS ? mtr + K * tv.wf * KF * KF : tv.Mb, tv.wb, ex, seg, ln);
 
     // 6. main-block rows to the value gradients
     if constexpr (IC) {
+        __syncthreads(); // the staging area holds the row table until here
         constexpr int PER = LB * SR / NT;
         for (int rbase = 0; rbase < K * L; rbase += SR) {
             if (r0 >= rbase && r0 < rbase + SR) {
@@ -247,31 +253,37 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
 }
 
 template <int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int NT>
-void launch_cfg(BuilderPlan const& p, const double* gcoef, Layout cl, double* gvals, Layout vl, double* gdl,
+bool launch_cfg(BuilderPlan const& p, TiledView const& tv, const double* gcoef, Layout cl, double* gvals, Layout vl, double* gdl,
                 double* gdr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
-    if (p.tiled_t.rs != KF + KB + 1 + (FDIV ? 1 : 0))
+    if (tv.rs != KF + KB + 1 + (FDIV ? 1 : 0))
         throw Error(DDCX_ERR_INVALID, "row table record length does not match the band shape");
     constexpr int LB = NT / K;
     constexpr int KE = KF > KB ? KF : KB;
     constexpr size_t static_lds =
-        size_t(KE * K * LB + kMaxGBlocksVjp * kNbMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
-    size_t const table = (size_t(K) * L * p.tiled_t.rs + gamma_lds_doubles(p.tview_t)) * sizeof(double);
+        size_t(KE * K * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     bool const ic = vl.rs == 1 && cl.rs == 1;
-    size_t const stage = ic ? size_t(LB) * stage_pitch(K * L) * sizeof(double) + 2 * LB * sizeof(uint32_t) : 0;
-    bool const tlds = static_lds + table + stage <= size_t(160 * 1024) && p.tiled_t.rs <= 10;
-    size_t const lds = (tlds ? table : 0) + stage;
-    int64_t const blocks = (nbatch + LB - 1) / LB;
+    size_t const stage = ic ? size_t(LB) * stage_pitch(K * L, LB) * sizeof(double) : 0;
+    size_t const rest = size_t(tv.ngb) * tv.nb * LB * sizeof(double) + (ic ? 2 * LB * sizeof(uint32_t) : 0);
+    size_t const table = std::max(size_t(K) * L * tv.rs * sizeof(double), stage) + rest +
+                         (gamma_lds_doubles(tv) + (transfer_in_lds(LB) ? transfer_doubles(tv) : 0)) * sizeof(double);
+    bool const tlds = static_lds + table <= size_t(160 * 1024) && tv.rs <= 10;
+    size_t const lds = tlds ? table : stage + rest;
     auto go = [&]<bool TL, bool I>() {
         auto kern = build_vjp_tiled_kernel<LB, K, L, KF, KB, FDIV, BDIVF, TL, I>;
         if (lds > 0)
             hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
                       "hipFuncSetAttribute");
-        hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, p.tview_t, p.view, gcoef, cl, gvals,
+        hipLaunchKernelGGL(kern, dim3(tile_grid<LB>(nbatch)), dim3(NT), lds, stream, tv, p.view, gcoef, cl, gvals,
                            vl, gdl, gdr, dlay, nbatch);
     };
-    if (ic) {
+    if constexpr (transfer_in_lds(LB)) {
+        // the small-batch tiles exist with the table in LDS only
+        if (!tlds) return false;
+        if (ic) go.template operator()<true, true>();
+        else go.template operator()<true, false>();
+    } else if (ic) {
         if (tlds) go.template operator()<true, true>();
         else go.template operator()<false, true>();
     } else {
@@ -279,17 +291,16 @@ void launch_cfg(BuilderPlan const& p, const double* gcoef, Layout cl, double* gv
         else go.template operator()<false, false>();
     }
     hip_check(hipGetLastError(), "build_vjp_tiled_kernel launch");
+    return true;
 }
 
 // NT threads per workgroup: NT / K lines of K segments of L rows
 template <int K, int L, int NT = 1024>
-bool launch_K(BuilderPlan const& p, const double* gcoef, Layout cl, double* gvals, Layout vl, double* gdl,
+bool launch_K(BuilderPlan const& p, TiledHost const& t, TiledView const& tv, const double* gcoef, Layout cl, double* gvals, Layout vl, double* gdl,
               double* gdr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
-    TiledHost const& t = p.tiled_t;
     auto go = [&]<int KF, int KB, bool FD, bool BD>() {
-        launch_cfg<K, L, KF, KB, FD, BD, NT>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-        return true;
+        return launch_cfg<K, L, KF, KB, FD, BD, NT>(p, tv, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
     };
     if (t.bwd_divfirst) {
         if (t.kf == 1 && t.kb == 1 && !t.fwd_div) return go.template operator()<1, 1, false, true>();
@@ -312,18 +323,21 @@ bool launch_build_vjp_tiled(BuilderPlan const& p, const double* gcoef, Layout cl
     if (!p.tiled_t.ok) return false;
     if (!offsets_fit(vl, p.tiled_t.K * p.tiled_t.L + p.tview_t.q0, nbatch) || !offsets_fit(cl, p.view.size, nbatch))
         return false;
-    if (p.tiled_t.K == 32 && p.tiled_t.L == 32)
-        return launch_K<32, 32>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-    if (p.tiled_t.K == 64 && p.tiled_t.L == 32)
-        return launch_K<64, 32>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-    // short lines
-    if (p.tiled_t.K == 16 && p.tiled_t.L == 8)
-        return launch_K<16, 8, 512>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-    if (p.tiled_t.K == 16 && p.tiled_t.L == 9)
-        return launch_K<16, 9, 512>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-    if (p.tiled_t.K == 32 && p.tiled_t.L == 8)
-        return launch_K<32, 8>(p, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
-    return false;
+    int const K = p.tiled_t.K, L = p.tiled_t.L;
+    auto go = [&]<int KK, int LL, int NT>(TiledHost const& t, TiledView const& tv) {
+        return launch_K<KK, LL, NT>(p, t, tv, gcoef, cl, gvals, vl, gdl, gdr, dlay, nbatch, stream);
+    };
+    auto one = [&]<int KK, int LL, int NT>() { return go.template operator()<KK, LL, NT>(p.tiled_t, p.tview_t); };
+    // the small-batch tiles of the build (build_tiled_small.hip: 1000 cells x
+    // 1000 lines 21.8 -> 12.8 us, rows contiguous 28.1 -> 13.8;
+    // build_tiled_short.hip: 200 cells x 1000 lines 9.4 -> 7.9, 11.5 -> 8.8)
+    if (small_batch(nbatch, 1) && p.tiled_ts.ok && go.template operator()<64, 16, 512>(p.tiled_ts, p.tview_ts))
+        return true;
+    if (L == 32) return K == 32 ? one.template operator()<32, 32, 1024>() : one.template operator()<64, 32, 1024>();
+    if (K == 8) return L == 4 ? one.template operator()<8, 4, 256>() : one.template operator()<8, 8, 256>();
+    if (K == 16) return L == 8 ? one.template operator()<16, 8, 512>() : one.template operator()<16, 9, 512>();
+    if (small_batch(nbatch, 2) && one.template operator()<32, 8, 256>()) return true;
+    return one.template operator()<32, 8, 1024>();
 }
 
 } // namespace ddcx

@@ -31,6 +31,7 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     constexpr int NT = LB * K;
     constexpr int ROWS = NT / LB; // point rows per pass (= K)
     constexpr int U = 8;
+    constexpr bool MLDS = transfer_in_lds(LB);
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
     __shared__ double b2s[kNbMax][LB];
@@ -43,7 +44,8 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     int const tid = threadIdx.x;
     int const ln = tid % LB;
     int const seg = tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
     int64_t const lc = active ? line : line0;
@@ -77,16 +79,16 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
         b2 = rhs_src(bv, vals, vl, vb, dl, dr, dlay, lay(dlay, 0, lc), seg < tv.top ? seg : tv.nq + seg);
     SegBorder const sb = tv.seg[seg];
     double* const gpad = dyn + K * L * RS;
+    double* const mtr = gpad + tv.ngb * L * tv.nb; // segment transfer products (MLDS)
     {
-        int const n2 = (K * L * RS) / 2;
-        const double2* src = reinterpret_cast<const double2*>(tv.rt);
-        double2* dst = reinterpret_cast<double2*>(dyn);
-        for (int idx = tid; idx < n2; idx += NT) dst[idx] = src[idx];
+        stage_table<NT, K * L, RS>(tv.rt, dyn, tid);
+        if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
         stage_border<NT, true>(tv, bl, gpad, tid);
         if (seg < tv.nb) b2s[seg][ln] = b2;
         __syncthreads();
     }
-    tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, dyn + r0 * RS, RS, tv, ex, seg, ln);
+    tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, dyn + r0 * RS, RS, MLDS ? mtr : tv.Mf, tv.wf,
+                                                    MLDS ? mtr + K * tv.wf * KF * KF : tv.Mb, tv.wb, ex, seg, ln);
 
     int const nb = tv.nb;
     int const off = bv.offset;
@@ -173,7 +175,7 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     }
 }
 
-template <int K, int KF, int KB, bool FDIV, bool BDIVF, int D>
+template <int K, int NT, int KF, int KB, bool FDIV, bool BDIVF, int D>
 void launch_one(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double* coef, Layout cl,
                 const double* vals, Layout vl, const double* dl, const double* dr, Layout dlay, double* out,
                 const double* coords, Layout pl, int64_t npts, int64_t nbatch, hipStream_t stream, size_t lds,
@@ -181,18 +183,17 @@ void launch_one(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, doub
 {
     if (p.tiled_f.rs != KF + KB + 1 + (FDIV ? 1 : 0))
         throw Error(DDCX_ERR_INVALID, "row table record length does not match the band shape");
-    constexpr int NT = 1024, LB = NT / K, L = 16;
+    constexpr int LB = NT / K, L = 16;
     auto kern = fused_build_eval_kernel<LB, K, L, KF, KB, FDIV, BDIVF, D>;
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   int(lds)),
               "hipFuncSetAttribute");
-    int64_t const blocks = (nbatch + LB - 1) / LB;
-    hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, p.tview_f, p.view, b, rules, vals,
+    hipLaunchKernelGGL(kern, dim3(tile_grid<LB>(nbatch)), dim3(NT), lds, stream, p.tview_f, p.view, b, rules, vals,
                        vl, dl, dr, dlay, coef, cl, out, coords, pl, npts, nbatch, fpts, fshift);
     hip_check(hipGetLastError(), "fused_build_eval_kernel launch");
 }
 
-template <int K>
+template <int K, int NT = 1024>
 bool launch_K(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double* coef, Layout cl,
               const double* vals, Layout vl, const double* dl, const double* dr, Layout dlay, double* out,
               const double* coords, Layout pl, int64_t npts, int64_t nbatch, hipStream_t stream, size_t lds,
@@ -203,7 +204,7 @@ bool launch_K(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double
     bool done = false;
     auto go = [&]<int KF, int KB, bool FD, bool BD, int D>() {
         if (!done && deg == D) {
-            launch_one<K, KF, KB, FD, BD, D>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl,
+            launch_one<K, NT, KF, KB, FD, BD, D>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl,
                                             npts, nbatch, stream, lds, fpts, fshift);
             done = true;
         }
@@ -243,23 +244,34 @@ bool launch_build_eval_fused(BuilderPlan const& p, BSplinesPlan const& bs, Rules
     if (feet_shift && npts != int64_t(p.points.size())) return false;
     const double* const fpts = feet_shift ? p.d_points : nullptr;
     if (vl.rs == 1 || pl.rs == 1 || (coef && cl.rs == 1)) return false; // batch-contiguous layouts only
-    int const K = t.K, L = t.L, LB = 1024 / K;
+    int const K = t.K, L = t.L;
     if (L != 16 || (K != 64 && K != 128)) return false;
     if (!offsets_fit(vl, int64_t(K) * L + p.tview_f.q0, nbatch)) return false;
-    // dynamic LDS: the row table and Q^-1 gamma blocks during the build, then
-    // the coefficient tile
-    size_t const table = (size_t(K) * L * t.rs + gamma_lds_doubles(p.tview_f)) * sizeof(double);
-    size_t const tile = size_t(bs.size()) * LB * sizeof(double);
-    size_t const lds = std::max(table, tile);
-    int const KE = std::max(t.kf, t.kb);
-    size_t const stat = size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
-    if (lds + stat > size_t(160 * 1024)) return false;
     BSplinesView const b = bs.device_view();
-    if (K == 64)
-        return launch_K<64>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl, npts, nbatch,
-                            stream, lds, fpts, feet_shift);
-    return launch_K<128>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl, npts, nbatch, stream,
-                         lds, fpts, feet_shift);
+    int const KE = std::max(t.kf, t.kb);
+    // LDS of a workgroup of LB lines: the row table and Q^-1 gamma blocks (and
+    // the transfer products) during the build, then the coefficient tile; 0
+    // when it does not fit
+    auto lds_of = [&](int LB, bool transfer) {
+        size_t const table = (size_t(K) * L * t.rs + gamma_lds_doubles(p.tview_f) +
+                              (transfer ? transfer_doubles(p.tview_f) : 0)) *
+                             sizeof(double);
+        size_t const lds = std::max(table, size_t(bs.size()) * LB * sizeof(double));
+        size_t const stat = size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+        return lds + stat > size_t(160 * 1024) ? size_t(0) : lds;
+    };
+    auto go = [&]<int KK, int NT>() {
+        size_t const lds = lds_of(NT / KK, transfer_in_lds(NT / KK));
+        return lds > 0 && launch_K<KK, NT>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl, npts,
+                                           nbatch, stream, lds, fpts, feet_shift);
+    };
+    // small batches (build_tiled_small.hip), 4 or 8 lines per workgroup: an
+    // advection step of uniform cubic 512 cells x 1000 lines takes 15.5 us on 4
+    // lines, 15.9 on 8 and 19.0 on 16; x 2000 lines 20.1, 16.3 and 18.9;
+    // 1000 cells x 256 lines 18.2, 19.6 and 25.0
+    if (K == 64 && 2 * nbatch <= 8 * int64_t(cu_count()) && go.template operator()<64, 256>()) return true;
+    if (K == 64 && small_batch(nbatch, 1) && go.template operator()<64, 512>()) return true;
+    return K == 64 ? go.template operator()<64, 1024>() : go.template operator()<128, 1024>();
 }
 
 } // namespace ddcx

@@ -661,7 +661,7 @@ void BuilderPlan::upload()
         return Places{pack.add(th.Mf), pack.add(th.Mb), pack.add(th.rt), pack.add(segment_borders(th, border)),
                       pack.add(cols)};
     };
-    Places const p = add_tiled(tiled), p_f = add_tiled(tiled_f), p_t = add_tiled(tiled_t);
+    Places const p = add_tiled(tiled), p_f = add_tiled(tiled_f), p_t = add_tiled(tiled_t), p_ts = add_tiled(tiled_ts);
     RefineHost const& R = refine;
     size_t const r_rt = pack.add(R.rt32), r_Mf = pack.add(R.Mf32), r_Mb = pack.add(R.Mb32),
                  r_gseg = pack.add(R.t.gseg), r_Gblk = pack.add(R.Gblk32), r_rq = pack.add(R.rq),
@@ -698,6 +698,7 @@ void BuilderPlan::upload()
     view_of(tiled, p, false, tview);
     view_of(tiled_f, p_f, false, tview_f);
     view_of(tiled_t, p_t, true, tview_t);
+    view_of(tiled_ts, p_ts, true, tview_ts);
     if (refine.ok) {
         RefineView& rv = rview;
         rv.K = R.t.K;

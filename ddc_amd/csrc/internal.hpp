@@ -352,9 +352,9 @@ struct BuilderPlan {
     BuildView view{}; // device pointers filled by upload()
     // tables of the tiled build (build_tiled_kernel.hpp), of the fused build +
     // eval kernel (fused_build_eval.hip) and of the transposed solve
-    // (build_vjp_tiled.hip)
-    TiledHost tiled, tiled_f, tiled_t;
-    TiledView tview{}, tview_f{}, tview_t{};
+    // (build_vjp_tiled.hip; tiled_ts for small batches of 256 to 1024 rows)
+    TiledHost tiled, tiled_f, tiled_t, tiled_ts;
+    TiledView tview{}, tview_f{}, tview_t{}, tview_ts{};
     BorderHost border;
     RefineHost refine;
     RefineView rview{};
@@ -364,7 +364,7 @@ struct BuilderPlan {
 };
 
 // segments holding Q^-1 gamma blocks that the tiled adjoint can reduce over
-constexpr int kMaxGBlocksVjp = 8;
+constexpr int kMaxGBlocksVjp = 16;
 
 void make_tiled(BuilderPlan& p);
 // per segment of a tiling, its part of the border step

@@ -156,11 +156,37 @@ __device__ __forceinline__ void getrs_small(int nb, const double* a, const int* 
 // of kStageRows rows of all LB lines: each line's rows are read and written
 // as contiguous runs, and every thread takes its L rows from LDS.
 constexpr int kStageRows = 256;
-constexpr int kStagePitch = kStageRows + 1; // doubles; odd pitch spreads the LDS banks
 // the chunk of a K x L tiling: the whole padded line when it is shorter
 // (K * L rows; the short tilings have K * L = 128 or 144, so the pitch stays odd)
-constexpr int stage_rows(int kl) { return kl < kStageRows ? kl : kStageRows; }
-constexpr int stage_pitch(int kl) { return stage_rows(kl) + 1; }
+// and on the small-batch tiles of a few lines, where one chunk has one barrier
+// pair and all its loads in flight at once; an odd pitch spreads the LDS banks
+constexpr int stage_rows(int kl, int lb) { return kl < kStageRows || lb <= 8 ? kl : kStageRows; }
+constexpr int stage_pitch(int kl, int lb) { return stage_rows(kl, lb) | 1; }
+
+// Tile of workgroup b.  A tile of fewer than 16 lines shares its 128-byte
+// cache lines with its neighbours in the batch-contiguous layout, and
+// consecutive workgroups go to different XCDs, each with its own L2: there the
+// eight XCDs take contiguous ranges of tiles instead.  The grid is then 8 *
+// ceil(ntiles / 8), and tiles at or past ntiles are left at once.
+template <int LB>
+__device__ __forceinline__ int64_t tile_of(unsigned b, unsigned grid)
+{
+    if constexpr (LB >= 16) return b;
+    else return int64_t(b % 8) * (grid / 8) + b / 8;
+}
+
+// Small batches: at most one tile of 8 lines per CU (64 x 16 tiling) or two
+// (32 x 8 tiling).  Up to there the 8-line tiles are faster than the 16- and
+// 32-line ones, past it their shorter runs cost more than the idle CUs
+// (figures in build_tiled_small.hip and build_tiled_short.hip).
+inline bool small_batch(int64_t nbatch, int tiles_per_cu) { return nbatch <= 8 * int64_t(tiles_per_cu) * cu_count(); }
+
+template <int LB>
+inline unsigned tile_grid(int64_t nbatch)
+{
+    int64_t const n = (nbatch + LB - 1) / LB;
+    return unsigned(LB >= 16 ? n : (n + 7) / 8 * 8);
+}
 
 // The tiled kernels address a tile as a workgroup-uniform base plus 32-bit
 // per-lane offsets; true when every offset of the batch fits.
@@ -182,7 +208,7 @@ inline bool offsets_fit(Layout const& l, int64_t rows, int64_t nbatch)
 // row table are [Lf(KF) | Ub(KB) | rDb | rDf (FDIV)].  The forward sweep ends
 // with a barrier; the backward sweep does not.
 template <int LB, int K, int L, int KF, bool FDIV, int OLF, int ORDF>
-__device__ __forceinline__ void tiled_forward(double (&y)[L], const double* T, int RS, TiledView const& tv,
+__device__ __forceinline__ void tiled_forward(double (&y)[L], const double* T, int RS, const double* Mf, int wf,
                                               double (*ex)[K][LB], int seg, int ln)
 {
     double s[KF];
@@ -207,10 +233,10 @@ __device__ __forceinline__ void tiled_forward(double (&y)[L], const double* T, i
     double in[KF];
 #pragma unroll
     for (int k = 0; k < KF; ++k) in[k] = 0.0;
-    for (int w = 1; w <= tv.wf; ++w) {
+    for (int w = 1; w <= wf; ++w) {
         int const src = seg - w;
         if (src >= 0) {
-            const double* m = tv.Mf + (size_t(seg) * tv.wf + (w - 1)) * (KF * KF);
+            const double* m = Mf + (seg * wf + (w - 1)) * (KF * KF);
 #pragma unroll
             for (int a = 0; a < KF; ++a)
 #pragma unroll
@@ -237,7 +263,7 @@ __device__ __forceinline__ void tiled_forward(double (&y)[L], const double* T, i
 }
 
 template <int LB, int K, int L, int KB, bool BDIVF, int OUB, int ORDB>
-__device__ __forceinline__ void tiled_backward(double (&y)[L], const double* T, int RS, TiledView const& tv,
+__device__ __forceinline__ void tiled_backward(double (&y)[L], const double* T, int RS, const double* Mb, int wb,
                                                double (*ex)[K][LB], int seg, int ln)
 {
     double s[KB];
@@ -267,10 +293,10 @@ __device__ __forceinline__ void tiled_backward(double (&y)[L], const double* T, 
     double in[KB];
 #pragma unroll
     for (int k = 0; k < KB; ++k) in[k] = 0.0;
-    for (int w = 1; w <= tv.wb; ++w) {
+    for (int w = 1; w <= wb; ++w) {
         int const src = seg + w;
         if (src < K) {
-            const double* m = tv.Mb + (size_t(seg) * tv.wb + (w - 1)) * (KB * KB);
+            const double* m = Mb + (seg * wb + (w - 1)) * (KB * KB);
 #pragma unroll
             for (int a = 0; a < KB; ++a)
 #pragma unroll
@@ -301,11 +327,53 @@ __device__ __forceinline__ void tiled_backward(double (&y)[L], const double* T, 
 }
 
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int KE>
-__device__ __forceinline__ void tiled_sweeps(double (&y)[L], const double* T, int RS, TiledView const& tv,
-                                             double (*ex)[K][LB], int seg, int ln)
+__device__ __forceinline__ void tiled_sweeps(double (&y)[L], const double* T, int RS, const double* Mf, int wf,
+                                             const double* Mb, int wb, double (*ex)[K][LB], int seg, int ln)
 {
-    tiled_forward<LB, K, L, KF, FDIV, 0, KF + KB + 1>(y, T, RS, tv, ex, seg, ln);
-    tiled_backward<LB, K, L, KB, BDIVF, KF, KF + KB>(y, T, RS, tv, ex, seg, ln);
+    tiled_forward<LB, K, L, KF, FDIV, 0, KF + KB + 1>(y, T, RS, Mf, wf, ex, seg, ln);
+    tiled_backward<LB, K, L, KB, BDIVF, KF, KF + KB>(y, T, RS, Mb, wb, ex, seg, ln);
+}
+
+// The small-batch tiles (4 and 8 lines) also keep the
+// segment transfer products in LDS: the two carry steps then wait on no
+// global load.  The larger tiles have no LDS to spare for them.
+constexpr bool transfer_in_lds(int lb) { return lb <= 8; }
+inline size_t transfer_doubles(TiledView const& tv)
+{
+    return size_t(tv.K) * (tv.wf * tv.kf * tv.kf + tv.wb * tv.kb * tv.kb);
+}
+
+template <int NT>
+__device__ __forceinline__ void stage_transfer(TiledView const& tv, double* dst, int tid)
+{
+    int const nf = tv.K * tv.wf * tv.kf * tv.kf, nb = tv.K * tv.wb * tv.kb * tv.kb;
+    for (int k = tid; k < nf; k += NT) dst[k] = tv.Mf[k];
+    for (int k = tid; k < nb; k += NT) dst[nf + k] = tv.Mb[k];
+}
+
+// The row table to LDS: every load of a thread in flight before its first
+// LDS write (RS <= 10 doubles per row)
+template <int NT, int ROWS, int RS>
+__device__ __forceinline__ void stage_table(const double* rt, double* dst, int tid)
+{
+    static_assert(ROWS * RS % 2 == 0);
+    constexpr int N2 = ROWS * RS / 2, PER = (N2 + NT - 1) / NT;
+    const double2* src = reinterpret_cast<const double2*>(rt);
+    double2* d2 = reinterpret_cast<double2*>(dst);
+    constexpr int CH = PER < 16 ? PER : 16;
+    for (int k0 = 0; k0 < PER; k0 += CH) {
+        double2 v[CH];
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            int const idx = tid + (k0 + k) * NT;
+            v[k] = src[idx < N2 ? idx : N2 - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < CH; ++k) {
+            int const idx = tid + (k0 + k) * NT;
+            if (idx < N2) d2[idx] = v[k];
+        }
+    }
 }
 
 // Split staging of the row table, for tables that do not fit LDS whole:

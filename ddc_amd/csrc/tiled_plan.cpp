@@ -313,11 +313,12 @@ void make_tiled(BuilderPlan& p)
     // (32 lines give 256-byte rows in batch-contiguous layouts)
     int const nq = p.prob.q.n;
     if (nq < 256) {
-        // short lines (64 to 255 rows): 16 segments of 8 or 9 rows up to 144
-        // rows (512-thread workgroups), else 32 segments of 8 rows
-        int const K = nq <= 144 ? 16 : 32, L = nq <= 128 || nq > 144 ? 8 : 9;
-        tile_tables(p.prob, K, L, kCarryTol, p.tiled, false, 64);
-        tile_tables(p.prob, K, L, kCarryTol, p.tiled_t, true, 64);
+        // short lines: 8 segments of 4 or 8 rows up to 64 rows, 16 segments of
+        // 8 or 9 rows up to 144 rows (512-thread workgroups), else 32 segments
+        // of 8 rows
+        int const K = nq <= 64 ? 8 : nq <= 144 ? 16 : 32, L = nq <= 32 ? 4 : nq <= 128 || nq > 144 ? 8 : 9;
+        tile_tables(p.prob, K, L, kCarryTol, p.tiled, false, 2);
+        tile_tables(p.prob, K, L, kCarryTol, p.tiled_t, true, 2);
     } else {
         int const K = nq <= 1024 ? 32 : 64;
         tile_tables(p.prob, K, 32, kCarryTol, p.tiled);
@@ -326,12 +327,13 @@ void make_tiled(BuilderPlan& p)
     // the fused build + eval kernel keeps 16 (nq <= 1024) or 8 lines per
     // workgroup so that their coefficient tile fits in LDS: 16-row segments
     tile_tables(p.prob, p.prob.q.n <= 1024 ? 64 : 128, 16, kCarryTol, p.tiled_f);
-    if (p.tiled_t.ok) {
+    if (nq >= 256 && nq <= 1024) tile_tables(p.prob, 64, 16, kCarryTol, p.tiled_ts, true);
+    for (TiledHost* t : {&p.tiled_t, &p.tiled_ts}) {
         int nblk = 0;
-        for (int g : p.tiled_t.gseg) nblk += g >= 0;
-        if (nblk > kMaxGBlocksVjp) {
-            p.tiled_t.ok = false;
-            p.tiled_t.why = "border couplings spread over too many segments";
+        for (int g : t->gseg) nblk += g >= 0;
+        if (t->ok && nblk > kMaxGBlocksVjp) {
+            t->ok = false;
+            t->why = "border couplings spread over too many segments";
         }
     }
 }

@@ -1,0 +1,72 @@
+"""Builds and their adjoints where the tiled kernels change shape: main blocks
+of up to 64 rows (8 segments of 4 or 8), and the batch sizes at which the 8-line
+tiles of small batches hand over to the 16- and 32-line ones, against the CPU
+oracle (relative error in the max norm <= 1e-13, as for every FP64 build)."""
+import numpy as np
+import pytest
+
+from cases import Case, G, H, HH, P
+from conftest import rel_err
+from test_gpu_build import _run
+from test_gpu_vjp import _vjp
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-13
+
+# ncells around the sizes at which nq (ncells less the border) crosses 32 and 64
+SHORT = [Case(3, True, P, ncells=n) for n in (6, 32, 33, 34, 64, 65, 66)] + [
+    Case(1, True, P, ncells=20),
+    Case(2, False, G, ncells=31, mesh="random"),
+    Case(3, False, H, ncells=33, mesh="random"),
+    Case(4, False, P, ncells=63, mesh="jitter"),
+    Case(5, True, P, ncells=30),
+    Case(5, False, G, ncells=40, mesh="jitter"),
+    Case(5, False, HH, ncells=62, mesh="uniform"),
+]
+
+
+@pytest.mark.parametrize("case", SHORT, ids=lambda c: c.id)
+@pytest.mark.parametrize("layout", ["batch_contiguous", "interp_contiguous"])
+@pytest.mark.parametrize("nbatch", [1, 33])
+def test_short_lines(case, layout, nbatch, cuda):
+    got, ref = _run(case, nbatch, layout, cuda, seed=3)
+    assert rel_err(got, ref) <= TOL
+    got, ref = _vjp(case, nbatch, layout, cuda, seed=4)
+    assert rel_err(got, ref) <= TOL
+
+
+@pytest.mark.parametrize("case,tiles", [(Case(3, True, P, ncells=300), 1), (Case(3, False, G, ncells=1000), 1),
+                                        (Case(5, True, P, ncells=700), 1), (Case(4, False, P, ncells=501, mesh="jitter"), 1),
+                                        (Case(3, True, P, ncells=200), 2), (Case(5, False, H, ncells=180, mesh="jitter"), 2)],
+                         ids=lambda c: getattr(c, "id", None))
+@pytest.mark.parametrize("layout", ["batch_contiguous", "interp_contiguous"])
+def test_batch_thresholds(case, tiles, layout, cuda):
+    import torch
+
+    limit = 8 * tiles * torch.cuda.get_device_properties(cuda).multi_processor_count
+    for nbatch in (9, limit - 7, limit + 1):
+        got, ref = _run(case, nbatch, layout, cuda, seed=5)
+        assert rel_err(got, ref) <= TOL, nbatch
+        got, ref = _vjp(case, nbatch, layout, cuda, seed=6)
+        assert np.all(np.isfinite(got)) and rel_err(got, ref) <= TOL, nbatch
+
+
+@pytest.mark.parametrize("case", [Case(3, True, P, ncells=300), Case(5, True, P, ncells=1000)], ids=lambda c: c.id)
+def test_advect_thresholds(case, cuda):
+    """The fused step on 4, 8 and 16 lines per workgroup."""
+    import torch
+
+    import ddc_amd as D
+
+    orc = case.oracle()
+    bs, builder = case.product()
+    ev = D.SplineEvaluator(bs)
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    rng = np.random.default_rng(1)
+    for nbatch in (3, 4 * cus + 1, 8 * cus + 1):
+        f = rng.standard_normal((orc.npts, nbatch))
+        shift = rng.uniform(-0.03, 0.03, nbatch)
+        ref = orc.eval(builder.interpolation_points()[:, None] - shift[None, :], orc.build(f))
+        out = torch.full((orc.npts, nbatch), np.nan, dtype=torch.float64, device=cuda)
+        D.advect(builder, ev, out, torch.from_numpy(f).to(cuda), torch.from_numpy(shift).to(cuda))
+        assert rel_err(out.cpu().numpy(), ref) <= TOL, nbatch
