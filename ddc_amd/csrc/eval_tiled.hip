@@ -15,149 +15,16 @@
 // Values on plain batch-contiguous arrays take eval_stream_kernel, a
 // persistent form that loads the next tile while the current one is
 // evaluated.
-#include "internal.hpp"
+#include "eval_tiled_kernel.hpp"
 
 namespace ddcx {
 
 namespace {
 
-__device__ __forceinline__ int64_t lay(Layout const& L, int64_t r, int64_t l)
-{
-    return r * L.rs + (l % L.inner) * L.is + (l / L.inner) * L.os;
-}
-
-template <int D, int ORDER, int KIND>
-__device__ __forceinline__ double point_value(BSplinesView const& b, const double* kn, Rules1D rules, double x,
-                                              const double* tile, int pitch)
-{
-    double v[D + 1];
-    int jmin;
-    if constexpr (ORDER == 0) {
-        if (b.periodic) {
-            if (x < b.rmin || x > b.rmax) x -= floor((x - b.rmin) / b.length) * b.length;
-        } else if (x < b.rmin) {
-            if (rules.lower == DDCX_EXTRAP_NULL) return 0.0;
-            x = rules.pos_lower;
-        } else if (x > b.rmax) {
-            if (rules.upper == DDCX_EXTRAP_NULL) return 0.0;
-            x = rules.pos_upper;
-        }
-        jmin = eval_basis<D, true, KIND>(b, kn, x, v);
-    } else {
-        double der[(D + 1) * (ORDER + 1)];
-        jmin = eval_basis_and_n_derivs<D, ORDER, true, KIND>(b, kn, x, der);
-#pragma unroll
-        for (int i = 0; i < D + 1; ++i) v[i] = der[i * (ORDER + 1) + ORDER];
-    }
-    double y = 0.0;
-#pragma unroll
-    for (int i = 0; i < D + 1; ++i) y += tile[(jmin + i) * pitch] * v[i];
-    return y;
-}
-
-template <int D, int ORDER, int LB, int NT, bool LINE_MAJOR, int KIND>
-__global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D rules, double* __restrict__ out,
-                                                        const double* __restrict__ coords, Layout xl, Layout pl,
-                                                        int64_t npts,
-                                                        const double* __restrict__ coef, Layout cl, int64_t nbatch,
-                                                        int ncoef, int pitch, int nknots)
-{
-    extern __shared__ double smem[];
-    double* tile = smem;
-    double* kn = smem + size_t(ncoef) * pitch;
-    uint32_t* cells = reinterpret_cast<uint32_t*>(kn + nknots);
-    constexpr int ROWS = NT / LB;
-    // points per pipeline stage per thread: as many as the registers hold
-    // without spilling (derivative tables of non-uniform bases are the largest)
-    constexpr int U = ORDER == 0 ? 8
-                      : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
-                                              : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
-    constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
-    int const tid = threadIdx.x;
-    int const ln = LINE_MAJOR ? tid / ROWS : tid % LB;
-    int const prow = LINE_MAJOR ? tid % ROWS : tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
-    int64_t const line = line0 + ln;
-    bool const active = line < nbatch;
-    int64_t const lc = active ? line : 0;
-    int64_t const cb = lay(cl, 0, lc);
-    int64_t const pb = lay(pl, 0, lc);
-    // Point i of the line is at cp[i * prs].  Indices past the end are clamped
-    // to the last point: such a slot loads the last coordinate and stores the
-    // last point's own value again, so every load and store of the loop below
-    // is unconditional and the loads of the next stage stay in flight while
-    // the current stage is evaluated.
-    int const last = int(npts) - 1;
-    uint32_t const prs = uint32_t(pl.rs), xrs = uint32_t(xl.rs);
-    const double* __restrict__ cp = coords + lay(xl, 0, lc);
-    double* __restrict__ op = out + pb;
-    auto at = [&](int ii) { return uint64_t(uint32_t(min(ii, last))) * prs; };
-    auto atx = [&](int ii) { return uint64_t(uint32_t(min(ii, last))) * xrs; };
-    // first batch of coordinates, then the whole coefficient tile: every load
-    // of the tile is in flight before the first LDS write
-    double xa[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) xa[u] = __builtin_nontemporal_load(&cp[atx(prow + u * ROWS)]);
-    // the tile is loaded in chunks of TC elements per thread, every load of a
-    // chunk in flight before its LDS writes
-    if constexpr (LINE_MAJOR) {
-        int const nl = int(min<int64_t>(LB, nbatch - line0));
-        int const nel = nl * ncoef;
-        for (int e0 = tid; e0 < nel; e0 += TC * NT) {
-            double tv[TC];
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const e = e0 + k * NT;
-                int const l = e / ncoef, r = e - l * ncoef;
-                tv[k] = e < nel ? coef[lay(cl, r, line0 + l)] : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const e = e0 + k * NT;
-                int const l = e / ncoef, r = e - l * ncoef;
-                if (e < nel) tile[r * pitch + l] = tv[k];
-            }
-        }
-    } else {
-        for (int c0 = prow; c0 < ncoef; c0 += TC * ROWS) {
-            double tv[TC];
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const r = c0 + k * ROWS;
-                tv[k] = r < ncoef ? coef[cb + int64_t(r) * cl.rs] : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const r = c0 + k * ROWS;
-                if (r < ncoef) tile[r * pitch + ln] = tv[k];
-            }
-        }
-    }
-    if (!is_uniform_kind(KIND, b.uniform)) {
-        for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
-        for (int k = tid; k < b.nbucket; k += NT) cells[k] = b.cells[k];
-    }
-    __syncthreads();
-    if (!active) return;
-    const double* knots = is_uniform_kind(KIND, b.uniform) ? nullptr : kn;
-    BSplinesView bl = b;
-    bl.cells = b.nbucket > 0 ? cells : nullptr;
-    const double* tl = tile + ln;
-    // software pipeline: the next batch of coordinates is in flight while the
-    // current one is evaluated and stored
-    for (int i = prow; i <= last; i += U * ROWS) {
-        double xb[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) xb[u] = __builtin_nontemporal_load(&cp[atx(i + (U + u) * ROWS)]);
-        double y[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) y[u] = point_value<D, ORDER, KIND>(bl, knots, rules, xa[u], tl, pitch);
-#pragma unroll
-        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
-#pragma unroll
-        for (int u = 0; u < U; ++u) xa[u] = xb[u];
-    }
-}
+using tiled::kMaxLds;
+using tiled::lay;
+using tiled::load_tile;
+using tiled::point_value;
 
 // Buffer resources (raw buffers, stride 0) for the streaming kernel: a load
 // at a byte offset at or past num_records returns 0 and a store there is
@@ -314,13 +181,13 @@ __global__ void __launch_bounds__(NT) eval_stream_kernel(BSplinesView b, Rules1D
 // spline itself is evaluated (0 where an extrapolation rule applies), and the
 // coefficient gradient of the LB lines accumulated in an LDS tile with LDS
 // atomics, then written once (every row, so no separate zeroing).
-template <int D, int LB, int NT, bool LINE_MAJOR>
+template <int D, int LB, int NT>
 __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rules1D rules,
                                                             const double* __restrict__ coords,
                                                             const double* __restrict__ w, double* __restrict__ gx,
                                                             Layout pl, int64_t npts, const double* __restrict__ coef,
                                                             double* __restrict__ gcoef, Layout cl, int64_t nbatch,
-                                                            int ncoef, int pitch, int nknots)
+                                                            int ncoef, int pitch, int nknots, int line_major)
 {
     extern __shared__ double smem[];
     double* tile = smem;
@@ -331,48 +198,16 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
     constexpr int U = 4;
     constexpr int TC = 16;
     int const tid = threadIdx.x;
-    int const ln = LINE_MAJOR ? tid / ROWS : tid % LB;
-    int const prow = LINE_MAJOR ? tid % ROWS : tid / LB;
+    int const ln = line_major ? tid / ROWS : tid % LB;
+    int const prow = line_major ? tid % ROWS : tid / LB;
     int64_t const line0 = int64_t(blockIdx.x) * LB;
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
     int64_t const lc = active ? line : 0;
     int64_t const cb = lay(cl, 0, lc);
     int64_t const pb = lay(pl, 0, lc);
-    int const nl = int(min<int64_t>(LB, nbatch - line0));
-    int const nel = nl * ncoef;
     // coefficient tile (as in eval_tiled_kernel) and a zeroed gradient tile
-    if constexpr (LINE_MAJOR) {
-        for (int e0 = tid; e0 < nel; e0 += TC * NT) {
-            double tv[TC];
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const e = e0 + k * NT;
-                int const l = e / ncoef, r = e - l * ncoef;
-                tv[k] = e < nel ? coef[lay(cl, r, line0 + l)] : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const e = e0 + k * NT;
-                int const l = e / ncoef, r = e - l * ncoef;
-                if (e < nel) tile[r * pitch + l] = tv[k];
-            }
-        }
-    } else {
-        for (int c0 = prow; c0 < ncoef; c0 += TC * ROWS) {
-            double tv[TC];
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const r = c0 + k * ROWS;
-                tv[k] = r < ncoef ? coef[cb + int64_t(r) * cl.rs] : 0.0;
-            }
-#pragma unroll
-            for (int k = 0; k < TC; ++k) {
-                int const r = c0 + k * ROWS;
-                if (r < ncoef) tile[r * pitch + ln] = tv[k];
-            }
-        }
-    }
+    load_tile<LB, NT, TC>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
     for (int k = tid; k < ncoef * pitch; k += NT) gt[k] = 0.0;
     if (!b.uniform) {
         for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
@@ -416,17 +251,10 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
         }
     }
     __syncthreads();
-    if constexpr (LINE_MAJOR) {
-        for (int e = tid; e < nel; e += NT) {
-            int const l = e / ncoef, r = e - l * ncoef;
-            gcoef[lay(cl, r, line0 + l)] = gt[r * pitch + l];
-        }
-    } else if (active) {
+    if (active) {
         for (int r = prow; r < ncoef; r += ROWS) gcoef[cb + int64_t(r) * cl.rs] = gt[r * pitch + ln];
     }
 }
-
-constexpr size_t kMaxLds = 160 * 1024;
 
 // Adjoint of the value form for batch-contiguous arrays on 16-line tiles (as
 // the evaluators; eval_vjp_tiled_kernel holds two tiles and so takes 8
@@ -458,19 +286,7 @@ __global__ void __launch_bounds__(NT) eval_vjp_2pass_kernel(BSplinesView b, Rule
     int64_t const lc = active ? line : 0;
     int64_t const cb = lay(cl, 0, lc);
     int64_t const pb = lay(pl, 0, lc);
-    for (int c0 = prow; c0 < ncoef; c0 += TC * ROWS) {
-        double tv[TC];
-#pragma unroll
-        for (int k = 0; k < TC; ++k) {
-            int const r = c0 + k * ROWS;
-            tv[k] = r < ncoef ? coef[cb + int64_t(r) * cl.rs] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < TC; ++k) {
-            int const r = c0 + k * ROWS;
-            if (r < ncoef) tile[r * pitch + ln] = tv[k];
-        }
-    }
+    load_tile<LB, NT, TC>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
     if (!b.uniform) {
         for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
         for (int k = tid; k < b.nbucket; k += NT) cells[k] = b.cells[k];
@@ -616,20 +432,8 @@ bool launch_orders(BSplinesPlan const& bs, Rules1D rules, double* out, const dou
     BSplinesView const b = bs.device_view();
     size_t const extra = nknots * sizeof(double) + size_t(b.nbucket) * sizeof(uint32_t);
     auto fits = [&](int lb, int pitch) { return size_t(ncoef) * pitch * sizeof(double) + extra <= kMaxLds; };
-    bool const line_major = pl.rs == 1;
     auto go = [&]<int LB, int NT>(int pitch) {
-        size_t const lds = size_t(ncoef) * pitch * sizeof(double) + extra;
-        auto kern = b.uniform ? (line_major ? eval_tiled_kernel<D, ORDER, LB, NT, true, kUniformBasis>
-                                            : eval_tiled_kernel<D, ORDER, LB, NT, false, kUniformBasis>)
-                              : (line_major ? eval_tiled_kernel<D, ORDER, LB, NT, true, kNonUniformBasis>
-                                            : eval_tiled_kernel<D, ORDER, LB, NT, false, kNonUniformBasis>);
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
-                  "hipFuncSetAttribute");
-        int64_t const blocks = (nbatch + LB - 1) / LB;
-        hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, b, rules, out, coords, xl, pl, npts,
-                           coef, cl, nbatch, ncoef, pitch, nknots);
-        hip_check(hipGetLastError(), "eval_tiled_kernel launch");
+        tiled::launch_eval_tile<D, ORDER, LB, NT>(bs, rules, out, coords, xl, pl, npts, coef, cl, nbatch, pitch, stream);
         return true;
     };
     if (ncoef > 2560) return false;
@@ -673,7 +477,8 @@ bool launch_eval_tiled(BSplinesPlan const& bs, Rules1D rules, int order, double*
     if ((pl.rs == 1) != (cl.rs == 1)) return false;
     // 32-bit point indices and point strides in the kernel
     if (npts >= (int64_t(1) << 30) || pl.rs >= (int64_t(1) << 32) || xl.rs >= (int64_t(1) << 32)) return false;
-    bool launched = false;
+    bool launched = launch_eval_small(bs, rules, order, out, coords, xl, pl, npts, coef, cl, nbatch, stream);
+    if (launched) return true;
     dispatch_degree(bs.view.degree, [&]<int D>() {
         auto ord = [&]<int O>() {
             if constexpr (O <= D) {
@@ -733,14 +538,14 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
     }
     dispatch_degree(b.degree, [&]<int D>() {
         constexpr int LB = 8, NT = 1024;
-        auto kern = line_major ? eval_vjp_tiled_kernel<D, LB, NT, true> : eval_vjp_tiled_kernel<D, LB, NT, false>;
+        auto kern = eval_vjp_tiled_kernel<D, LB, NT>;
         size_t const lds = lds_of(pitch);
         hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
                   "hipFuncSetAttribute");
         int64_t const blocks = (nbatch + LB - 1) / LB;
         hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, b, rules, coords, w, gx, pl,
-                           npts, coef, gcoef, cl, nbatch, ncoef, pitch, nknots);
+                           npts, coef, gcoef, cl, nbatch, ncoef, pitch, nknots, line_major ? 1 : 0);
         hip_check(hipGetLastError(), "eval_vjp_tiled_kernel launch");
         launched = true;
     });

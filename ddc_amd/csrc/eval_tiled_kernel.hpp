@@ -1,0 +1,162 @@
+// The LDS-staged batched evaluation kernel (described in eval_tiled.hip) and
+// its launcher, shared by eval_tiled.hip and eval_small.hip.
+#pragma once
+
+#include "tiled_common.hpp"
+
+namespace ddcx {
+namespace tiled {
+
+constexpr size_t kMaxLds = 160 * 1024;
+
+// One point's value (ORDER 0, with the extrapolation rules) or derivative from
+// its line's tile.
+template <int D, int ORDER, int KIND>
+__device__ __forceinline__ double point_value(BSplinesView const& b, const double* kn, Rules1D rules, double x,
+                                              const double* tile, int pitch)
+{
+    double v[D + 1];
+    int jmin;
+    if constexpr (ORDER == 0) {
+        if (b.periodic) {
+            if (x < b.rmin || x > b.rmax) x -= floor((x - b.rmin) / b.length) * b.length;
+        } else if (x < b.rmin) {
+            if (rules.lower == DDCX_EXTRAP_NULL) return 0.0;
+            x = rules.pos_lower;
+        } else if (x > b.rmax) {
+            if (rules.upper == DDCX_EXTRAP_NULL) return 0.0;
+            x = rules.pos_upper;
+        }
+        jmin = eval_basis<D, true, KIND>(b, kn, x, v);
+    } else {
+        double der[(D + 1) * (ORDER + 1)];
+        jmin = eval_basis_and_n_derivs<D, ORDER, true, KIND>(b, kn, x, der);
+#pragma unroll
+        for (int i = 0; i < D + 1; ++i) v[i] = der[i * (ORDER + 1) + ORDER];
+    }
+    double y = 0.0;
+#pragma unroll
+    for (int i = 0; i < D + 1; ++i) y += tile[(jmin + i) * pitch] * v[i];
+    return y;
+}
+
+// The coefficient tile of a workgroup's lines to LDS: thread (line ln, row
+// prow) takes the rows prow, prow + NT / LB, ... of its line, in chunks of TC
+// whose loads are all in flight before the first LDS write.  Batch-contiguous:
+// the lanes of a row read LB consecutive lines; interpolation-contiguous: the
+// threads of a line read consecutive rows of it.
+template <int LB, int NT, int TC>
+__device__ __forceinline__ void load_tile(double* tile, int pitch, const double* __restrict__ c, int64_t rs, int ncoef,
+                                          int ln, int prow)
+{
+    constexpr int ROWS = NT / LB;
+    for (int c0 = prow; c0 < ncoef; c0 += TC * ROWS) {
+        double tv[TC];
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            int const r = c0 + k * ROWS;
+            tv[k] = r < ncoef ? c[int64_t(r) * rs] : 0.0;
+        }
+#pragma unroll
+        for (int k = 0; k < TC; ++k) {
+            int const r = c0 + k * ROWS;
+            if (r < ncoef) tile[r * pitch + ln] = tv[k];
+        }
+    }
+}
+
+template <int D, int ORDER, int LB, int NT, int KIND>
+__global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D rules, double* __restrict__ out,
+                                                        const double* __restrict__ coords, Layout xl, Layout pl,
+                                                        int64_t npts,
+                                                        const double* __restrict__ coef, Layout cl, int64_t nbatch,
+                                                        int ncoef, int pitch, int nknots, int line_major)
+{
+    extern __shared__ double smem[];
+    double* tile = smem;
+    double* kn = smem + size_t(ncoef) * pitch;
+    uint32_t* cells = reinterpret_cast<uint32_t*>(kn + nknots);
+    constexpr int ROWS = NT / LB;
+    // points per pipeline stage per thread: as many as the registers hold
+    // without spilling (derivative tables of non-uniform bases are the largest)
+    constexpr int U = LB < 16 && NT < 1024 ? 4
+                      : ORDER == 0 ? 8
+                      : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
+                                              : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
+    constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
+    int const tid = threadIdx.x;
+    int const ln = line_major ? tid / ROWS : tid % LB;
+    int const prow = line_major ? tid % ROWS : tid / LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    if (LB < 16 && line0 >= nbatch) return; // whole workgroup
+    int64_t const line = line0 + ln;
+    bool const active = line < nbatch;
+    int64_t const lc = active ? line : 0;
+    int64_t const cb = lay(cl, 0, lc);
+    int64_t const pb = lay(pl, 0, lc);
+    // Point i of the line is at cp[i * prs].  Indices past the end are clamped
+    // to the last point: such a slot loads the last coordinate and stores the
+    // last point's own value again, so every load and store of the loop below
+    // is unconditional and the loads of the next stage stay in flight while
+    // the current stage is evaluated.
+    int const last = int(npts) - 1;
+    uint32_t const prs = uint32_t(pl.rs), xrs = uint32_t(xl.rs);
+    const double* __restrict__ cp = coords + lay(xl, 0, lc);
+    double* __restrict__ op = out + pb;
+    auto at = [&](int ii) { return uint64_t(uint32_t(min(ii, last))) * prs; };
+    auto atx = [&](int ii) { return uint64_t(uint32_t(min(ii, last))) * xrs; };
+    // first batch of coordinates, then the whole coefficient tile: every load
+    // of the tile is in flight before the first LDS write
+    double xa[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) xa[u] = __builtin_nontemporal_load(&cp[atx(prow + u * ROWS)]);
+    // the tile is loaded in chunks of TC elements per thread, every load of a
+    // chunk in flight before its LDS writes
+    load_tile<LB, NT, TC>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
+    if (!is_uniform_kind(KIND, b.uniform)) {
+        for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
+        for (int k = tid; k < b.nbucket; k += NT) cells[k] = b.cells[k];
+    }
+    __syncthreads();
+    if (!active) return;
+    const double* knots = is_uniform_kind(KIND, b.uniform) ? nullptr : kn;
+    BSplinesView bl = b;
+    bl.cells = b.nbucket > 0 ? cells : nullptr;
+    const double* tl = tile + ln;
+    // software pipeline: the next batch of coordinates is in flight while the
+    // current one is evaluated and stored
+    for (int i = prow; i <= last; i += U * ROWS) {
+        double xb[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xb[u] = __builtin_nontemporal_load(&cp[atx(i + (U + u) * ROWS)]);
+        double y[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) y[u] = point_value<D, ORDER, KIND>(bl, knots, rules, xa[u], tl, pitch);
+#pragma unroll
+        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
+#pragma unroll
+        for (int u = 0; u < U; ++u) xa[u] = xb[u];
+    }
+}
+
+// eval_tiled_kernel on tiles of LB lines with the given LDS pitch
+template <int D, int ORDER, int LB, int NT>
+void launch_eval_tile(BSplinesPlan const& bs, Rules1D rules, double* out, const double* coords, Layout xl, Layout pl,
+                      int64_t npts, const double* coef, Layout cl, int64_t nbatch, int pitch, hipStream_t stream)
+{
+    int const ncoef = bs.size();
+    int const nknots = bs.view.uniform ? 0 : int(bs.knots_host.size());
+    BSplinesView const b = bs.device_view();
+    size_t const lds = (size_t(ncoef) * pitch + nknots) * sizeof(double) + size_t(b.nbucket) * sizeof(uint32_t);
+    auto kern = b.uniform ? eval_tiled_kernel<D, ORDER, LB, NT, kUniformBasis>
+                          : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis>;
+    hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  int(lds)),
+              "hipFuncSetAttribute");
+    hipLaunchKernelGGL(kern, dim3(tile_grid<LB>(nbatch)), dim3(NT), lds, stream, b, rules, out, coords, xl, pl, npts,
+                       coef, cl, nbatch, ncoef, pitch, nknots, pl.rs == 1 ? 1 : 0);
+    hip_check(hipGetLastError(), "eval_tiled_kernel launch");
+}
+
+} // namespace tiled
+} // namespace ddcx

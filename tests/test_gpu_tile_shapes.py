@@ -70,3 +70,39 @@ def test_advect_thresholds(case, cuda):
         out = torch.full((orc.npts, nbatch), np.nan, dtype=torch.float64, device=cuda)
         D.advect(builder, ev, out, torch.from_numpy(f).to(cuda), torch.from_numpy(shift).to(cuda))
         assert rel_err(out.cpu().numpy(), ref) <= TOL, nbatch
+
+
+@pytest.mark.parametrize("case", [Case(3, True, P, ncells=90), Case(2, True, G, ncells=70), Case(5, True, P, ncells=300),
+                                  Case(4, False, P, ncells=101, mesh="jitter"), Case(3, False, G, ncells=1000)],
+                         ids=lambda c: c.id)
+@pytest.mark.parametrize("axis", [0, 1])
+def test_eval_thresholds(case, axis, cuda):
+    """Values and first derivatives on 4, 8 and 16 lines per workgroup, with
+    points outside the domain for the values."""
+    import torch
+
+    import ddc_amd as D
+
+    orc = case.oracle()
+    bs, _ = case.product()
+    ev = D.SplineEvaluator(bs, D.ConstantExtrapolationRule(), D.NullExtrapolationRule())
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    rng = np.random.default_rng(2)
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a if axis == 0 else a.T)).to(cuda)
+
+    for nbatch in (8, 4 * cus - 1, 4 * cus + 1, 8 * cus - 3, 8 * cus + 1):
+        coef = rng.standard_normal((orc.size, nbatch))
+        if case.periodic:
+            coef[-case.degree:] = coef[:case.degree]
+        x = rng.uniform(-0.05, 1.05, (67, nbatch))
+        out = torch.empty_like(dev(x))
+        ev(out, dev(x), dev(coef), axis=axis)
+        got = out.cpu().numpy() if axis == 0 else out.cpu().numpy().T
+        ref = orc.eval(x, coef, extrap=("constant", "null"))
+        assert rel_err(got, ref) <= TOL, nbatch
+        x = np.clip(x, 0.0, 1.0)
+        ev.deriv(1, out, dev(x), dev(coef), axis=axis)
+        got = out.cpu().numpy() if axis == 0 else out.cpu().numpy().T
+        assert rel_err(got, orc.eval(x, coef, deriv=1, extrap=("constant", "null"))) <= 10 * TOL, nbatch
