@@ -136,4 +136,8 @@ def check(status):
 
 
 def call(name, *args):
-    check(getattr(lib(), name)(*args))
+    # a bound entry point is an instance attribute of the loaded library: one
+    # dictionary lookup after its first use
+    status = getattr(_lib or lib(), name)(*args)
+    if status != DDCX_OK:
+        check(status)

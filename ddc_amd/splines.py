@@ -102,11 +102,12 @@ def n_boundary_equations(bc, degree):
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # torch.cuda.current_stream().cuda_stream without the Stream object
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _check_f64_cuda(t, name):
@@ -123,6 +124,11 @@ def batched_layout(t, axis):
     contiguous with each other (stride[d] == shape[d+1] * stride[d+1]) merge
     into one; at most two batch dimensions may remain.  Returns
     (layout, nbatch)."""
+    if t.dim() == 2:  # one batch dimension: nothing to merge
+        (n0, n1), (s0, s1) = t.shape, t.stride()
+        if axis % 2 == 0:
+            return ddcx_layout(s0, n1, s1, 0), n1
+        return ddcx_layout(s1, n0, s0, 0), n0
     axis = axis % t.dim()
     groups = []  # [count, stride] of merged batch dimensions, outermost first
     for side in (range(axis), range(axis + 1, t.dim())):
