@@ -29,8 +29,8 @@ struct BSplinesView {
     double rmax;     // coordinate(break_point_domain.back())
     double length;   // rmax - rmin
     const double* knots; // non-uniform knots (ncells + 1 + 2*degree), device or host memory
-    // Non-uniform cell search brackets: nbucket equal buckets over [rmin, rmax];
-    // cells[k] packs the first (low 16 bits) and last (high 16 bits) cell that
+    // Non-uniform cell search brackets: nbucket equal buckets over [rmin, rmax]
+    // (bucket_of); cells[k] packs the first (low 16 bits) and last (high 16 bits) cell that
     // bucket k overlaps.  nullptr: plain binary search over all cells.
     const uint32_t* cells;
     int nbucket;
@@ -65,37 +65,38 @@ __host__ __device__ inline int uniform_cell(BSplinesView const& b, double x, dou
     return icell;
 }
 
+// Bucket of x among the nbucket equal buckets over [rmin, rmax] (points
+// outside: the first or last one).  The host computes the same function of the
+// break points for the brackets: it is monotone in x (so are the rounded
+// subtraction and product), hence a cell that holds x is in the bracket of x's
+// bucket, with no rounding to allow for.
+__host__ __device__ inline int bucket_of(BSplinesView const& b, int nbucket, double inv_bucket, double x)
+{
+    int const k = int((x - b.rmin) * inv_bucket);
+    return k < 0 ? 0 : (k >= nbucket ? nbucket - 1 : k);
+}
+
 // NonUniformBSplines::Impl::find_cell_start, bsplines_non_uniform.hpp:668-695.
 // Returns the knot index of the cell start (break point domain starts at
-// knot index `degree`).
+// knot index `degree`).  The cell is unique, so any search gives the reference's.
 __host__ __device__ inline int nonuniform_cell(BSplinesView const& b, const double* knots, double x)
 {
-    int const front = b.degree;
-    int const back = b.degree + b.ncells;
-    if (x <= knots[front]) return front;
-    if (x >= knots[back]) return back - 1;
-    int low = front;
-    int high = back;
+    int base = b.degree, n = b.ncells - 1; // the cell is one of base .. base + n
     if (b.cells) {
-        // Start the same search from the bracket of x's bucket.  The result is
-        // the unique cell with knots[icell] <= x < knots[icell + 1], so it is
-        // the reference's whatever bracket holds it; a bracket missed through
-        // rounding of the bucket index falls back to the full range.
-        int k = int((x - b.rmin) * b.inv_bucket);
-        k = k < 0 ? 0 : (k >= b.nbucket ? b.nbucket - 1 : k);
-        uint32_t const e = b.cells[k];
-        int const lo = front + int(e & 0xffffu);
-        int const hi = front + int(e >> 16) + 1;
-        if (x >= knots[lo]) low = lo;
-        if (x < knots[hi]) high = hi;
+        uint32_t const e = b.cells[bucket_of(b, b.nbucket, b.inv_bucket, x)];
+        base += int(e & 0xffffu);
+        n = int(e >> 16) - int(e & 0xffffu);
     }
-    int icell = low + (high - low) / 2;
-    while (x < knots[icell] || x >= knots[icell + 1]) {
-        if (x < knots[icell]) high = icell;
-        else low = icell;
-        icell = low + (high - low) / 2;
+    while (n > 0) {
+        int const half = (n + 1) >> 1;
+        if (knots[base + half] <= x) {
+            base += half;
+            n -= half;
+        } else {
+            n = half - 1;
+        }
     }
-    return icell;
+    return base;
 }
 
 // The extrapolation rules of a 1D evaluator (SplineEvaluator's lower and
@@ -219,17 +220,41 @@ __host__ __device__ inline void uniform_basis_from_offset(double offset, double*
     }
 }
 
+// The inverses of M positive divisors from one refined hardware reciprocal of
+// their product: prefix products forward, the running inverse backward, 3
+// multiplications per divisor instead of a reciprocal and four fmas each.
+// Outside [2^-960, 2^960] each divisor takes its own reciprocal; SAFE: the host
+// has checked that no cell's product leaves the range (products_safe), so the
+// branch goes.  (In a loop over several points it made the compiler keep the
+// divisors of all of them: 668 B of spills for 8 cubic points.)
+template <int M, bool SAFE>
+__host__ __device__ inline void invert_together(double const (&den)[M], double (&pre)[M], double (&inv)[M])
+{
+    pre[0] = den[0];
+#pragma unroll
+    for (int k = 1; k < M; ++k) pre[k] = pre[k - 1] * den[k];
+    double const mag = fabs(pre[M - 1]);
+    if (SAFE || (mag >= 0x1p-960 && mag <= 0x1p960)) {
+        double rv = fast_rcp(pre[M - 1]);
+#pragma unroll
+        for (int k = M - 1; k > 0; --k) {
+            inv[k] = rv * pre[k - 1];
+            rv *= den[k];
+        }
+        inv[0] = rv;
+    } else {
+#pragma unroll
+        for (int k = 0; k < M; ++k) inv[k] = fast_rcp(den[k]);
+    }
+}
+
 // de Boor with left/right arrays, NonUniformBSplines eval_basis,
 // bsplines_non_uniform.hpp:461-497; `icell` is the knot index from
 // nonuniform_cell.  FAST (device evaluation): the update is one fma, and the
 // D(D+1)/2 divisors right[r] + left[j - r], which do not depend on the
-// recurrence's values, are inverted together: one refined hardware
-// reciprocal of their product, then each inverse as that reciprocal times
-// the product of the others (prefix products forward, the running inverse
-// backward), 3 multiplications per divisor instead of a reciprocal and four
-// fmas each. Every divisor is at least the cell's width, so the product is
-// positive; outside [2^-960, 2^960] each divisor takes its own reciprocal.
-template <int D, bool FAST = false>
+// recurrence's values, are inverted together (every divisor is at least the
+// cell's width, so their product is positive).
+template <int D, bool FAST = false, bool SAFE = false>
 __host__ __device__ inline void nonuniform_basis(const double* knots, int icell, double x, double* values)
 {
     double left[D > 0 ? D : 1];
@@ -250,22 +275,7 @@ __host__ __device__ inline void nonuniform_basis(const double* knots, int icell,
 #pragma unroll
                 for (int r = 0; r < j + 1; ++r) den[k++] = right[r] + left[j - r];
         }
-        pre[0] = den[0];
-#pragma unroll
-        for (int k = 1; k < M; ++k) pre[k] = pre[k - 1] * den[k];
-        double const mag = fabs(pre[M - 1]);
-        if (mag >= 0x1p-960 && mag <= 0x1p960) {
-            double rv = fast_rcp(pre[M - 1]);
-#pragma unroll
-            for (int k = M - 1; k > 0; --k) {
-                inv[k] = rv * pre[k - 1];
-                rv *= den[k];
-            }
-            inv[0] = rv;
-        } else {
-#pragma unroll
-            for (int k = 0; k < M; ++k) inv[k] = fast_rcp(den[k]);
-        }
+        invert_together<M, SAFE>(den, pre, inv);
         int k = 0;
 #pragma unroll
         for (int j = 0; j < D; ++j) {
@@ -295,9 +305,95 @@ __host__ __device__ inline void nonuniform_basis(const double* knots, int icell,
     }
 }
 
+// Values v and first derivatives dv of the D + 1 splines on a point's cell
+// (device evaluation): the recurrence runs to degree D - 1, whose values M give
+// both, with the divisors of the last level inverted once,
+//   B_k' = D (M_{k-1} / w_{k-1} - M_k / w_k),  w_r = right_r + left_{D-1-r},
+// and v by the last step of the recurrence.  NURBS A2.3 for one derivative
+// without its tables.
+template <int D, bool SAFE = false>
+__host__ __device__ inline void nonuniform_basis_deriv(const double* knots, int icell, double x, double* v, double* dv)
+{
+    constexpr int M = D * (D + 1) / 2, W = M - D;
+    double left[D], right[D], den[M], pre[M], inv[M];
+#pragma unroll
+    for (int j = 0; j < D; ++j) {
+        left[j] = x - knots[icell - j];
+        right[j] = knots[icell + j + 1] - x;
+    }
+    {
+        int k = 0;
+#pragma unroll
+        for (int j = 0; j < D; ++j)
+#pragma unroll
+            for (int r = 0; r < j + 1; ++r) den[k++] = right[r] + left[j - r];
+    }
+    invert_together<M, SAFE>(den, pre, inv);
+    v[0] = 1.0;
+    int k = 0;
+#pragma unroll
+    for (int j = 0; j < D - 1; ++j) {
+        double saved = 0.0;
+#pragma unroll
+        for (int r = 0; r < j + 1; ++r) {
+            double const temp = v[r] * inv[k++];
+            v[r] = fma(right[r], temp, saved);
+            saved = left[j - r] * temp;
+        }
+        v[j + 1] = saved;
+    }
+    double saved = 0.0, before = 0.0;
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+        double const temp = v[r] * inv[W + r];
+        dv[r] = (before - temp) * D;
+        before = temp;
+        v[r] = fma(right[r], temp, saved);
+        saved = left[D - 1 - r] * temp;
+    }
+    dv[D] = before * D;
+    v[D] = saved;
+}
+
+template <int D>
+__host__ __device__ inline void uniform_basis_deriv(double offset, double inv_step, double* v, double* dv)
+{
+    uniform_basis_from_offset<D, true>(offset, v);
+    double xx = -offset, saved = 0.0, before = 0.0;
+#pragma unroll
+    for (int r = 0; r < D; ++r) {
+        xx += 1;
+        dv[r] = (before - v[r]) * inv_step;
+        before = v[r];
+        double const temp = v[r] * (1.0 / D);
+        v[r] = fma(xx, temp, saved);
+        saved = (D - xx) * temp;
+    }
+    dv[D] = before * inv_step;
+    v[D] = saved;
+}
+
+// Whether the product of a cell's D(D+1)/2 divisors (the knot differences that
+// contain the cell), and every prefix of it in invert_together's order, stays
+// within [2^-900, 2^900] in every cell.  The divisors of a point differ from
+// the knot differences by rounding only.
+inline bool products_safe(int degree, int ncells, const double* knots)
+{
+    for (int c = degree; c < degree + ncells; ++c) {
+        double p = 1.0;
+        for (int j = 0; j < degree; ++j)
+            for (int r = 0; r < j + 1; ++r) {
+                p *= knots[c + r + 1] - knots[c - (j - r)];
+                if (!(p >= 0x1p-900 && p <= 0x1p900)) return false;
+            }
+    }
+    return true;
+}
+
 // Basis kind of a kernel instantiation: decided by BSplinesView::uniform at
 // run time, or fixed at compile time so that the other branch is not emitted.
-enum BasisKind : int { kAnyBasis = -1, kNonUniformBasis = 0, kUniformBasis = 1 };
+// kSafeNonUniform: non-uniform with products_safe divisors.
+enum BasisKind : int { kAnyBasis = -1, kNonUniformBasis = 0, kUniformBasis = 1, kSafeNonUniform = 2 };
 
 __host__ __device__ constexpr bool is_uniform_kind(int kind, int uniform)
 {
@@ -337,10 +433,28 @@ template <int D, int N, bool FAST = false, int KIND = kAnyBasis>
 __host__ __device__ inline int eval_basis_and_n_derivs(BSplinesView const& b, const double* knots, double x,
                                                        double* derivs)
 {
+    bool const uni = is_uniform_kind(KIND, b.uniform);
+    int jmin;
+    if constexpr (FAST && N == 1) {
+        double v[D + 1], dv[D + 1];
+        if (uni) {
+            double offset;
+            jmin = uniform_cell(b, x, offset);
+            uniform_basis_deriv<D>(offset, b.inv_step, v, dv);
+        } else {
+            int const icell = nonuniform_cell(b, knots, x);
+            nonuniform_basis_deriv<D>(knots, icell, x, v, dv);
+            jmin = icell - D;
+        }
+#pragma unroll
+        for (int i = 0; i < D + 1; ++i) {
+            derivs[i * 2] = v[i];
+            derivs[i * 2 + 1] = dv[i];
+        }
+        return jmin;
+    }
     double ndu[D + 1][D + 1];
     double a[D + 1][2];
-    int jmin;
-    bool const uni = is_uniform_kind(KIND, b.uniform);
     if (uni) {
         double offset;
         jmin = uniform_cell(b, x, offset);

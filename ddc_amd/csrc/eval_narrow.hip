@@ -1,0 +1,66 @@
+// eval_tiled_kernel on tiles of 4 or 8 lines, 512 threads, for values and first
+// derivatives of degrees 2 to 5.
+//
+// The 16-line tile fills most of a CU's LDS and has 1024 threads: small batches
+// leave CUs idle, short lines leave threads idle (16 lines of 100 points are 1.6
+// points per thread), and one resident workgroup alternates between loading its
+// tile and its points.  Narrow tiles put two or more workgroups on a CU.  Their
+// runs in batch-contiguous arrays are 32 or 64 bytes, which costs bandwidth where
+// the arrays come from HBM and the lines are long; neighbouring tiles run on one
+// XCD, whose L2 then holds the shared lines.  Times in us, the 16-line kernels ->
+// here (value form; batch-contiguous, then rows contiguous):
+//  - small batches, latency-bound: uniform cubic 512 points x 1000 lines 11.6 ->
+//    7.2, 10.8 -> 5.9; 1000 x 1000 17.2 -> 9.6, 16.1 -> 7.5; non-uniform 32.3 ->
+//    15.7, 31.0 -> 14.0; 2000 lines of 1000 points 16.8 -> 12.6 on 8 lines, 19.6
+//    on 4;
+//  - rows contiguous, any batch: uniform cubic 64 x 90001 184 -> 110, 300 x 90001
+//    198 -> 167, 600 x 60000 241 -> 166, 1024 x 65536 322 -> 290; non-uniform 700
+//    x 60001 369 -> 248; where two 8-line tiles do not fit a CU 4 lines: non-
+//    uniform 1024 x 65536 443 -> 421 (517 on 8 lines), 2000 x 20000 200 -> 168;
+//  - batch-contiguous, up to 512 points: 64 x 65536 122 -> 82, 256 x 65536 140 ->
+//    105, 512 x 65536 200 -> 191, non-uniform 266 -> 244.  Above, the streaming
+//    kernel is faster (1024 x 65536 357, here 500), unless the batch has too few
+//    tiles for it (600 x 12000 quartic 57 -> 48) or the rows do not start at
+//    128-byte lines, where 16-line runs straddle two (600 x 60001 451 -> 374, 1000
+//    x 60001 736 -> 699, non-uniform 751 -> 657);
+//  - except uniform bases with more than 400 points in batches of one 16-line
+//    tile per CU: 500 x 4000 11.8, here 14.4.
+#include "eval_tiled_kernel.hpp"
+
+namespace ddcx {
+
+bool launch_eval_narrow(BSplinesPlan const& bs, Rules1D rules, int order, double* out, const double* coords, Layout xl,
+                        Layout pl, int64_t npts, const double* coef, Layout cl, int64_t nbatch, hipStream_t stream)
+{
+    int const degree = bs.view.degree;
+    if (order > 1 || degree < 2 || degree > 5) return false;
+    size_t const extra = (bs.view.uniform ? 0 : bs.knots_host.size()) * sizeof(double) +
+                         bs.cells_host.size() * sizeof(uint32_t);
+    // LDS of a tile with the given (odd) pitch
+    auto lds = [&](int pitch) { return size_t(bs.size()) * pitch * sizeof(double) + extra; };
+    int64_t const cus = cu_count();
+    bool const two = lds(9) <= tiled::kMaxLds / 2;
+    int lines = 0;
+    if (nbatch <= 4 * cus) lines = 4;
+    else if (nbatch <= 8 * cus) lines = 8;
+    else if (pl.rs == 1) lines = two ? 8 : 4;
+    else if (bs.view.uniform && nbatch <= 16 * cus && npts > 400) lines = 0;
+    else if (pl.rs % 16 != 0 || (two && (npts <= 512 || nbatch < 32 * cus))) lines = 8;
+    if (lines == 0 || lds(lines + 1) > tiled::kMaxLds) return false;
+    auto go = [&]<int D, int ORDER>() {
+        if (lines == 4)
+            tiled::launch_eval_tile<D, ORDER, 4, 512>(bs, rules, out, coords, xl, pl, npts, coef, cl, nbatch, 5, stream);
+        else
+            tiled::launch_eval_tile<D, ORDER, 8, 512>(bs, rules, out, coords, xl, pl, npts, coef, cl, nbatch, 9, stream);
+    };
+    auto pick = [&]<int D>() { order == 0 ? go.template operator()<D, 0>() : go.template operator()<D, 1>(); };
+    switch (degree) {
+    case 2: pick.template operator()<2>(); break;
+    case 3: pick.template operator()<3>(); break;
+    case 4: pick.template operator()<4>(); break;
+    default: pick.template operator()<5>(); break;
+    }
+    return true;
+}
+
+} // namespace ddcx

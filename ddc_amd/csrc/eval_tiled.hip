@@ -7,24 +7,27 @@
 // brackets in LDS, and then evaluates all the points of those lines with
 // coalesced coordinate loads and output stores.  HBM sees every coefficient,
 // coordinate and output once.  Two thread mappings:
-//  - batch-contiguous (LINE_MAJOR = false): lanes take consecutive lines, so
+//  - batch-contiguous (line_major = 0): lanes take consecutive lines, so
 //    tile rows and point rows are read as LB*8-byte runs;
-//  - interpolation-contiguous (LINE_MAJOR = true): the tile is read line by
+//  - interpolation-contiguous (line_major = 1): the tile is read line by
 //    line (size() contiguous doubles each) and the NT/LB threads of a line
 //    take consecutive points of it.
-// Values on plain batch-contiguous arrays take eval_stream_kernel, a
-// persistent form that loads the next tile while the current one is
-// evaluated.
+// Values and first derivatives on plain batch-contiguous arrays take
+// eval_stream_kernel, a persistent form that loads the next tile while the
+// current one is evaluated; small batches, short lines and interpolation-
+// contiguous arrays take narrower tiles (eval_narrow.hip).
 #include "eval_tiled_kernel.hpp"
 
 namespace ddcx {
 
 namespace {
 
+using tiled::basis_and_deriv;
 using tiled::kMaxLds;
 using tiled::lay;
 using tiled::load_tile;
-using tiled::point_value;
+using tiled::nonuniform_cells;
+using tiled::point_values;
 
 // Buffer resources (raw buffers, stride 0) for the streaming kernel: a load
 // at a byte offset at or past num_records returns 0 and a store there is
@@ -156,8 +159,7 @@ __global__ void __launch_bounds__(NT) eval_stream_kernel(BSplinesView b, Rules1D
 #pragma unroll
             for (int j = s * PS; j < (s + 1) * PS && j < PR; ++j) pf[j] = buffer_load<kNonTemporal>(rkn, cr(j, ltn));
             double y[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) y[u] = point_value<D, ORDER, KIND>(bl, knots, rules, xa[u], tl, pitch);
+            point_values<D, ORDER, KIND, U>(bl, knots, rules, xa, tl, pitch, y);
 #pragma unroll
             for (int u = 0; u < U; ++u) buffer_store<kNonTemporal>(y[u], ro, pt(s * U * ROWS + prow + u * ROWS, lt));
 #pragma unroll
@@ -177,11 +179,25 @@ __global__ void __launch_bounds__(NT) eval_stream_kernel(BSplinesView b, Rules1D
     }
 }
 
-// Adjoint of the value form on the same tiles: gx = w * f'(x) where the
-// spline itself is evaluated (0 where an extrapolation rule applies), and the
+// Adjoint of the value form on 8-line tiles: gx = w * f'(x) where the spline
+// itself is evaluated (0 where an extrapolation rule applies), and the
 // coefficient gradient of the LB lines accumulated in an LDS tile with LDS
 // atomics, then written once (every row, so no separate zeroing).
-template <int D, int LB, int NT>
+//
+// Two tiles in LDS leave room for 8 lines, 64-byte runs in batch-contiguous
+// arrays.  Neighbouring tiles on one XCD at the same time share their 128-byte
+// lines in its L2 (so the loads and stores are not non-temporal: with them quartic
+// 1024 x 20011 took 441 us instead of 309), one point per thread ahead keeps few
+// rows in flight, and the basis of the kernel's kind alone needs 96 registers
+// where the run-time choice spilled for quintic splines.  us, before -> after:
+// uniform quintic 1024 x 65536 999 -> 842 (rows contiguous 777 -> 621), cubic 60000
+// lines 676 -> 621 (623 -> 492; a form with one 16-line LDS tile and two passes
+// over the points took 656), non-uniform cubic 1024 x 65536 1086 -> 882 (932 ->
+// 677), quintic 1266 -> 1001 (1207 -> 884).  256 threads when lines are short (up
+// to 384 points; 8 lines of 100 points do not fill 1024 threads) and the batch is
+// not: 100 x 90001 196 -> 129 (197 -> 87), 300 x 90001 quintic 540 -> 397 (410 ->
+// 269); 500 x 60000 340 on 1024 threads, 359 on 256; 300 x 1000 8.9 and 10.8.
+template <int D, int LB, int NT, int KIND>
 __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rules1D rules,
                                                             const double* __restrict__ coords,
                                                             const double* __restrict__ w, double* __restrict__ gx,
@@ -195,12 +211,17 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
     double* kn = gt + size_t(ncoef) * pitch;
     uint32_t* cells = reinterpret_cast<uint32_t*>(kn + nknots);
     constexpr int ROWS = NT / LB;
-    constexpr int U = 4;
+    constexpr int U = 1;
     constexpr int TC = 16;
     int const tid = threadIdx.x;
     int const ln = line_major ? tid / ROWS : tid % LB;
     int const prow = line_major ? tid % ROWS : tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
+    // two tiles of 64-byte runs share their 128-byte lines: workgroups b and b +
+    // 8, which run on one XCD, take neighbouring tiles
+    static_assert(LB == 8);
+    unsigned const bx = blockIdx.x;
+    int64_t const line0 = int64_t(bx / 16 * 16 + bx % 8 * 2 + bx / 8 % 2) * LB;
+    if (line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
     int64_t const lc = active ? line : 0;
@@ -209,44 +230,70 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
     // coefficient tile (as in eval_tiled_kernel) and a zeroed gradient tile
     load_tile<LB, NT, TC>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
     for (int k = tid; k < ncoef * pitch; k += NT) gt[k] = 0.0;
-    if (!b.uniform) {
+    if constexpr (KIND != kUniformBasis) {
         for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
         for (int k = tid; k < b.nbucket; k += NT) cells[k] = b.cells[k];
     }
     __syncthreads();
-    const double* knots = b.uniform ? nullptr : kn;
+    const double* knots = KIND == kUniformBasis ? nullptr : kn;
     BSplinesView bl = b;
     bl.cells = b.nbucket > 0 ? cells : nullptr;
     if (active) {
         const double* tl = tile + ln;
         double* gl = gt + ln;
-        for (int64_t i = prow; i < npts; i += U * ROWS) {
+        // software pipeline: the next U points are read while the current ones
+        // are worked through; indices past the end read the last point
+        int const last = int(npts) - 1; // npts >= 64
+        uint32_t const prs = uint32_t(pl.rs);
+        const double* __restrict__ cp = coords + pb;
+        const double* __restrict__ wp = w + pb;
+        double* __restrict__ gp = gx + pb;
+        auto at = [&](int ii) { return uint64_t(uint32_t(min(ii, last))) * prs; };
+        double xn[U], wn[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            xn[u] = cp[at(prow + u * ROWS)];
+            wn[u] = wp[at(prow + u * ROWS)];
+        }
+        for (int i = prow; i <= last; i += U * ROWS) {
             double xa[U], wa[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                xa[u] = ii < npts ? coords[pb + ii * pl.rs] : 0.0;
-                wa[u] = ii < npts ? w[pb + ii * pl.rs] : 0.0;
+                xa[u] = xn[u];
+                wa[u] = wn[u];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                if (ii >= npts) continue;
-                double x = xa[u];
+                xn[u] = cp[at(i + (U + u) * ROWS)];
+                wn[u] = wp[at(i + (U + u) * ROWS)];
+            }
+            // bits: the spline is evaluated (not a Null rule's 0), a rule applies
+            uint32_t in = 0, rule = 0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
                 bool outside;
-                if (!apply_bc(bl, rules, x, outside)) {
-                    gx[pb + ii * pl.rs] = 0.0;
+                if (apply_bc(bl, rules, xa[u], outside)) in |= 1u << u;
+                if (outside) rule |= 1u << u;
+            }
+            int icell[U] = {};
+            if constexpr (KIND == kSafeNonUniform) nonuniform_cells<U>(bl, knots, xa, icell);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                int const ii = i + u * ROWS;
+                if (ii > last) continue;
+                if (!((in >> u) & 1u)) {
+                    gp[at(ii)] = 0.0;
                     continue;
                 }
-                double der[(D + 1) * 2];
-                int const jmin = eval_basis_and_n_derivs<D, 1, true>(bl, knots, x, der);
+                double v[D + 1], dv[D + 1];
+                int const jmin = basis_and_deriv<D, KIND>(bl, knots, xa[u], icell[u], v, dv);
                 double dy = 0.0;
 #pragma unroll
                 for (int k = 0; k < D + 1; ++k) {
-                    dy += tl[(jmin + k) * pitch] * der[k * 2 + 1];
-                    atomicAdd(&gl[(jmin + k) * pitch], wa[u] * der[k * 2]);
+                    dy += tl[(jmin + k) * pitch] * dv[k];
+                    atomicAdd(&gl[(jmin + k) * pitch], wa[u] * v[k]);
                 }
-                gx[pb + ii * pl.rs] = outside ? 0.0 : wa[u] * dy;
+                gp[at(ii)] = (rule >> u) & 1u ? 0.0 : wa[u] * dy;
             }
         }
     }
@@ -256,118 +303,22 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
     }
 }
 
-// Adjoint of the value form for batch-contiguous arrays on 16-line tiles (as
-// the evaluators; eval_vjp_tiled_kernel holds two tiles and so takes 8
-// lines), with one LDS tile used twice: first the coefficients, for
-// gx = w * f'(x) over all the tile's points; then the coefficient gradient,
-// accumulated over the same points read again and written once.  Same
-// arithmetic per point as eval_vjp_tiled_kernel.
-template <int D, int LB, int NT>
-__global__ void __launch_bounds__(NT) eval_vjp_2pass_kernel(BSplinesView b, Rules1D rules,
-                                                            const double* __restrict__ coords,
-                                                            const double* __restrict__ w, double* __restrict__ gx,
-                                                            Layout pl, int64_t npts, const double* __restrict__ coef,
-                                                            double* __restrict__ gcoef, Layout cl, int64_t nbatch,
-                                                            int ncoef, int pitch, int nknots)
-{
-    extern __shared__ double smem[];
-    double* tile = smem;
-    double* kn = tile + size_t(ncoef) * pitch;
-    uint32_t* cells = reinterpret_cast<uint32_t*>(kn + nknots);
-    constexpr int ROWS = NT / LB;
-    constexpr int U = 4;
-    constexpr int TC = 16;
-    int const tid = threadIdx.x;
-    int const ln = tid % LB;
-    int const prow = tid / LB;
-    int64_t const line0 = int64_t(blockIdx.x) * LB;
-    int64_t const line = line0 + ln;
-    bool const active = line < nbatch;
-    int64_t const lc = active ? line : 0;
-    int64_t const cb = lay(cl, 0, lc);
-    int64_t const pb = lay(pl, 0, lc);
-    load_tile<LB, NT, TC>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
-    if (!b.uniform) {
-        for (int k = tid; k < nknots; k += NT) kn[k] = b.knots[k];
-        for (int k = tid; k < b.nbucket; k += NT) cells[k] = b.cells[k];
-    }
-    __syncthreads();
-    const double* knots = b.uniform ? nullptr : kn;
-    BSplinesView bl = b;
-    bl.cells = b.nbucket > 0 ? cells : nullptr;
-    double* tl = tile + ln;
-    // pass 1: gx from the coefficient tile
-    if (active) {
-        for (int64_t i = prow; i < npts; i += U * ROWS) {
-            double xa[U], wa[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                xa[u] = ii < npts ? coords[pb + ii * pl.rs] : 0.0;
-                wa[u] = ii < npts ? w[pb + ii * pl.rs] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                if (ii >= npts) continue;
-                double x = xa[u];
-                bool outside;
-                if (!apply_bc(bl, rules, x, outside)) {
-                    gx[pb + ii * pl.rs] = 0.0;
-                    continue;
-                }
-                double der[(D + 1) * 2];
-                int const jmin = eval_basis_and_n_derivs<D, 1, true>(bl, knots, x, der);
-                double dy = 0.0;
-#pragma unroll
-                for (int k = 0; k < D + 1; ++k) dy += tl[(jmin + k) * pitch] * der[k * 2 + 1];
-                gx[pb + ii * pl.rs] = outside ? 0.0 : wa[u] * dy;
-            }
-        }
-    }
-    __syncthreads();
-    for (int k = tid; k < ncoef * pitch; k += NT) tile[k] = 0.0;
-    __syncthreads();
-    // pass 2: the coefficient gradient, the points read again
-    if (active) {
-        for (int64_t i = prow; i < npts; i += U * ROWS) {
-            double xa[U], wa[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                xa[u] = ii < npts ? coords[pb + ii * pl.rs] : 0.0;
-                wa[u] = ii < npts ? w[pb + ii * pl.rs] : 0.0;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                int64_t const ii = i + int64_t(u) * ROWS;
-                if (ii >= npts) continue;
-                double x = xa[u];
-                bool outside;
-                if (!apply_bc(bl, rules, x, outside)) continue;
-                double v[D + 1];
-                int const jmin = eval_basis<D, true>(bl, knots, x, v);
-#pragma unroll
-                for (int k = 0; k < D + 1; ++k) atomicAdd(&tl[(jmin + k) * pitch], wa[u] * v[k]);
-            }
-        }
-    }
-    __syncthreads();
-    if (active)
-        for (int r = prow; r < ncoef; r += ROWS) gcoef[cb + int64_t(r) * cl.rs] = tile[r * pitch + ln];
-}
-
-
-
-// eval_stream_kernel for the value form (and the first derivative of uniform
-// bases up to degree 3) when its shape fits: plain
-// batch-contiguous points and coefficients (element (row, line) at row * rs +
-// line), npts <= NST * U * ROWS, size() <= PR * ROWS, buffers below 4 GiB
-// including the offsets of the point slots past the end of a line.  Uniform
-// bases: 512 threads, 8 points per thread and stage, 33 prefetch rows; non-
-// uniform bases (whose cell search wants more waves to hide its dependent
-// LDS reads): 768 threads, 4 points per thread and stage, 22 prefetch rows,
-// degrees up to 3.
+// eval_stream_kernel for the value form and the first derivative (up to degree
+// 3) when its shape fits: plain batch-contiguous points and coefficients
+// (element (row, line) at row * rs + line), npts <= NST * U * ROWS, size() <= PR *
+// ROWS, buffers below 4 GiB including the offsets of the point slots past the end
+// of a line.  Uniform bases: 512 threads, 33 prefetch rows; non-uniform bases
+// (whose cell search wants more waves to hide its dependent LDS reads): 768
+// threads, 22 prefetch rows, degrees up to 3.
+//
+// U = 2 points per thread and stage: 64 (or 96) rows of each array at a time.
+// The workgroups walk the rows nearly together, and the fewer rows are in flight
+// the fewer DRAM pages compete: a plain copy in 16-line tiles at this stride
+// runs at 4.0 TB/s with 512 rows in flight per workgroup and at 4.7 with 128 to
+// 256.  us at 1024 x 65536 for U = 8 / 4 / 2 / 1: cubic 369 / 356 / 351 / 376,
+// quintic 400 / 382 / 378 / 387; 300 x 100000 284 / 243 / 232 / 247; first
+// derivative of cubic 355 (U = 4) / 349 / 341; non-uniform cubic 457 (U = 4) /
+// 439 / 434.
 template <int D, int ORDER>
 bool launch_stream(BSplinesPlan const& bs, Rules1D rules, double* out, const double* coords, Layout pl,
                    int64_t npts, const double* coef, Layout cl, int64_t nbatch, hipStream_t stream)
@@ -406,19 +357,24 @@ bool launch_stream(BSplinesPlan const& bs, Rules1D rules, double* out, const dou
         hip_check(hipGetLastError(), "eval_stream_kernel launch");
         return true;
     };
+    bool const safe = bs.safe_products && b.nbucket > 0;
+    // stages for at least npts points: 512, 768 or 1024 (uniform), 768 or 1152
+    auto uniform = [&] {
+        return npts <= 16 * 32   ? go.template operator()<kUniformBasis, 512, 2, 8, 33>()
+               : npts <= 24 * 32 ? go.template operator()<kUniformBasis, 512, 2, 12, 33>()
+                                 : go.template operator()<kUniformBasis, 512, 2, 16, 33>();
+    };
+    auto nonuniform = [&] {
+        return npts <= 16 * 48 ? go.template operator()<kSafeNonUniform, 768, 2, 8, 22>()
+                               : go.template operator()<kSafeNonUniform, 768, 2, 12, 22>();
+    };
     if constexpr (ORDER == 0) {
-        if (b.uniform)
-            return npts <= 2 * 8 * 32 ? go.template operator()<kUniformBasis, 512, 8, 2, 33>()
-                                      : go.template operator()<kUniformBasis, 512, 8, 4, 33>();
+        if (b.uniform) return uniform();
         if constexpr (D <= 3) // higher degrees spill in this form and keep eval_tiled_kernel
-            return npts <= 4 * 4 * 48 ? go.template operator()<kNonUniformBasis, 768, 4, 4, 22>()
-                                      : go.template operator()<kNonUniformBasis, 768, 4, 6, 22>();
+            if (safe) return nonuniform();
     } else if constexpr (D <= 3) {
-        // the first derivative's basis takes more registers: 4 points per
-        // thread and stage; uniform bases only (the non-uniform form spills)
-        if (b.uniform)
-            return npts <= 4 * 4 * 32 ? go.template operator()<kUniformBasis, 512, 4, 4, 33>()
-                                      : go.template operator()<kUniformBasis, 512, 4, 8, 33>();
+        if (safe) return nonuniform();
+        if (b.uniform) return uniform();
     }
     return false;
 }
@@ -477,7 +433,7 @@ bool launch_eval_tiled(BSplinesPlan const& bs, Rules1D rules, int order, double*
     if ((pl.rs == 1) != (cl.rs == 1)) return false;
     // 32-bit point indices and point strides in the kernel
     if (npts >= (int64_t(1) << 30) || pl.rs >= (int64_t(1) << 32) || xl.rs >= (int64_t(1) << 32)) return false;
-    bool launched = launch_eval_small(bs, rules, order, out, coords, xl, pl, npts, coef, cl, nbatch, stream);
+    bool launched = launch_eval_narrow(bs, rules, order, out, coords, xl, pl, npts, coef, cl, nbatch, stream);
     if (launched) return true;
     dispatch_degree(bs.view.degree, [&]<int D>() {
         auto ord = [&]<int O>() {
@@ -500,6 +456,8 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
 {
     if (npts < 64 || nbatch < 8) return false;
     if ((pl.rs == 1) != (cl.rs == 1)) return false;
+    // 32-bit point indices and point strides in the kernels
+    if (npts >= (int64_t(1) << 30) || pl.rs >= (int64_t(1) << 32)) return false;
     int const ncoef = bs.size();
     if (ncoef > 2560) return false;
     int const nknots = bs.view.uniform ? 0 : int(bs.knots_host.size());
@@ -512,42 +470,24 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
     else return false;
     bool const line_major = pl.rs == 1;
     bool launched = false;
-    if (!line_major && nbatch >= 16 * 2 * int64_t(cu_count()) && b.uniform && b.degree <= 3) {
-        // batch-contiguous, uniform bases up to degree 3, at least two tiles
-        // per CU: 16-line tiles, one LDS tile used for both passes (measured
-        // faster than the 8-line kernel there; with the dearer basis of
-        // non-uniform or quintic splines, computing it twice costs more than
-        // the wider tile gains, and small batches want the 8-line kernel's
-        // twice as many workgroups)
-        size_t const lds2 = size_t(ncoef) * 17 * sizeof(double) + extra;
-        if (lds2 <= kMaxLds) {
-            dispatch_degree(b.degree, [&]<int D>() {
-                constexpr int LB = 16, NT = 1024;
-                auto kern = eval_vjp_2pass_kernel<D, LB, NT>;
-                hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, int(lds2)),
-                          "hipFuncSetAttribute");
-                int64_t const blocks = (nbatch + LB - 1) / LB;
-                hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds2, stream, b, rules, coords, w, gx, pl,
-                                   npts, coef, gcoef, cl, nbatch, ncoef, 17, nknots);
-                hip_check(hipGetLastError(), "eval_vjp_2pass_kernel launch");
-                launched = true;
-            });
-            if (launched) return true;
-        }
-    }
     dispatch_degree(b.degree, [&]<int D>() {
-        constexpr int LB = 8, NT = 1024;
-        auto kern = eval_vjp_tiled_kernel<D, LB, NT>;
-        size_t const lds = lds_of(pitch);
-        hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
-                  "hipFuncSetAttribute");
-        int64_t const blocks = (nbatch + LB - 1) / LB;
-        hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, b, rules, coords, w, gx, pl,
-                           npts, coef, gcoef, cl, nbatch, ncoef, pitch, nknots, line_major ? 1 : 0);
-        hip_check(hipGetLastError(), "eval_vjp_tiled_kernel launch");
-        launched = true;
+        auto go = [&]<int NT>() {
+            constexpr int LB = 8;
+            auto kern = b.uniform ? eval_vjp_tiled_kernel<D, LB, NT, kUniformBasis>
+                        : bs.safe_products && b.nbucket > 0 ? eval_vjp_tiled_kernel<D, LB, NT, kSafeNonUniform>
+                                                            : eval_vjp_tiled_kernel<D, LB, NT, kNonUniformBasis>;
+            size_t const lds = lds_of(pitch);
+            hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),
+                      "hipFuncSetAttribute");
+            int64_t const blocks = ((nbatch + LB - 1) / LB + 15) / 16 * 16;
+            hipLaunchKernelGGL(kern, dim3(unsigned(blocks)), dim3(NT), lds, stream, b, rules, coords, w, gx, pl, npts,
+                               coef, gcoef, cl, nbatch, ncoef, pitch, nknots, line_major ? 1 : 0);
+            hip_check(hipGetLastError(), "eval_vjp_tiled_kernel launch");
+            launched = true;
+        };
+        if (npts <= 384 && nbatch > 8 * int64_t(cu_count())) go.template operator()<256>();
+        else go.template operator()<1024>();
     });
     return launched;
 }

@@ -1,5 +1,5 @@
 // The LDS-staged batched evaluation kernel (described in eval_tiled.hip) and
-// its launcher, shared by eval_tiled.hip and eval_small.hip.
+// its launcher, shared by eval_tiled.hip and eval_narrow.hip.
 #pragma once
 
 #include "tiled_common.hpp"
@@ -9,35 +9,120 @@ namespace tiled {
 
 constexpr size_t kMaxLds = 160 * 1024;
 
-// One point's value (ORDER 0, with the extrapolation rules) or derivative from
-// its line's tile.
+// nonuniform_cell of U points at once, without branches between them: every
+// step of the search reads one knot per point, so the U chains of dependent LDS
+// reads overlap, and a wave leaves when its widest bracket is searched.  (One
+// point after the other, each in its own loop, the chains follow each other.)
+// The bases staged here have brackets whenever they have fewer than 65536 cells.
+template <int U>
+__device__ __forceinline__ void nonuniform_cells(BSplinesView const& b, const double* kn, double const (&x)[U],
+                                                 int (&icell)[U])
+{
+    int n[U];
+    int widest = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        uint32_t const e = b.cells[bucket_of(b, b.nbucket, b.inv_bucket, x[u])];
+        icell[u] = b.degree + int(e & 0xffffu);
+        n[u] = int(e >> 16) - int(e & 0xffffu);
+        widest = max(widest, n[u]);
+    }
+    while (__any(widest > 0)) {
+        widest = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int const half = (n[u] + 1) >> 1; // 0 once n is 0: the cell's own lower knot, no move
+            bool const up = kn[icell[u] + half] <= x[u];
+            icell[u] += up ? half : 0;
+            n[u] = up ? n[u] - half : half - 1;
+            widest = max(widest, n[u]);
+        }
+    }
+}
+
+// The value (ORDER 0) or derivative of a point in a known cell (kSafeNonUniform,
+// orders 0 and 1) or of any point.
 template <int D, int ORDER, int KIND>
-__device__ __forceinline__ double point_value(BSplinesView const& b, const double* kn, Rules1D rules, double x,
-                                              const double* tile, int pitch)
+__device__ __forceinline__ double tile_value(BSplinesView const& b, const double* kn, double x, int icell,
+                                             const double* tile, int pitch)
 {
     double v[D + 1];
     int jmin;
-    if constexpr (ORDER == 0) {
-        if (b.periodic) {
-            if (x < b.rmin || x > b.rmax) x -= floor((x - b.rmin) / b.length) * b.length;
-        } else if (x < b.rmin) {
-            if (rules.lower == DDCX_EXTRAP_NULL) return 0.0;
-            x = rules.pos_lower;
-        } else if (x > b.rmax) {
-            if (rules.upper == DDCX_EXTRAP_NULL) return 0.0;
-            x = rules.pos_upper;
-        }
+    if constexpr (ORDER == 0 && KIND == kSafeNonUniform) {
+        nonuniform_basis<D, true, true>(kn, icell, x, v);
+        jmin = icell - D;
+    } else if constexpr (ORDER == 0) {
         jmin = eval_basis<D, true, KIND>(b, kn, x, v);
+    } else if constexpr (ORDER == 1 && KIND == kSafeNonUniform) {
+        double values[D + 1];
+        nonuniform_basis_deriv<D, true>(kn, icell, x, values, v);
+        jmin = icell - D;
     } else {
         double der[(D + 1) * (ORDER + 1)];
         jmin = eval_basis_and_n_derivs<D, ORDER, true, KIND>(b, kn, x, der);
 #pragma unroll
         for (int i = 0; i < D + 1; ++i) v[i] = der[i * (ORDER + 1) + ORDER];
     }
-    double y = 0.0;
+    double s = 0.0;
 #pragma unroll
-    for (int i = 0; i < D + 1; ++i) y += tile[(jmin + i) * pitch] * v[i];
-    return y;
+    for (int i = 0; i < D + 1; ++i) s += tile[(jmin + i) * pitch] * v[i];
+    return s;
+}
+
+// Values v and first derivatives dv of the splines on x's cell; returns the
+// first spline.  icell: x's cell (kSafeNonUniform; found before, for several
+// points at once).
+template <int D, int KIND>
+__device__ __forceinline__ int basis_and_deriv(BSplinesView const& b, const double* kn, double x, int icell, double* v,
+                                               double* dv)
+{
+    if constexpr (KIND == kSafeNonUniform) {
+        nonuniform_basis_deriv<D, true>(kn, icell, x, v, dv);
+        return icell - D;
+    } else {
+        double der[(D + 1) * 2];
+        int const jmin = eval_basis_and_n_derivs<D, 1, true, KIND>(b, kn, x, der);
+#pragma unroll
+        for (int k = 0; k < D + 1; ++k) {
+            v[k] = der[k * 2];
+            dv[k] = der[k * 2 + 1];
+        }
+        return jmin;
+    }
+}
+
+// The values (ORDER 0, with the extrapolation rules) or derivatives of U points
+// of one line from its tile.
+template <int D, int ORDER, int KIND, int U>
+__device__ __forceinline__ void point_values(BSplinesView const& b, const double* kn, Rules1D rules, double (&x)[U],
+                                             const double* tile, int pitch, double (&y)[U])
+{
+    if constexpr (KIND == kSafeNonUniform && ORDER <= 1) {
+        int icell[U];
+        uint32_t zero = 0; // bit u: the Null rule gives 0
+        if constexpr (ORDER == 0) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                bool outside;
+                if (!apply_bc(b, rules, x[u], outside)) zero |= 1u << u;
+            }
+        }
+        nonuniform_cells<U>(b, kn, x, icell);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            double const s = tile_value<D, ORDER, KIND>(b, kn, x[u], icell[u], tile, pitch);
+            y[u] = (zero >> u) & 1u ? 0.0 : s;
+            // keeps the knots and divisors of one point at a time in registers
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            bool outside;
+            if (ORDER == 0 && !apply_bc(b, rules, x[u], outside)) y[u] = 0.0;
+            else y[u] = tile_value<D, ORDER, KIND>(b, kn, x[u], 0, tile, pitch);
+        }
+    }
 }
 
 // The coefficient tile of a workgroup's lines to LDS: thread (line ln, row
@@ -79,8 +164,10 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
     constexpr int ROWS = NT / LB;
     // points per pipeline stage per thread: as many as the registers hold
     // without spilling (derivative tables of non-uniform bases are the largest)
-    constexpr int U = LB < 16 && NT < 1024 ? 4
+    constexpr int U = ORDER == 1 && KIND == kNonUniformBasis ? 1
+                      : LB < 16 && NT < 1024 ? 4
                       : ORDER == 0 ? 8
+                      : ORDER == 1 && KIND == kSafeNonUniform ? 8
                       : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
                                               : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
     constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
@@ -130,8 +217,7 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
 #pragma unroll
         for (int u = 0; u < U; ++u) xb[u] = __builtin_nontemporal_load(&cp[atx(i + (U + u) * ROWS)]);
         double y[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) y[u] = point_value<D, ORDER, KIND>(bl, knots, rules, xa[u], tl, pitch);
+        point_values<D, ORDER, KIND, U>(bl, knots, rules, xa, tl, pitch, y);
 #pragma unroll
         for (int u = 0; u < U; ++u) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
 #pragma unroll
@@ -149,7 +235,9 @@ void launch_eval_tile(BSplinesPlan const& bs, Rules1D rules, double* out, const 
     BSplinesView const b = bs.device_view();
     size_t const lds = (size_t(ncoef) * pitch + nknots) * sizeof(double) + size_t(b.nbucket) * sizeof(uint32_t);
     auto kern = b.uniform ? eval_tiled_kernel<D, ORDER, LB, NT, kUniformBasis>
-                          : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis>;
+                : ORDER <= 1 && bs.safe_products && b.nbucket > 0
+                    ? eval_tiled_kernel<D, ORDER, LB, NT, ORDER <= 1 ? kSafeNonUniform : kNonUniformBasis>
+                    : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis>;
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   int(lds)),
               "hipFuncSetAttribute");

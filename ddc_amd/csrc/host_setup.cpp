@@ -539,17 +539,17 @@ std::shared_ptr<BSplinesPlan> make_bsplines(ddcx_bsplines_desc const& d)
     v.nbucket = 0;
     v.inv_bucket = 0.0;
     if (!v.uniform && d.ncells < 65536) {
-        // one bucket per cell on average; bucket k covers
-        // [rmin + k w, rmin + (k+1) w), w = (rmax - rmin) / nbucket
+        // one bucket per cell on average; cell c reaches from the bucket of its
+        // lower break point to that of its upper one
         int const nbk = d.ncells;
-        double const w = v.length / nbk;
         p->inv_bucket = double(nbk) / v.length;
         p->cells_host.resize(nbk);
+        auto bucket = [&](int c) { return bucket_of(v, nbk, p->inv_bucket, p->knots_host[D + c]); };
+        p->safe_products = products_safe(D, d.ncells, p->knots_host.data());
+        int lo = 0, hi = 0;
         for (int k = 0; k < nbk; ++k) {
-            double const e0 = v.rmin + double(k) * w;
-            double const e1 = std::min(v.rmin + double(k + 1) * w, v.rmax);
-            int const lo = nonuniform_cell(v, p->knots_host.data(), e0) - D;
-            int const hi = nonuniform_cell(v, p->knots_host.data(), e1) - D;
+            while (lo + 1 < d.ncells && bucket(lo + 1) < k) ++lo;
+            while (hi + 1 < d.ncells && bucket(hi + 1) <= k) ++hi;
             p->cells_host[k] = uint32_t(lo) | (uint32_t(hi) << 16);
         }
     }

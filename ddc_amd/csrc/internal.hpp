@@ -140,6 +140,7 @@ struct BSplinesPlan {
     // whole range
     std::vector<uint32_t> cells_host;
     double inv_bucket = 0.0;
+    bool safe_products = false; // products_safe of a non-uniform basis
     DeviceBuffer cells_dev;
     std::vector<double> integrals; // integrals() over the full spline domain (size() entries)
     DeviceBuffer integrals_dev;
@@ -419,9 +420,9 @@ void launch_build_vjp(BuilderPlan const& p, const double* gcoef, Layout cl, doub
 bool launch_eval_tiled(BSplinesPlan const& bs, Rules1D rules, int order, double* out, const double* coords,
                        Layout xl, Layout pl, int64_t npts, const double* coef, Layout cl, int64_t nbatch,
                        hipStream_t stream);
-// the same for small batches (eval_small.hip)
-bool launch_eval_small(BSplinesPlan const& bs, Rules1D rules, int order, double* out, const double* coords, Layout xl,
-                       Layout pl, int64_t npts, const double* coef, Layout cl, int64_t nbatch, hipStream_t stream);
+// the same for small batches (eval_narrow.hip)
+bool launch_eval_narrow(BSplinesPlan const& bs, Rules1D rules, int order, double* out, const double* coords, Layout xl,
+                        Layout pl, int64_t npts, const double* coef, Layout cl, int64_t nbatch, hipStream_t stream);
 bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* coords, const double* w,
                            double* gx, Layout pl, int64_t npts, const double* coef, double* gcoef, Layout cl,
                            int64_t nbatch, hipStream_t stream);

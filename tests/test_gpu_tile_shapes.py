@@ -106,3 +106,66 @@ def test_eval_thresholds(case, axis, cuda):
         ev.deriv(1, out, dev(x), dev(coef), axis=axis)
         got = out.cpu().numpy() if axis == 0 else out.cpu().numpy().T
         assert rel_err(got, orc.eval(x, coef, deriv=1, extrap=("constant", "null"))) <= 10 * TOL, nbatch
+
+
+@pytest.mark.parametrize("case", [Case(3, True, P, ncells=450), Case(4, False, G, ncells=600, mesh="jitter"),
+                                  Case(3, True, G, ncells=1100), Case(5, False, H, ncells=1100, mesh="jitter")],
+                         ids=lambda c: c.id)
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("npts,extra", [(450, 1), (600, 15)])
+def test_eval_wide_batches(case, axis, npts, extra, cuda):
+    """Past the small batches: the 16-line tile, the streaming kernel's 768-point
+    form (rows that start at 128-byte lines) and the narrow tiles of the others."""
+    import torch
+
+    import ddc_amd as D
+
+    orc = case.oracle()
+    bs, _ = case.product()
+    ev = D.SplineEvaluator(bs, D.ConstantExtrapolationRule(), D.NullExtrapolationRule())
+    cus = torch.cuda.get_device_properties(cuda).multi_processor_count
+    rng = np.random.default_rng(4)
+    for nbatch in (8 * cus + extra, 32 * cus + 16 * extra):
+        coef = rng.standard_normal((orc.size, nbatch))
+        if case.periodic:
+            coef[-case.degree:] = coef[:case.degree]
+        x = rng.uniform(0.0, 1.0, (npts, nbatch))
+        tx, tc = ((torch.from_numpy(a).to(cuda) if axis == 0 else torch.from_numpy(np.ascontiguousarray(a.T)).to(cuda))
+                  for a in (x, coef))
+        out = torch.full_like(tx, float("nan"))
+        for order in (0, 1):
+            (ev(out, tx, tc, axis=axis) if order == 0 else ev.deriv(1, out, tx, tc, axis=axis))
+            got = out.cpu().numpy() if axis == 0 else out.cpu().numpy().T
+            assert rel_err(got, orc.eval(x, coef, deriv=order, extrap=("constant", "null"))) <= TOL * 10 ** order
+
+
+@pytest.mark.parametrize("case", [Case(3, True, P, ncells=100), Case(5, True, G, ncells=128),
+                                  Case(3, False, G, ncells=128), Case(5, False, P, ncells=90, mesh="jitter")],
+                         ids=lambda c: c.id)
+@pytest.mark.parametrize("axis", [0, 1])
+def test_eval_vjp_short_lines(case, axis, cuda):
+    """The adjoint on 256 threads (up to 384 points) and on 1024, with odd numbers
+    of 8-line tiles; coordinates <= 1e-13, coefficients <= 1e-12."""
+    import torch
+
+    import ddc_amd as D
+
+    orc = case.oracle()
+    bs, _ = case.product()
+    ev = D.SplineEvaluator(bs, D.ConstantExtrapolationRule(), D.NullExtrapolationRule())
+    nbatch = 8 * torch.cuda.get_device_properties(cuda).multi_processor_count + 13
+    rng = np.random.default_rng(3)
+
+    def dev(a):
+        return torch.from_numpy(np.ascontiguousarray(a if axis == 0 else a.T)).to(cuda)
+
+    for npts in (64, 384, 385):
+        coef = rng.standard_normal((orc.size, nbatch))
+        if case.periodic:
+            coef[-case.degree:] = coef[:case.degree]
+        x, w = rng.uniform(-0.02, 1.02, (npts, nbatch)), rng.standard_normal((npts, nbatch))
+        gx, gc = torch.full_like(dev(x), float("nan")), torch.full_like(dev(coef), float("nan"))
+        ev.eval_vjp(dev(x), dev(w), dev(coef), gx, gc, axis=axis)
+        got_c, got_x = ((t.cpu().numpy() if axis == 0 else t.cpu().numpy().T) for t in (gc, gx))
+        ref_c, ref_x = orc.eval_vjp(x, w, coef, extrap=("constant", "null"))
+        assert rel_err(got_x, ref_x) <= 1e-13 and rel_err(got_c, ref_c) <= 1e-12, npts
