@@ -30,6 +30,16 @@ namespace tiled_build {
 
 using namespace tiled;
 
+// Long lines in batch-contiguous arrays (the whole table in LDS): one workgroup
+// per resident place walks the tiles, so that the table and border data are
+// staged once, and each row of the next tile is requested as the current one's
+// row is stored.  us, a workgroup per tile -> this: uniform cubic 1024 x 65536
+// 247 -> 241, quintic 302 -> 281, non-uniform cubic 285 -> 271, cubic 300 x 100000
+// 226 -> 209, 512 x 8192 21.8 -> 19.4.  With the table staged in halves (quintic
+// Hermite 2048 x 32768) the staging waits behind the tile's loads: 383 -> 418, so
+// those keep a workgroup per tile.
+constexpr bool loops(int L, bool ic, int tmode) { return L == 32 && !ic && tmode == 1; }
+
 // TMODE: 0 row table read from global memory (L2), 1 staged in LDS whole,
 // 2 staged in LDS one sweep's fields at a time (tables too large for 1)
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int TMODE, bool IC>
@@ -45,6 +55,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     constexpr bool TLDS = TMODE != 0;
     constexpr bool MLDS = TMODE == 1 && transfer_in_lds(LB);
     constexpr int RSF = KF + (FDIV ? 1 : 0), RSB = KB + 1; // split records
+    constexpr bool LOOP = loops(L, IC, TMODE);
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
     __shared__ double b2s[kNbMax][LB];
@@ -53,26 +64,33 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     extern __shared__ double rt_lds[];
 
     int const tid = threadIdx.x;
-    int const ln = tid % LB;
-    int const seg = tid / LB;
-    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    int ln = tid % LB;
+    int seg = tid / LB;
+    int64_t line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
     if (LB < 16 && line0 >= nbatch) return; // whole workgroup
-    int64_t const line = line0 + ln;
-    bool const active = line < nbatch;
-    int64_t const lc = active ? line : line0;
-    int64_t const vb = lay(vl, 0, lc);
-    int64_t const cb = lay(cl, 0, lc);
-    int const r0 = seg * L;
+    int r0 = seg * L;
     int const nq = tv.nq;
     constexpr int RS = KF + KB + 1 + (FDIV ? 1 : 0); // row record length, fixed by the band shape
     // Workgroup-uniform bases plus 32-bit per-lane offsets (the host checks
     // that every offset of a tile fits), so that each load/store needs one
     // address register instead of two.
-    const double* __restrict__ vwg = vals + lay(vl, 0, line0);
-    double* __restrict__ cwg = coef + lay(cl, 0, line0);
-    uint32_t const vlo = uint32_t(vb - lay(vl, 0, line0)) + uint32_t(tv.q0 + r0) * uint32_t(vl.rs);
-    uint32_t const clo = uint32_t(cb - lay(cl, 0, line0));
-    uint32_t const vrs = uint32_t(vl.rs), crs = uint32_t(cl.rs);
+    const double* __restrict__ vwg;
+    double* __restrict__ cwg;
+    uint32_t vlo, clo; // of the line's first main-block row of this segment, and of its coefficient row 0
+    bool active;
+    // this thread's line of the tile that starts at l0 (lines past the batch: the first)
+    auto line_of = [&](int64_t l0) { return l0 + ln < nbatch ? l0 + ln : l0; };
+    auto at_vals = [&](int64_t l0) {
+        vwg = vals + lay(vl, 0, l0);
+        vlo = uint32_t(lay(vl, 0, line_of(l0)) - lay(vl, 0, l0)) + uint32_t(tv.q0 + r0) * uint32_t(vl.rs);
+    };
+    auto at_coef = [&](int64_t l0) {
+        active = l0 + ln < nbatch;
+        cwg = coef + lay(cl, 0, l0);
+        clo = uint32_t(lay(cl, 0, line_of(l0)) - lay(cl, 0, l0));
+    };
+    at_vals(line0);
+    at_coef(line0);
 
     // dynamic LDS: the row table (TLDS) in the space of the staging area (IC,
     // LB x stage_pitch doubles, in use before the table is loaded and after its
@@ -86,8 +104,27 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     uint32_t* loff = reinterpret_cast<uint32_t*>(
         (TLDS ? mtr : gpad) + (MLDS ? K * (tv.wf * KF * KF + tv.wb * KB * KB) : 0));
     int const nl = int(min<int64_t>(LB, nbatch - line0));
+    int off = bv.offset;
+    int nbas = bv.nbasis;
+    int const nb = tv.nb;
 
     double y[L];
+    // Row i of the segment.  Past the main block (last segments): row nq - 1, in
+    // bounds; the table's padding rows couple it to nothing and it is not
+    // stored.  Values and coefficients are touched once: non-temporal loads and
+    // stores keep them from displacing what the next kernel reads.
+    int last = nq - 1 - r0;
+    uint32_t vrs = uint32_t(vl.rs), crs = uint32_t(cl.rs);
+    auto load_row = [&](int i) { return __builtin_nontemporal_load(&vwg[vlo + uint32_t(min(i, last)) * vrs]); };
+    // the border rows' right-hand side and the segment's part of the border
+    // step do not depend on the sweeps: read first, ahead of the tile
+    auto load_border = [&](int64_t l0) {
+        if (seg >= nb || l0 + ln >= nbatch) return 0.0;
+        return rhs_src(bv, vals, vl, lay(vl, 0, l0 + ln), dl, dr, dlay, lay(dlay, 0, l0 + ln),
+                       seg < tv.top ? seg : nq + seg);
+    };
+    double b2 = load_border(line0);
+    SegBorder sb = tv.seg[seg];
     if constexpr (IC) {
         constexpr int PER = LB * SR / NT; // staged elements per thread and chunk
         if (tid < LB) {
@@ -116,65 +153,46 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
             }
             __syncthreads();
         }
-    } else if (r0 + L <= nq) {
-        // values and coefficients are touched once: non-temporal loads and
-        // stores keep them from displacing what the next kernel reads
+    } else if (last >= L - 1) {
 #pragma unroll
         for (int i = 0; i < L; ++i) y[i] = __builtin_nontemporal_load(&vwg[vlo + uint32_t(i) * vrs]);
     } else {
-        // last segments: rows at or past nq read row nq - 1 (in bounds) and are zeroed
-        uint32_t const vl0 = vlo - uint32_t(r0) * vrs; // row q0 of this line
 #pragma unroll
-        for (int i = 0; i < L; ++i) {
-            double const v = __builtin_nontemporal_load(&vwg[vl0 + uint32_t(min(r0 + i, nq - 1)) * vrs]);
-            y[i] = r0 + i < nq ? v : 0.0;
-        }
+        for (int i = 0; i < L; ++i) y[i] = load_row(i);
     }
 
-    // the border rows' right-hand side and the segment's part of the border
-    // step do not depend on the sweeps: read now, with the tile
-    double b2 = 0.0;
-    if (seg < tv.nb && active)
-        b2 = rhs_src(bv, vals, vl, vb, dl, dr, dlay, lay(dlay, 0, lc), seg < tv.top ? seg : tv.nq + seg);
-    SegBorder const sb = tv.seg[seg];
+    if constexpr (TMODE == 1) {
+        stage_table<NT, K * L, RS>(tv.rt, rt_lds, tid);
+        if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
+    }
+    stage_border<NT, TLDS>(tv, bl, gpad, tid);
 
-    // per-row table and border data: staged in LDS when they fit (one copy
-    // per workgroup)
+    // LOOP: the workgroup walks the tiles blockIdx.x, blockIdx.x + gridDim.x, ...
+    for (;;) {
+    // the compiler is not to keep every row's offsets in registers across the loop
+    if constexpr (LOOP) {
+        asm volatile("" : "+v"(last), "+s"(vrs), "+s"(crs), "+v"(r0), "+v"(seg), "+v"(ln));
+        asm volatile("" : "+v"(sb.mask), "+v"(sb.slot0), "+v"(sb.gblk), "+s"(off), "+s"(nbas));
+    }
+    if (seg < nb) b2s[seg][ln] = b2;
     if constexpr (TMODE == 2) {
         // the forward sweep's fields, then (after its closing barrier) the
         // backward sweep's, in the same LDS region
         stage_half<NT, KF, KB, FDIV, true>(tv.rt, RS, K * L, rt_lds, tid);
-        stage_border<NT, true>(tv, bl, gpad, tid);
-        if (seg < tv.nb) b2s[seg][ln] = b2;
         __syncthreads();
         tiled_forward<LB, K, L, KF, FDIV, 0, KF>(y, rt_lds + r0 * RSF, RSF, tv.Mf, tv.wf, ex, seg, ln);
         stage_half<NT, KF, KB, FDIV, false>(tv.rt, RS, K * L, rt_lds, tid);
         __syncthreads();
         tiled_backward<LB, K, L, KB, BDIVF, 0, KB>(y, rt_lds + r0 * RSB, RSB, tv.Mb, tv.wb, ex, seg, ln);
     } else {
-        const double* T;
-        if constexpr (TLDS) {
-            stage_table<NT, K * L, RS>(tv.rt, rt_lds, tid);
-            if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
-            stage_border<NT, true>(tv, bl, gpad, tid);
-            if (seg < tv.nb) b2s[seg][ln] = b2;
-            __syncthreads();
-            T = rt_lds + r0 * RS;
-        } else {
-            stage_border<NT, false>(tv, bl, gpad, tid); // without the Q^-1 gamma blocks
-            if (seg < tv.nb) b2s[seg][ln] = b2;
-            __syncthreads();
-            T = tv.rt + size_t(r0) * RS;
-        }
+        __syncthreads();
+        const double* const T = TLDS ? rt_lds + r0 * RS : tv.rt + size_t(r0) * RS;
         const double* const Mf = MLDS ? mtr : tv.Mf;
         const double* const Mb = MLDS ? mtr + K * tv.wf * KF * KF : tv.Mb;
         tiled_sweeps<LB, K, L, KF, KB, FDIV, BDIVF, KE>(y, T, RS, Mf, tv.wf, Mb, tv.wb, ex, seg, ln);
     }
 
     // ---------------- border (2x2 blocks) ----------------
-    int const nb = tv.nb;
-    int const off = bv.offset;
-    int const nbas = bv.nbasis;
     if (nb > 0) {
         gather_coupled<LB, L>(y, sb, lamx, ln);
         __syncthreads();
@@ -183,10 +201,10 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
             x2s[seg][ln] = x2;
             if (active) {
                 int const j = (seg < tv.top ? seg : nq + seg) + off;
-                coef[cb + int64_t(j) * cl.rs] = x2;
+                cwg[clo + uint32_t(j) * crs] = x2;
                 if (bv.periodic) {
-                    if (j - nbas >= 0) coef[cb + int64_t(j - nbas) * cl.rs] = x2;
-                    if (j + nbas < nbas + bv.degree) coef[cb + int64_t(j + nbas) * cl.rs] = x2;
+                    if (j - nbas >= 0) cwg[clo + uint32_t(j - nbas) * crs] = x2;
+                    if (j + nbas < nbas + bv.degree) cwg[clo + uint32_t(j + nbas) * crs] = x2;
                 }
             }
         }
@@ -219,30 +237,45 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
             __syncthreads();
         }
     }
-    if (active) {
-        uint32_t const c0 = clo + uint32_t(tv.top + r0 + off) * crs;
-        if constexpr (IC) {
-            // rows stored above
-        } else if (r0 + L <= nq) {
+    if (active && bv.periodic && (r0 < bv.degree || r0 + L > nbas - off)) {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            int const prow = tv.top + r0 + i;
+            if (prow < nq) {
+                int const j0 = prow + off - nbas;
+                if (j0 >= 0) cwg[clo + uint32_t(j0) * crs] = y[i];
+                int const j2 = prow + off + nbas;
+                if (j2 < nbas + bv.degree) cwg[clo + uint32_t(j2) * crs] = y[i];
+            }
+        }
+    }
+    if constexpr (IC) return; // rows stored above
+    uint32_t const c0 = clo + uint32_t(tv.top + r0 + off) * crs;
+    int64_t const next = line0 + int64_t(gridDim.x) * LB;
+    if (!LOOP || next >= nbatch) {
+        if (!active) return;
+        if (last >= L - 1) {
 #pragma unroll
             for (int i = 0; i < L; ++i) __builtin_nontemporal_store(y[i], &cwg[c0 + uint32_t(i) * crs]);
         } else {
 #pragma unroll
             for (int i = 0; i < L; ++i)
-                if (r0 + i < nq) __builtin_nontemporal_store(y[i], &cwg[c0 + uint32_t(i) * crs]);
+                if (i <= last) __builtin_nontemporal_store(y[i], &cwg[c0 + uint32_t(i) * crs]);
         }
-        if (bv.periodic && (r0 < bv.degree || r0 + L > nbas - off)) {
+        return;
+    }
+    // a row leaves and the next tile's row takes its register (every line of
+    // this tile is in the batch: a later tile exists)
+    at_vals(next);
 #pragma unroll
-            for (int i = 0; i < L; ++i) {
-                int const prow = tv.top + r0 + i;
-                if (prow < nq) {
-                    int const j0 = prow + off - nbas;
-                    if (j0 >= 0) cwg[clo + uint32_t(j0) * crs] = y[i];
-                    int const j2 = prow + off + nbas;
-                    if (j2 < nbas + bv.degree) cwg[clo + uint32_t(j2) * crs] = y[i];
-                }
-            }
-        }
+    for (int i = 0; i < L; ++i) {
+        if (i <= last) __builtin_nontemporal_store(y[i], &cwg[c0 + uint32_t(i) * crs]);
+        y[i] = load_row(i);
+        chunk_fence(i);
+    }
+    b2 = load_border(next);
+    at_coef(next);
+    line0 = next;
     }
 }
 
@@ -256,7 +289,9 @@ void launch_one(BuilderPlan const& p, TiledView const& tv, size_t lds, double* c
         hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       int(lds)),
                   "hipFuncSetAttribute");
-    hipLaunchKernelGGL(kern, dim3(tile_grid<LB>(nbatch)), dim3(NT), lds, stream, tv, p.view, vals, vl, dl, dr, dlay,
+    unsigned grid = tile_grid<LB>(nbatch);
+    if (loops(L, IC, TMODE)) grid = std::min(grid, unsigned(cu_count()) * (1024 / NT)); // 128 registers: 1024 threads per CU
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, stream, tv, p.view, vals, vl, dl, dr, dlay,
                        coef, cl, nbatch);
     hip_check(hipGetLastError(), "build_tiled_kernel launch");
 }

@@ -105,6 +105,7 @@ inline size_t gamma_lds_doubles(TiledView const& tv) { return size_t(tv.ngb) * t
 
 __device__ __forceinline__ int64_t lay(Layout const& L, int64_t r, int64_t l)
 {
+    if (l < L.inner) return r * L.rs + l * L.is; // one batch dimension: no 64-bit division
     return r * L.rs + (l % L.inner) * L.is + (l / L.inner) * L.os;
 }
 
