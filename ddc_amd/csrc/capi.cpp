@@ -534,7 +534,7 @@ ddcx_status ddcx_evaluator2d_eval_vjp_binned_static(const ddcx_evaluator* e1, co
         if (nbatch == 0) return;
         require(coef && gcoef, "null data pointer");
         require(npts == 0 || (coords && w && gx), "null data pointer");
-        int64_t const need = ddcx::eval2d_vjp_workspace(*e1->bs, *e2->bs, npts, nbatch);
+        int64_t const need = ddcx::eval2d_vjp_workspace(*e1->bs, *e2->bs, npts, nbatch, true);
         if (need == 0)
             throw ddcx::Error(DDCX_ERR_UNSUPPORTED, "binned 2D adjoint: grid or degree out of range");
         if (need > int64_t(DDCX_STATIC_SCRATCH_BYTES))
@@ -614,7 +614,7 @@ ddcx_status ddcx_evaluatornd_eval_binned(const ddcx_evaluator* const* evs, int n
         nd_setup(evs, nd, orders, bs, lower, upper);
         require(coef_strides, "null coefficient strides");
         require(npts >= 0 && nbatch >= 0, "negative size");
-        int64_t const need = ddcx::evalnd_binned_workspace(bs, nd, npts, nbatch);
+        int64_t const need = ddcx::evalnd_binned_workspace(bs, nd, npts, nbatch, true);
         if (need == 0)
             throw ddcx::Error(DDCX_ERR_UNSUPPORTED, "binned N-D evaluation: 3 dimensions of one degree <= 5 only");
         require(work_bytes >= need, "binned N-D evaluation: workspace smaller than ddcx_evaluatornd_eval_workspace");

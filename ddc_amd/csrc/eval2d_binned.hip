@@ -54,18 +54,6 @@ __device__ __forceinline__ int bin_of_xy(BSplinesView const& b1, BSplinesView co
     return (cell_jmin(b1, x1) / g.T) * g.nt2 + cell_jmin(b2, x2) / g.T;
 }
 
-// tile of point t, or -1 (Null rule: gx = 0 written here when `write_gx`)
-__device__ __forceinline__ int bin_of(BSplinesView const& b1, BSplinesView const& b2, Rules2D rules, Bin2D const& g,
-                                      const double* coords, double* gx, int64_t t, bool write_gx)
-{
-    int const bin = bin_of_xy(b1, b2, rules, g, coords[2 * t], coords[2 * t + 1]);
-    if (bin < 0 && write_gx) {
-        gx[2 * t] = 0.0;
-        gx[2 * t + 1] = 0.0;
-    }
-    return bin;
-}
-
 __global__ void __launch_bounds__(256) zero_patch_kernel(double* __restrict__ g, int s1, int s2, int64_t cbs,
                                                          int64_t st1, int64_t st2, int64_t nbatch)
 {
@@ -79,12 +67,13 @@ __global__ void __launch_bounds__(256) zero_patch_kernel(double* __restrict__ g,
 __global__ void __launch_bounds__(kBinT) bin_count_kernel(BSplinesView b1, BSplinesView b2, Rules2D rules, Bin2D g,
                                                           const double* __restrict__ coords, double* __restrict__ gx,
                                                           int64_t npts, int64_t bpb, int* __restrict__ counts,
-                                                          uint16_t* __restrict__ bins)
+                                                          int groups, uint16_t* __restrict__ bins)
 {
     __shared__ int hist[kMaxBins];
     extern __shared__ double lds_tabs[];
     int64_t const l = blockIdx.x / bpb;
-    int64_t const p0 = (blockIdx.x % bpb) * int64_t(kBinT * kBinPts);
+    static_assert(kBinT * kBinPts == kChunk, "the same points per workgroup as in the scatter");
+    int64_t const p0 = (blockIdx.x % bpb) * int64_t(kChunk);
     for (int k = threadIdx.x; k < g.nbins; k += kBinT) hist[k] = 0;
     stage_tables_2d(b1, b2, lds_tabs, threadIdx.x, kBinT);
     __syncthreads();
@@ -110,8 +99,9 @@ __global__ void __launch_bounds__(kBinT) bin_count_kernel(BSplinesView b1, BSpli
         }
     }
     __syncthreads();
+    int* const cg = counts + (l * groups + blockIdx.x % groups) * g.nbins;
     for (int k = threadIdx.x; k < g.nbins; k += kBinT)
-        if (hist[k]) atomicAdd(&counts[l * g.nbins + k], hist[k]);
+        if (hist[k]) atomicAdd(&cg[k], hist[k]);
 }
 
 template <int D1, int D2>
@@ -263,13 +253,14 @@ void* static_scratch()
     return ptrs[size_t(dev)];
 }
 
-int64_t eval2d_vjp_workspace(BSplinesPlan const& bp1, BSplinesPlan const& bp2, int64_t npts, int64_t nbatch)
+int64_t eval2d_vjp_workspace(BSplinesPlan const& bp1, BSplinesPlan const& bp2, int64_t npts, int64_t nbatch,
+                             bool least)
 {
     Bin2D const g = bins_for(bp1, bp2, nbatch);
     if (g.nbins == 0 || npts >= (int64_t(1) << 31) || bp1.view.degree > 5 || bp2.view.degree > 5 ||
         !staged_tables_fit_2d(bp1.device_view(), bp2.device_view(), kTabLds))
         return 0;
-    return carve(g.nbins, 3, npts, nbatch, nullptr).bytes;
+    return carve(g.nbins, 3, npts, nbatch, nullptr, least ? 1 : groups_for(npts)).bytes;
 }
 
 void launch_eval2d_vjp_binned(BSplinesPlan const& bp1, BSplinesPlan const& bp2, Rules2D const& rules,
@@ -281,21 +272,21 @@ void launch_eval2d_vjp_binned(BSplinesPlan const& bp1, BSplinesPlan const& bp2, 
     bp2.ensure_device();
     BSplinesView const b1 = bp1.device_view(), b2 = bp2.device_view();
     Bin2D const g = bins_for(bp1, bp2, nbatch);
-    int64_t const need = eval2d_vjp_workspace(bp1, bp2, npts, nbatch);
+    int64_t const need = eval2d_vjp_workspace(bp1, bp2, npts, nbatch, true);
     if (need == 0) throw Error(DDCX_ERR_UNSUPPORTED, "binned 2D adjoint: grid or degree out of range");
     if (work_bytes < need) throw Error(DDCX_ERR_INVALID, "binned 2D adjoint: workspace too small");
-    Work const ws = carve(g.nbins, 3, npts, nbatch, work);
+    Work const ws = carve_within(g.nbins, 3, npts, nbatch, work, work_bytes);
     auto blocks = grid_blocks;
     int const s1 = bp1.size(), s2 = bp2.size();
     hipLaunchKernelGGL(zero_patch_kernel, dim3(blocks(int64_t(s1) * s2 * nbatch, 256)), dim3(256), 0, stream, gcoef,
                        s1, s2, cbs, st1, st2, nbatch);
-    hipLaunchKernelGGL(fill_int_kernel, dim3(blocks(nbatch * g.nbins, 256)), dim3(256), 0, stream, ws.counts,
-                       nbatch * g.nbins);
+    int64_t const ncount = nbatch * g.nbins * ws.groups;
+    hipLaunchKernelGGL(fill_int_kernel, dim3(blocks(ncount, 256)), dim3(256), 0, stream, ws.counts, ncount);
     if (npts > 0) {
-        int64_t const bpb = (npts + kBinT * kBinPts - 1) / (kBinT * kBinPts);
+        int64_t const bpb = (npts + kChunk - 1) / kChunk;
         size_t const tabs = staged_tables_bytes_2d(b1, b2);
         hipLaunchKernelGGL(bin_count_kernel, dim3(blocks(bpb * nbatch, 1)), dim3(kBinT), tabs, stream, b1, b2, rules,
-                           g, coords, gx, npts, bpb, ws.counts, ws.bins);
+                           g, coords, gx, npts, bpb, ws.counts, ws.groups, ws.bins);
         scan_and_scatter<2, true>(g.nbins, coords, w, npts, nbatch, ws, stream);
         bool launched = false;
         dispatch_degree(b1.degree, [&]<int D1>() {

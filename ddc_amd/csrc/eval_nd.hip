@@ -395,13 +395,14 @@ __device__ __forceinline__ bool nd_place(NdArgs const& a, double (&x)[N], int an
 // get their value here
 __global__ void __launch_bounds__(kNdBinT) ndbin_count_kernel(NdArgs a, Bin3D g, const double* __restrict__ coords,
                                                               double* __restrict__ out, int64_t npts, int64_t bpb,
-                                                              int* __restrict__ counts, uint16_t* __restrict__ bins,
-                                                              int any_order)
+                                                              int* __restrict__ counts, int groups,
+                                                              uint16_t* __restrict__ bins, int any_order)
 {
     __shared__ int hist[binning::kMaxBins];
     extern __shared__ double lds_tabs[];
     int64_t const l = blockIdx.x / bpb;
-    int64_t const p0 = (blockIdx.x % bpb) * int64_t(kNdBinT * kNdBinPts);
+    static_assert(kNdBinT * kNdBinPts == binning::kChunk, "the same points per workgroup as in the scatter");
+    int64_t const p0 = (blockIdx.x % bpb) * int64_t(binning::kChunk);
     for (int k = threadIdx.x; k < g.nbins; k += kNdBinT) hist[k] = 0;
     stage_tables_nd<3>(a, lds_tabs, threadIdx.x, kNdBinT);
     __syncthreads();
@@ -437,8 +438,9 @@ __global__ void __launch_bounds__(kNdBinT) ndbin_count_kernel(NdArgs a, Bin3D g,
         }
     }
     __syncthreads();
+    int* const cg = counts + (l * groups + blockIdx.x % groups) * g.nbins;
     for (int k = threadIdx.x; k < g.nbins; k += kNdBinT)
-        if (hist[k]) atomicAdd(&counts[l * g.nbins + k], hist[k]);
+        if (hist[k]) atomicAdd(&cg[k], hist[k]);
 }
 
 template <int D, bool ANY>
@@ -634,14 +636,14 @@ Bin3D bins3d(NdArgs const& a, int nd)
 
 } // namespace
 
-int64_t evalnd_binned_workspace(BSplinesPlan const* const* bs, int nd, int64_t npts, int64_t nbatch)
+int64_t evalnd_binned_workspace(BSplinesPlan const* const* bs, int nd, int64_t npts, int64_t nbatch, bool least)
 {
     // sizes only: the views' shapes, no device access
     NdArgs a{};
     for (int k = 0; k < nd && k < kMaxNd; ++k) a.b[k] = bs[k]->device_view();
     Bin3D const g = bins3d(a, nd);
     if (g.nbins == 0 || npts >= (int64_t(1) << 31)) return 0;
-    return binning::carve(g.nbins, 3, npts, nbatch, nullptr).bytes;
+    return binning::carve(g.nbins, 3, npts, nbatch, nullptr, least ? 1 : binning::groups_for(npts)).bytes;
 }
 
 void launch_evalnd_binned(BSplinesPlan const* const* bs, int nd, const int* orders, const int* lower,
@@ -652,19 +654,19 @@ void launch_evalnd_binned(BSplinesPlan const* const* bs, int nd, const int* orde
     using namespace binning;
     NdArgs const a = make_args(bs, nd, orders, lower, upper, st);
     Bin3D const g = bins3d(a, nd);
-    int64_t const need = evalnd_binned_workspace(bs, nd, npts, nbatch);
+    int64_t const need = evalnd_binned_workspace(bs, nd, npts, nbatch, true);
     if (need == 0) throw Error(DDCX_ERR_UNSUPPORTED, "binned N-D evaluation: 3 dimensions of one degree <= 5 only");
     if (work_bytes < need) throw Error(DDCX_ERR_INVALID, "binned N-D evaluation: workspace too small");
     if (npts * nbatch == 0) return;
     int any = 0;
     for (int k = 0; k < nd; ++k) any |= a.order[k];
-    Work const ws = carve(g.nbins, 3, npts, nbatch, work);
+    Work const ws = carve_within(g.nbins, 3, npts, nbatch, work, work_bytes);
     size_t const tabs = nd_tables_bytes(a, 3);
-    hipLaunchKernelGGL(fill_int_kernel, dim3(grid_blocks(nbatch * g.nbins, 256)), dim3(256), 0, stream, ws.counts,
-                       nbatch * g.nbins);
-    int64_t const bpb = (npts + kNdBinT * kNdBinPts - 1) / (kNdBinT * kNdBinPts);
+    int64_t const ncount = nbatch * g.nbins * ws.groups;
+    hipLaunchKernelGGL(fill_int_kernel, dim3(grid_blocks(ncount, 256)), dim3(256), 0, stream, ws.counts, ncount);
+    int64_t const bpb = (npts + kChunk - 1) / kChunk;
     hipLaunchKernelGGL(ndbin_count_kernel, dim3(grid_blocks(bpb * nbatch, 1)), dim3(kNdBinT), tabs, stream, a, g,
-                       coords, out, npts, bpb, ws.counts, ws.bins, any);
+                       coords, out, npts, bpb, ws.counts, ws.groups, ws.bins, any);
     scan_and_scatter<3, false>(g.nbins, coords, nullptr, npts, nbatch, ws, stream);
     bool launched = false;
     dispatch_degree(a.b[0].degree, [&]<int D>() {

@@ -443,8 +443,10 @@ void launch_evalnd(BSplinesPlan const* const* bs, int nd, const int* orders, con
                    double* out, const double* coords, int64_t npts, const double* coef, int64_t cbs,
                    const int64_t* st, int64_t nbatch, hipStream_t stream);
 // binned 3D evaluation (eval_nd.hip): workspace bytes (0: not supported for
-// this grid, use launch_evalnd), and the launch
-int64_t evalnd_binned_workspace(BSplinesPlan const* const* bs, int nd, int64_t npts, int64_t nbatch);
+// this grid, use launch_evalnd; least: the size below which a call is
+// refused), and the launch
+int64_t evalnd_binned_workspace(BSplinesPlan const* const* bs, int nd, int64_t npts, int64_t nbatch,
+                                bool least = false);
 void launch_evalnd_binned(BSplinesPlan const* const* bs, int nd, const int* orders, const int* lower,
                           const int* upper, double* out, const double* coords, int64_t npts, const double* coef,
                           int64_t cbs, const int64_t* st, int64_t nbatch, void* work, int64_t work_bytes,
@@ -462,7 +464,9 @@ void launch_eval2d(BSplinesPlan const& b1, BSplinesPlan const& b2, Rules2D const
                    const double* coords, int64_t npts, const double* coef, int64_t coef_batch_stride, int64_t st1,
                    int64_t st2, int64_t nbatch, hipStream_t stream);
 // binned 2D adjoint (eval2d_binned.hip): workspace bytes, 0 if unsupported
-int64_t eval2d_vjp_workspace(BSplinesPlan const& bp1, BSplinesPlan const& bp2, int64_t npts, int64_t nbatch);
+// (least: the size below which a call is refused)
+int64_t eval2d_vjp_workspace(BSplinesPlan const& bp1, BSplinesPlan const& bp2, int64_t npts, int64_t nbatch,
+                             bool least = false);
 // packed 2D evaluation (eval2d_packed.hip): workspace bytes per batch entry
 int64_t eval2d_packed_record_bytes(BSplinesPlan const& bp1, BSplinesPlan const& bp2);
 void launch_eval2d_packed(BSplinesPlan const& bp1, BSplinesPlan const& bp2, Rules2D const& rules, int o1, int o2,
