@@ -15,8 +15,8 @@
 //   3. the same for the backward sweep;
 //   4. 2x2-block border (splines_linear_problem_2x2_blocks.cpp:275-298):
 //      lambda couplings gathered through LDS, the small Schur system solved
-//      by one thread per line, the Q^-1 gamma correction applied in
-//      registers;
+//      by its inverse, one thread per border row and line, the Q^-1 gamma
+//      correction applied in registers;
 //   5. store, including the periodic duplicate rows (spline_builder.hpp:
 //      1074-1100).
 #pragma once
