@@ -576,6 +576,52 @@ inline bool staged_tables_fit_2d(BSplinesView const& b1, BSplinesView const& b2,
 }
 
 #ifdef __HIPCC__
+// nonuniform_cell of U points at once, without branches between them: every
+// step of the search reads one knot per point, so the U chains of dependent LDS
+// reads overlap, and a wave leaves when its widest bracket is searched.  (One
+// point after the other, each in its own loop, the chains follow each other.)
+// The basis must have brackets (all with fewer than 65536 cells have).
+template <int U>
+__device__ __forceinline__ void nonuniform_cells(BSplinesView const& b, const double* kn, double const (&x)[U],
+                                                 int (&icell)[U])
+{
+    int n[U];
+    int widest = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        uint32_t const e = b.cells[bucket_of(b, b.nbucket, b.inv_bucket, x[u])];
+        icell[u] = b.degree + int(e & 0xffffu);
+        n[u] = int(e >> 16) - int(e & 0xffffu);
+        widest = max(widest, n[u]);
+    }
+    while (__any(widest > 0)) {
+        widest = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int const half = (n[u] + 1) >> 1; // 0 once n is 0: the cell's own lower knot, no move
+            bool const up = kn[icell[u] + half] <= x[u];
+            icell[u] += up ? half : 0;
+            n[u] = up ? n[u] - half : half - 1;
+            widest = max(widest, n[u]);
+        }
+    }
+}
+
+// cell_jmin of U points at once, for bases with brackets
+template <int U>
+__device__ __forceinline__ void cells_jmin(BSplinesView const& b, double const (&x)[U], int (&jmin)[U])
+{
+    if (b.uniform) {
+        double offset;
+#pragma unroll
+        for (int u = 0; u < U; ++u) jmin[u] = uniform_cell(b, x[u], offset);
+    } else {
+        nonuniform_cells<U>(b, b.knots, x, jmin);
+#pragma unroll
+        for (int u = 0; u < U; ++u) jmin[u] -= b.degree;
+    }
+}
+
 // The workgroup's threads copy the tables to `lds` (8-byte aligned,
 // staged_tables_bytes_2d long) and point b1 / b2 at the copies, for either
 // basis kind, so that every knot and bracket read of the kernel is an LDS

@@ -40,6 +40,12 @@ constexpr int kChunk = kScatT * kScatPts; // points per workgroup, in the count 
 constexpr int kGroups = 8;              // parts of a tile's range: one per XCD
 constexpr size_t kLdsBytes = 160 * 1024;
 
+// j / T for cells 0 <= j < 2^26 and tile sides 1 < T <= 64, as the high half of
+// one product: inverse(T) exceeds 2^32 / T by less than 1, which moves the
+// quotient by less than j / 2^32, below the 1 / T it may.
+constexpr unsigned inverse(int T) { return unsigned(((uint64_t(1) << 32) + unsigned(T) - 1) / unsigned(T)); }
+__device__ __forceinline__ int tile_index(int j, unsigned inv_T) { return int(__umulhi(unsigned(j), inv_T)); }
+
 __global__ void __launch_bounds__(256) fill_int_kernel(int* __restrict__ p, int64_t n)
 {
     int64_t const i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;

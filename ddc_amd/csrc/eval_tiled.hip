@@ -26,7 +26,6 @@ using tiled::basis_and_deriv;
 using tiled::kMaxLds;
 using tiled::lay;
 using tiled::load_tile;
-using tiled::nonuniform_cells;
 using tiled::point_values;
 
 // Buffer resources (raw buffers, stride 0) for the streaming kernel: a load

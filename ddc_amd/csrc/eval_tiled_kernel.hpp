@@ -9,37 +9,6 @@ namespace tiled {
 
 constexpr size_t kMaxLds = 160 * 1024;
 
-// nonuniform_cell of U points at once, without branches between them: every
-// step of the search reads one knot per point, so the U chains of dependent LDS
-// reads overlap, and a wave leaves when its widest bracket is searched.  (One
-// point after the other, each in its own loop, the chains follow each other.)
-// The bases staged here have brackets whenever they have fewer than 65536 cells.
-template <int U>
-__device__ __forceinline__ void nonuniform_cells(BSplinesView const& b, const double* kn, double const (&x)[U],
-                                                 int (&icell)[U])
-{
-    int n[U];
-    int widest = 0;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        uint32_t const e = b.cells[bucket_of(b, b.nbucket, b.inv_bucket, x[u])];
-        icell[u] = b.degree + int(e & 0xffffu);
-        n[u] = int(e >> 16) - int(e & 0xffffu);
-        widest = max(widest, n[u]);
-    }
-    while (__any(widest > 0)) {
-        widest = 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            int const half = (n[u] + 1) >> 1; // 0 once n is 0: the cell's own lower knot, no move
-            bool const up = kn[icell[u] + half] <= x[u];
-            icell[u] += up ? half : 0;
-            n[u] = up ? n[u] - half : half - 1;
-            widest = max(widest, n[u]);
-        }
-    }
-}
-
 // The value (ORDER 0) or derivative of a point in a known cell (kSafeNonUniform,
 // orders 0 and 1) or of any point.
 template <int D, int ORDER, int KIND>
