@@ -309,34 +309,28 @@ __host__ __device__ inline void nonuniform_basis(const double* knots, int icell,
 // (device evaluation): the recurrence runs to degree D - 1, whose values M give
 // both, with the divisors of the last level inverted once,
 //   B_k' = D (M_{k-1} / w_{k-1} - M_k / w_k),  w_r = right_r + left_{D-1-r},
-// and v by the last step of the recurrence.  NURBS A2.3 for one derivative
-// without its tables.
-template <int D, bool SAFE = false>
+// and v by the last step of the recurrence: NURBS A2.3 for one derivative
+// without its tables.  Every divisor takes its own reciprocal: from one
+// reciprocal of their product (invert_together) the rms error of the weights is
+// 4.0e-16 instead of 1.7e-16 for cubic and 9.5e-16 instead of 2.3e-16 for
+// quintic splines, the product's range has to be watched, and the D(D+1)/2
+// prefixes spill for degree 6.
+template <int D>
 __host__ __device__ inline void nonuniform_basis_deriv(const double* knots, int icell, double x, double* v, double* dv)
 {
-    constexpr int M = D * (D + 1) / 2, W = M - D;
-    double left[D], right[D], den[M], pre[M], inv[M];
+    double left[D], right[D];
 #pragma unroll
     for (int j = 0; j < D; ++j) {
         left[j] = x - knots[icell - j];
         right[j] = knots[icell + j + 1] - x;
     }
-    {
-        int k = 0;
-#pragma unroll
-        for (int j = 0; j < D; ++j)
-#pragma unroll
-            for (int r = 0; r < j + 1; ++r) den[k++] = right[r] + left[j - r];
-    }
-    invert_together<M, SAFE>(den, pre, inv);
     v[0] = 1.0;
-    int k = 0;
 #pragma unroll
     for (int j = 0; j < D - 1; ++j) {
         double saved = 0.0;
 #pragma unroll
         for (int r = 0; r < j + 1; ++r) {
-            double const temp = v[r] * inv[k++];
+            double const temp = v[r] * fast_rcp(right[r] + left[j - r]);
             v[r] = fma(right[r], temp, saved);
             saved = left[j - r] * temp;
         }
@@ -345,7 +339,7 @@ __host__ __device__ inline void nonuniform_basis_deriv(const double* knots, int 
     double saved = 0.0, before = 0.0;
 #pragma unroll
     for (int r = 0; r < D; ++r) {
-        double const temp = v[r] * inv[W + r];
+        double const temp = v[r] * fast_rcp(right[r] + left[D - 1 - r]);
         dv[r] = (before - temp) * D;
         before = temp;
         v[r] = fma(right[r], temp, saved);

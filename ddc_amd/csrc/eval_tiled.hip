@@ -275,7 +275,7 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
                 if (outside) rule |= 1u << u;
             }
             int icell[U] = {};
-            if constexpr (KIND == kSafeNonUniform) nonuniform_cells<U>(bl, knots, xa, icell);
+            if constexpr (KIND == kNonUniformBasis) nonuniform_cells<U>(bl, knots, xa, icell);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 int const ii = i + u * ROWS;
@@ -356,24 +356,22 @@ bool launch_stream(BSplinesPlan const& bs, Rules1D rules, double* out, const dou
         hip_check(hipGetLastError(), "eval_stream_kernel launch");
         return true;
     };
-    bool const safe = bs.safe_products && b.nbucket > 0;
     // stages for at least npts points: 512, 768 or 1024 (uniform), 768 or 1152
     auto uniform = [&] {
         return npts <= 16 * 32   ? go.template operator()<kUniformBasis, 512, 2, 8, 33>()
                : npts <= 24 * 32 ? go.template operator()<kUniformBasis, 512, 2, 12, 33>()
                                  : go.template operator()<kUniformBasis, 512, 2, 16, 33>();
     };
-    auto nonuniform = [&] {
-        return npts <= 16 * 48 ? go.template operator()<kSafeNonUniform, 768, 2, 8, 22>()
-                               : go.template operator()<kSafeNonUniform, 768, 2, 12, 22>();
+    auto nonuniform = [&]<int KIND>() {
+        return npts <= 16 * 48 ? go.template operator()<KIND, 768, 2, 8, 22>()
+                               : go.template operator()<KIND, 768, 2, 12, 22>();
     };
-    if constexpr (ORDER == 0) {
+    // higher degrees of the other forms spill and keep eval_tiled_kernel
+    if constexpr (ORDER == 0 || D <= 3)
         if (b.uniform) return uniform();
-        if constexpr (D <= 3) // higher degrees spill in this form and keep eval_tiled_kernel
-            if (safe) return nonuniform();
-    } else if constexpr (D <= 3) {
-        if (safe) return nonuniform();
-        if (b.uniform) return uniform();
+    if constexpr (D <= 3) {
+        if constexpr (ORDER == 1) return nonuniform.template operator()<kNonUniformBasis>();
+        else if (bs.safe_products) return nonuniform.template operator()<kSafeNonUniform>();
     }
     return false;
 }
@@ -473,8 +471,7 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
         auto go = [&]<int NT>() {
             constexpr int LB = 8;
             auto kern = b.uniform ? eval_vjp_tiled_kernel<D, LB, NT, kUniformBasis>
-                        : bs.safe_products && b.nbucket > 0 ? eval_vjp_tiled_kernel<D, LB, NT, kSafeNonUniform>
-                                                            : eval_vjp_tiled_kernel<D, LB, NT, kNonUniformBasis>;
+                                  : eval_vjp_tiled_kernel<D, LB, NT, kNonUniformBasis>;
             size_t const lds = lds_of(pitch);
             hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)),

@@ -9,8 +9,15 @@ namespace tiled {
 
 constexpr size_t kMaxLds = 160 * 1024;
 
-// The value (ORDER 0) or derivative of a point in a known cell (kSafeNonUniform,
-// orders 0 and 1) or of any point.
+// Whether a kernel finds the cells of several points at once: bases whose
+// divisor products are safe, and first derivatives, which form no product.
+constexpr bool cells_together(int order, int kind)
+{
+    return kind == kSafeNonUniform || (kind == kNonUniformBasis && order == 1);
+}
+
+// The value (ORDER 0) or derivative of a point in a known cell (cells_together)
+// or of any point.
 template <int D, int ORDER, int KIND>
 __device__ __forceinline__ double tile_value(BSplinesView const& b, const double* kn, double x, int icell,
                                              const double* tile, int pitch)
@@ -22,9 +29,9 @@ __device__ __forceinline__ double tile_value(BSplinesView const& b, const double
         jmin = icell - D;
     } else if constexpr (ORDER == 0) {
         jmin = eval_basis<D, true, KIND>(b, kn, x, v);
-    } else if constexpr (ORDER == 1 && KIND == kSafeNonUniform) {
+    } else if constexpr (ORDER == 1 && KIND == kNonUniformBasis) {
         double values[D + 1];
-        nonuniform_basis_deriv<D, true>(kn, icell, x, values, v);
+        nonuniform_basis_deriv<D>(kn, icell, x, values, v);
         jmin = icell - D;
     } else {
         double der[(D + 1) * (ORDER + 1)];
@@ -39,14 +46,13 @@ __device__ __forceinline__ double tile_value(BSplinesView const& b, const double
 }
 
 // Values v and first derivatives dv of the splines on x's cell; returns the
-// first spline.  icell: x's cell (kSafeNonUniform; found before, for several
-// points at once).
+// first spline.  icell: x's cell (non-uniform bases).
 template <int D, int KIND>
 __device__ __forceinline__ int basis_and_deriv(BSplinesView const& b, const double* kn, double x, int icell, double* v,
                                                double* dv)
 {
-    if constexpr (KIND == kSafeNonUniform) {
-        nonuniform_basis_deriv<D, true>(kn, icell, x, v, dv);
+    if constexpr (KIND == kNonUniformBasis) {
+        nonuniform_basis_deriv<D>(kn, icell, x, v, dv);
         return icell - D;
     } else {
         double der[(D + 1) * 2];
@@ -66,7 +72,7 @@ template <int D, int ORDER, int KIND, int U>
 __device__ __forceinline__ void point_values(BSplinesView const& b, const double* kn, Rules1D rules, double (&x)[U],
                                              const double* tile, int pitch, double (&y)[U])
 {
-    if constexpr (KIND == kSafeNonUniform && ORDER <= 1) {
+    if constexpr (cells_together(ORDER, KIND)) {
         int icell[U];
         uint32_t zero = 0; // bit u: the Null rule gives 0
         if constexpr (ORDER == 0) {
@@ -133,10 +139,8 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
     constexpr int ROWS = NT / LB;
     // points per pipeline stage per thread: as many as the registers hold
     // without spilling (derivative tables of non-uniform bases are the largest)
-    constexpr int U = ORDER == 1 && KIND == kNonUniformBasis ? 1
-                      : LB < 16 && NT < 1024 ? 4
-                      : ORDER == 0 ? 8
-                      : ORDER == 1 && KIND == kSafeNonUniform ? 8
+    constexpr int U = LB < 16 && NT < 1024 ? 4
+                      : ORDER == 0 || cells_together(ORDER, KIND) ? 8
                       : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
                                               : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
     constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
@@ -204,8 +208,8 @@ void launch_eval_tile(BSplinesPlan const& bs, Rules1D rules, double* out, const 
     BSplinesView const b = bs.device_view();
     size_t const lds = (size_t(ncoef) * pitch + nknots) * sizeof(double) + size_t(b.nbucket) * sizeof(uint32_t);
     auto kern = b.uniform ? eval_tiled_kernel<D, ORDER, LB, NT, kUniformBasis>
-                : ORDER <= 1 && bs.safe_products && b.nbucket > 0
-                    ? eval_tiled_kernel<D, ORDER, LB, NT, ORDER <= 1 ? kSafeNonUniform : kNonUniformBasis>
+                : ORDER == 0 && bs.safe_products
+                    ? eval_tiled_kernel<D, ORDER, LB, NT, ORDER == 0 ? kSafeNonUniform : kNonUniformBasis>
                     : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis>;
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   int(lds)),
