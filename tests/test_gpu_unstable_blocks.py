@@ -9,7 +9,7 @@ from cases import Case, P
 
 UNSTABLE = [Case(4, False, P, ncells=14, seed=4), Case(4, False, P, ncells=20, seed=18),
             Case(4, False, P, ncells=24, seed=44)]
-STABLE = [Case(5, False, P, ncells=14, seed=0), Case(4, False, P, ncells=24, seed=0),
+STABLE = [Case(4, False, P, ncells=14, seed=1), Case(4, False, P, ncells=24, seed=0),
           Case(5, False, P, ncells=64, seed=1), Case(4, False, P, ncells=300, seed=0)]
 
 
