@@ -220,31 +220,23 @@ __host__ __device__ inline void uniform_basis_from_offset(double offset, double*
     }
 }
 
-// The inverses of M positive divisors from one refined hardware reciprocal of
-// their product: prefix products forward, the running inverse backward, 3
-// multiplications per divisor instead of a reciprocal and four fmas each.
-// Outside [2^-960, 2^960] each divisor takes its own reciprocal; SAFE: the host
-// has checked that no cell's product leaves the range (products_safe), so the
-// branch goes.  (In a loop over several points it made the compiler keep the
-// divisors of all of them: 668 B of spills for 8 cubic points.)
-template <int M, bool SAFE>
-__host__ __device__ inline void invert_together(double const (&den)[M], double (&pre)[M], double (&inv)[M])
+// The recurrence of nonuniform_basis on a point's left and right distances;
+// inverse(k, d) gives 1 / d of the k-th divisor d (in the order of its use).
+template <int D, class Inverse>
+__host__ __device__ inline void nonuniform_recurrence(double const (&left)[D], double const (&right)[D], double* values,
+                                                      Inverse inverse)
 {
-    pre[0] = den[0];
+    int k = 0;
 #pragma unroll
-    for (int k = 1; k < M; ++k) pre[k] = pre[k - 1] * den[k];
-    double const mag = fabs(pre[M - 1]);
-    if (SAFE || (mag >= 0x1p-960 && mag <= 0x1p960)) {
-        double rv = fast_rcp(pre[M - 1]);
+    for (int j = 0; j < D; ++j) {
+        double saved = 0.0;
 #pragma unroll
-        for (int k = M - 1; k > 0; --k) {
-            inv[k] = rv * pre[k - 1];
-            rv *= den[k];
+        for (int r = 0; r < j + 1; ++r) {
+            double const temp = values[r] * inverse(k++, right[r] + left[j - r]);
+            values[r] = fma(right[r], temp, saved);
+            saved = left[j - r] * temp;
         }
-        inv[0] = rv;
-    } else {
-#pragma unroll
-        for (int k = 0; k < M; ++k) inv[k] = fast_rcp(den[k]);
+        values[j + 1] = saved;
     }
 }
 
@@ -253,7 +245,12 @@ __host__ __device__ inline void invert_together(double const (&den)[M], double (
 // nonuniform_cell.  FAST (device evaluation): the update is one fma, and the
 // D(D+1)/2 divisors right[r] + left[j - r], which do not depend on the
 // recurrence's values, are inverted together (every divisor is at least the
-// cell's width, so their product is positive).
+// cell's width, so their product is positive): one refined hardware reciprocal
+// of the product, prefix products forward, the running inverse backward, 3
+// multiplications per divisor instead of a reciprocal and four fmas each.
+// Where the product is outside [2^-960, 2^960] each divisor takes its own
+// reciprocal; SAFE: the host has checked that no cell's product leaves the range
+// (products_safe), so the branch goes.
 template <int D, bool FAST = false, bool SAFE = false>
 __host__ __device__ inline void nonuniform_basis(const double* knots, int icell, double x, double* values)
 {
@@ -267,26 +264,31 @@ __host__ __device__ inline void nonuniform_basis(const double* knots, int icell,
             left[j] = x - knots[icell - j];
             right[j] = knots[icell + j + 1] - x;
         }
-        double den[M], pre[M], inv[M];
+        double den[M], pre[M];
         {
             int k = 0;
 #pragma unroll
             for (int j = 0; j < D; ++j)
 #pragma unroll
-                for (int r = 0; r < j + 1; ++r) den[k++] = right[r] + left[j - r];
+                for (int r = 0; r < j + 1; ++r) {
+                    den[k] = right[r] + left[j - r];
+                    pre[k] = k == 0 ? den[0] : pre[k - 1] * den[k];
+                    ++k;
+                }
         }
-        invert_together<M, SAFE>(den, pre, inv);
-        int k = 0;
+        double const mag = fabs(pre[M - 1]);
+        if (SAFE || (mag >= 0x1p-960 && mag <= 0x1p960)) {
+            double inv[M];
+            double rv = fast_rcp(pre[M - 1]);
 #pragma unroll
-        for (int j = 0; j < D; ++j) {
-            double saved = 0.0;
-#pragma unroll
-            for (int r = 0; r < j + 1; ++r) {
-                double const temp = values[r] * inv[k++];
-                values[r] = fma(right[r], temp, saved);
-                saved = left[j - r] * temp;
+            for (int k = M - 1; k > 0; --k) {
+                inv[k] = rv * pre[k - 1];
+                rv *= den[k];
             }
-            values[j + 1] = saved;
+            inv[0] = rv;
+            nonuniform_recurrence<D>(left, right, values, [&](int k, double) { return inv[k]; });
+        } else {
+            nonuniform_recurrence<D>(left, right, values, [](int, double d) { return fast_rcp(d); });
         }
         return;
     }
@@ -311,7 +313,7 @@ __host__ __device__ inline void nonuniform_basis(const double* knots, int icell,
 //   B_k' = D (M_{k-1} / w_{k-1} - M_k / w_k),  w_r = right_r + left_{D-1-r},
 // and v by the last step of the recurrence: NURBS A2.3 for one derivative
 // without its tables.  Every divisor takes its own reciprocal: from one
-// reciprocal of their product (invert_together) the rms error of the weights is
+// reciprocal of their product (as in nonuniform_basis) the rms error of the weights is
 // 4.0e-16 instead of 1.7e-16 for cubic and 9.5e-16 instead of 2.3e-16 for
 // quintic splines, the product's range has to be watched, and the D(D+1)/2
 // prefixes spill for degree 6.
@@ -368,7 +370,7 @@ __host__ __device__ inline void uniform_basis_deriv(double offset, double inv_st
 }
 
 // Whether the product of a cell's D(D+1)/2 divisors (the knot differences that
-// contain the cell), and every prefix of it in invert_together's order, stays
+// contain the cell), and every prefix of it in nonuniform_basis's order, stays
 // within [2^-900, 2^900] in every cell.  The divisors of a point differ from
 // the knot differences by rounding only.
 inline bool products_safe(int degree, int ncells, const double* knots)
@@ -422,10 +424,11 @@ __host__ __device__ inline int cell_jmin(BSplinesView const& b, double x)
 
 // eval_basis_and_n_derivs (NURBS book A2.3), uniform bsplines_uniform.hpp:475-564
 // and non-uniform bsplines_non_uniform.hpp:561-664.  derivs is (D+1) x (N+1)
-// row-major.  Returns jmin.
-template <int D, int N, bool FAST = false, int KIND = kAnyBasis>
+// row-major.  Returns jmin.  KNOWN: `known` is the cell (knot index) of x in a
+// non-uniform basis, found before.
+template <int D, int N, bool FAST = false, int KIND = kAnyBasis, bool KNOWN = false>
 __host__ __device__ inline int eval_basis_and_n_derivs(BSplinesView const& b, const double* knots, double x,
-                                                       double* derivs)
+                                                       double* derivs, int known = 0)
 {
     bool const uni = is_uniform_kind(KIND, b.uniform);
     int jmin;
@@ -436,7 +439,7 @@ __host__ __device__ inline int eval_basis_and_n_derivs(BSplinesView const& b, co
             jmin = uniform_cell(b, x, offset);
             uniform_basis_deriv<D>(offset, b.inv_step, v, dv);
         } else {
-            int const icell = nonuniform_cell(b, knots, x);
+            int const icell = KNOWN ? known : nonuniform_cell(b, knots, x);
             nonuniform_basis_deriv<D>(knots, icell, x, v, dv);
             jmin = icell - D;
         }
@@ -469,7 +472,7 @@ __host__ __device__ inline int eval_basis_and_n_derivs(BSplinesView const& b, co
     } else {
         double left[D > 0 ? D : 1];
         double right[D > 0 ? D : 1];
-        int const icell = nonuniform_cell(b, knots, x);
+        int const icell = KNOWN ? known : nonuniform_cell(b, knots, x);
         jmin = icell - D;
         ndu[0][0] = 1.0;
 #pragma unroll
@@ -576,7 +579,7 @@ inline bool staged_tables_fit_2d(BSplinesView const& b1, BSplinesView const& b2,
 // point after the other, each in its own loop, the chains follow each other.)
 // The basis must have brackets (all with fewer than 65536 cells have).
 template <int U>
-__device__ __forceinline__ void nonuniform_cells(BSplinesView const& b, const double* kn, double const (&x)[U],
+__device__ __forceinline__ void nonuniform_cells(BSplinesView const& b, const double* kn, double const* x,
                                                  int (&icell)[U])
 {
     int n[U];

@@ -157,8 +157,11 @@ __global__ void __launch_bounds__(NT) eval_stream_kernel(BSplinesView b, Rules1D
             }
 #pragma unroll
             for (int j = s * PS; j < (s + 1) * PS && j < PR; ++j) pf[j] = buffer_load<kNonTemporal>(rkn, cr(j, ltn));
-            double y[U];
-            point_values<D, ORDER, KIND, U>(bl, knots, rules, xa, tl, pitch, y);
+            double y[U] = {};
+            // non-uniform bases: not for the slots past the end of the line (those of
+            // the wave's first lane come first)
+            if (KIND == kUniformBasis || s * U * ROWS + __builtin_amdgcn_readfirstlane(prow) < npts)
+                point_values<D, ORDER, KIND, U>(bl, knots, rules, xa, tl, pitch, y);
 #pragma unroll
             for (int u = 0; u < U; ++u) buffer_store<kNonTemporal>(y[u], ro, pt(s * U * ROWS + prow + u * ROWS, lt));
 #pragma unroll
@@ -372,6 +375,7 @@ bool launch_stream(BSplinesPlan const& bs, Rules1D rules, double* out, const dou
     if constexpr (D <= 3) {
         if constexpr (ORDER == 1) return nonuniform.template operator()<kNonUniformBasis>();
         else if (bs.safe_products) return nonuniform.template operator()<kSafeNonUniform>();
+        else return nonuniform.template operator()<kNonUniformBasis>();
     }
     return false;
 }

@@ -9,33 +9,26 @@ namespace tiled {
 
 constexpr size_t kMaxLds = 160 * 1024;
 
-// Whether a kernel finds the cells of several points at once: bases whose
-// divisor products are safe, and first derivatives, which form no product.
-constexpr bool cells_together(int order, int kind)
-{
-    return kind == kSafeNonUniform || (kind == kNonUniformBasis && order == 1);
-}
-
-// The value (ORDER 0) or derivative of a point in a known cell (cells_together)
-// or of any point.
+// The value (ORDER 0) or derivative of a point; icell: its cell (non-uniform
+// bases).
 template <int D, int ORDER, int KIND>
 __device__ __forceinline__ double tile_value(BSplinesView const& b, const double* kn, double x, int icell,
                                              const double* tile, int pitch)
 {
     double v[D + 1];
     int jmin;
-    if constexpr (ORDER == 0 && KIND == kSafeNonUniform) {
-        nonuniform_basis<D, true, true>(kn, icell, x, v);
+    if constexpr (ORDER == 0 && KIND != kUniformBasis) {
+        nonuniform_basis<D, true, KIND == kSafeNonUniform>(kn, icell, x, v);
         jmin = icell - D;
     } else if constexpr (ORDER == 0) {
         jmin = eval_basis<D, true, KIND>(b, kn, x, v);
-    } else if constexpr (ORDER == 1 && KIND == kNonUniformBasis) {
+    } else if constexpr (ORDER == 1 && KIND != kUniformBasis) {
         double values[D + 1];
         nonuniform_basis_deriv<D>(kn, icell, x, values, v);
         jmin = icell - D;
     } else {
         double der[(D + 1) * (ORDER + 1)];
-        jmin = eval_basis_and_n_derivs<D, ORDER, true, KIND>(b, kn, x, der);
+        jmin = eval_basis_and_n_derivs<D, ORDER, true, KIND, KIND != kUniformBasis>(b, kn, x, der, icell);
 #pragma unroll
         for (int i = 0; i < D + 1; ++i) v[i] = der[i * (ORDER + 1) + ORDER];
     }
@@ -51,7 +44,7 @@ template <int D, int KIND>
 __device__ __forceinline__ int basis_and_deriv(BSplinesView const& b, const double* kn, double x, int icell, double* v,
                                                double* dv)
 {
-    if constexpr (KIND == kNonUniformBasis) {
+    if constexpr (KIND != kUniformBasis) {
         nonuniform_basis_deriv<D>(kn, icell, x, v, dv);
         return icell - D;
     } else {
@@ -69,10 +62,10 @@ __device__ __forceinline__ int basis_and_deriv(BSplinesView const& b, const doub
 // The values (ORDER 0, with the extrapolation rules) or derivatives of U points
 // of one line from its tile.
 template <int D, int ORDER, int KIND, int U>
-__device__ __forceinline__ void point_values(BSplinesView const& b, const double* kn, Rules1D rules, double (&x)[U],
-                                             const double* tile, int pitch, double (&y)[U])
+__device__ __forceinline__ void point_values(BSplinesView const& b, const double* kn, Rules1D rules, double* x,
+                                             const double* tile, int pitch, double* y)
 {
-    if constexpr (cells_together(ORDER, KIND)) {
+    if constexpr (KIND != kUniformBasis) {
         int icell[U];
         uint32_t zero = 0; // bit u: the Null rule gives 0
         if constexpr (ORDER == 0) {
@@ -85,11 +78,15 @@ __device__ __forceinline__ void point_values(BSplinesView const& b, const double
         nonuniform_cells<U>(b, kn, x, icell);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
+            // keeps the knots and divisors of one point at a time in registers (with a
+            // branch in the basis the scheduling barrier alone does not)
+            if constexpr (ORDER == 0 && KIND == kNonUniformBasis)
+                if (u > 0) asm volatile("" : "+v"(x[u]), "+v"(y[u - 1]));
             double const s = tile_value<D, ORDER, KIND>(b, kn, x[u], icell[u], tile, pitch);
             y[u] = (zero >> u) & 1u ? 0.0 : s;
-            // keeps the knots and divisors of one point at a time in registers
-            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (ORDER == 0) __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_sched_barrier(0);
     } else {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -100,16 +97,33 @@ __device__ __forceinline__ void point_values(BSplinesView const& b, const double
     }
 }
 
+// point_values in groups of G points, of which `live` (the same number in all
+// lanes of a wave) are points of the line: groups past them are left out, and
+// their y as it was.
+template <int D, int ORDER, int KIND, int U, int G>
+__device__ __forceinline__ void live_values(BSplinesView const& b, const double* kn, Rules1D rules, double (&x)[U],
+                                            int live, const double* tile, int pitch, double (&y)[U])
+{
+    static_assert(U % G == 0);
+#pragma unroll
+    for (int u = 0; u < U; u += G)
+        if (u == 0 || u < live) point_values<D, ORDER, KIND, G>(b, kn, rules, x + u, tile, pitch, y + u);
+}
+
 // The coefficient tile of a workgroup's lines to LDS: thread (line ln, row
 // prow) takes the rows prow, prow + NT / LB, ... of its line, in chunks of TC
 // whose loads are all in flight before the first LDS write.  Batch-contiguous:
 // the lanes of a row read LB consecutive lines; interpolation-contiguous: the
-// threads of a line read consecutive rows of it.
+// threads of a line read consecutive rows of it.  Tiles of up to 4 rows per
+// thread take chunks of 4: the 16 or 20 steps of a chunk are issued whether they
+// have a row or not (16 cells x 120000 lines, rows contiguous, deriv(2): 191 us
+// instead of 163).
 template <int LB, int NT, int TC>
 __device__ __forceinline__ void load_tile(double* tile, int pitch, const double* __restrict__ c, int64_t rs, int ncoef,
                                           int ln, int prow)
 {
     constexpr int ROWS = NT / LB;
+    if (TC > 4 && ncoef <= 4 * ROWS) return load_tile<LB, NT, TC < 4 ? TC : 4>(tile, pitch, c, rs, ncoef, ln, prow);
     for (int c0 = prow; c0 < ncoef; c0 += TC * ROWS) {
         double tv[TC];
 #pragma unroll
@@ -140,9 +154,10 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
     // points per pipeline stage per thread: as many as the registers hold
     // without spilling (derivative tables of non-uniform bases are the largest)
     constexpr int U = LB < 16 && NT < 1024 ? 4
-                      : ORDER == 0 || cells_together(ORDER, KIND) ? 8
+                      : ORDER == 0 || (ORDER == 1 && KIND != kUniformBasis) ? 8
                       : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
                                               : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
+    constexpr int G = KIND == kUniformBasis ? U : ORDER == 0 ? 4 : 2; // points worked through together
     constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
     int const tid = threadIdx.x;
     int const ln = line_major ? tid / ROWS : tid % LB;
@@ -190,9 +205,14 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
 #pragma unroll
         for (int u = 0; u < U; ++u) xb[u] = __builtin_nontemporal_load(&cp[atx(i + (U + u) * ROWS)]);
         double y[U];
-        point_values<D, ORDER, KIND, U>(bl, knots, rules, xa, tl, pitch, y);
+        // The uniform basis is cheap, and its U points overlap; of the others only
+        // the points of the line are worked through (64 points of 16 lines are one
+        // of the U that a thread takes).  A wave's first lane holds its first point.
+        int const live = (last - __builtin_amdgcn_readfirstlane(i)) / ROWS + 1;
+        live_values<D, ORDER, KIND, U, G>(bl, knots, rules, xa, live, tl, pitch, y);
 #pragma unroll
-        for (int u = 0; u < U; ++u) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
+        for (int u = 0; u < U; ++u)
+            if (G == U || u / G * G < live) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
 #pragma unroll
         for (int u = 0; u < U; ++u) xa[u] = xb[u];
     }
