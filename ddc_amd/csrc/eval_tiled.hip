@@ -193,12 +193,16 @@ __global__ void __launch_bounds__(NT) eval_stream_kernel(BSplinesView b, Rules1D
 // rows in flight, and the basis of the kernel's kind alone needs 96 registers
 // where the run-time choice spilled for quintic splines.  us, before -> after:
 // uniform quintic 1024 x 65536 999 -> 842 (rows contiguous 777 -> 621), cubic 60000
-// lines 676 -> 621 (623 -> 492; a form with one 16-line LDS tile and two passes
-// over the points took 656), non-uniform cubic 1024 x 65536 1086 -> 882 (932 ->
-// 677), quintic 1266 -> 1001 (1207 -> 884).  256 threads when lines are short (up
-// to 384 points; 8 lines of 100 points do not fill 1024 threads) and the batch is
-// not: 100 x 90001 196 -> 129 (197 -> 87), 300 x 90001 quintic 540 -> 397 (410 ->
-// 269); 500 x 60000 340 on 1024 threads, 359 on 256; 300 x 1000 8.9 and 10.8.
+// lines 676 -> 621 (623 -> 492), non-uniform cubic 1024 x 65536 1086 -> 877 (932 ->
+// 697), quintic 1266 -> 1081 (1207 -> 884).
+//
+// Threads by the number of tiles that a CU's LDS holds, in batches of more than a
+// tile per CU: 1024 where one fits, 512 for two and three, 256 for four and more
+// in batches of four tiles per CU.  us on 256, 512 and 1024 threads, uniform cubic:
+// 60 cells, 64 points x 65536 31, 43, 70; 150 cells, 384 x 20000 44, 48, 58; 300
+// cells, 384 x 16384 44, 43, 51; 500 cells, 600 x 60000 398, 329, 357; 1024 cells,
+// 100 x 65536 453, 370, 373 and 1024 x 65536 1101, 818, 814; one tile per CU, 300
+// cells, 600 x 1000 16, 12, 11.
 template <int D, int LB, int NT, int KIND>
 __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rules1D rules,
                                                             const double* __restrict__ coords,
@@ -303,6 +307,91 @@ __global__ void __launch_bounds__(NT) eval_vjp_tiled_kernel(BSplinesView b, Rule
     if (active) {
         for (int r = prow; r < ncoef; r += ROWS) gcoef[cb + int64_t(r) * cl.rs] = gt[r * pitch + ln];
     }
+}
+
+// The adjoint on 16-line tiles of batch-contiguous arrays, with one LDS tile used
+// twice: first the coefficients, for gx = w f'(x) over all the tile's points; then
+// the coefficient gradient, accumulated over the same points read again and
+// written once.  Same arithmetic per point as eval_vjp_tiled_kernel.
+//
+// Against the 8-line tiles it halves the number of runs and works out the basis
+// twice, so it pays for uniform bases up to degree 3 where a CU holds only one of
+// those tiles and the coefficients outweigh the points, or the rows lie a large
+// power of two apart, which makes the runs dearer.  us, 8-line tiles and here,
+// cubic: 1024 cells x 65536, 100 points 373 and 294, 1024 points 814 and 791; 700
+// cells x 16384, 384 points 109 and 95; x 60000 (no power of two), 200 points of
+// 1024 cells 342 and 310, 1024 points 621 and 664.
+template <int D, int LB, int NT>
+__global__ void __launch_bounds__(NT) eval_vjp_2pass_kernel(BSplinesView b, Rules1D rules,
+                                                            const double* __restrict__ coords,
+                                                            const double* __restrict__ w, double* __restrict__ gx,
+                                                            Layout pl, int64_t npts, const double* __restrict__ coef,
+                                                            double* __restrict__ gcoef, Layout cl, int64_t nbatch,
+                                                            int ncoef, int pitch)
+{
+    extern __shared__ double smem[];
+    double* tile = smem;
+    constexpr int ROWS = NT / LB;
+    constexpr int U = 4;
+    int const tid = threadIdx.x;
+    int const ln = tid % LB;
+    int const prow = tid / LB;
+    int64_t const line0 = int64_t(blockIdx.x) * LB;
+    int64_t const line = line0 + ln;
+    bool const active = line < nbatch;
+    int64_t const lc = active ? line : 0;
+    int64_t const cb = lay(cl, 0, lc);
+    int64_t const pb = lay(pl, 0, lc);
+    load_tile<LB, NT, 16>(tile, pitch, coef + cb, cl.rs, ncoef, ln, prow);
+    __syncthreads();
+    double* tl = tile + ln;
+    // every point of the line, U at a time: put(point, x, w, evaluated, rule applied)
+    auto points = [&](auto put) {
+        if (!active) return;
+        for (int64_t i = prow; i < npts; i += U * ROWS) {
+            double xa[U], wa[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                int64_t const ii = i + int64_t(u) * ROWS;
+                xa[u] = ii < npts ? coords[pb + ii * pl.rs] : 0.0;
+                wa[u] = ii < npts ? w[pb + ii * pl.rs] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                int64_t const ii = i + int64_t(u) * ROWS;
+                if (ii >= npts) continue;
+                double x = xa[u];
+                bool outside;
+                bool const in = apply_bc(b, rules, x, outside);
+                put(ii, x, wa[u], in, outside);
+            }
+        }
+    };
+    points([&](int64_t ii, double x, double wv, bool in, bool outside) {
+        if (!in) {
+            gx[pb + ii * pl.rs] = 0.0;
+            return;
+        }
+        double v[D + 1], dv[D + 1];
+        int const jmin = basis_and_deriv<D, kUniformBasis>(b, nullptr, x, 0, v, dv);
+        double dy = 0.0;
+#pragma unroll
+        for (int k = 0; k < D + 1; ++k) dy += tl[(jmin + k) * pitch] * dv[k];
+        gx[pb + ii * pl.rs] = outside ? 0.0 : wv * dy;
+    });
+    __syncthreads();
+    for (int k = tid; k < ncoef * pitch; k += NT) tile[k] = 0.0;
+    __syncthreads();
+    points([&](int64_t, double x, double wv, bool in, bool) {
+        if (!in) return;
+        double v[D + 1], dv[D + 1];
+        int const jmin = basis_and_deriv<D, kUniformBasis>(b, nullptr, x, 0, v, dv);
+#pragma unroll
+        for (int k = 0; k < D + 1; ++k) atomicAdd(&tl[(jmin + k) * pitch], wv * v[k]);
+    });
+    __syncthreads();
+    if (active)
+        for (int r = prow; r < ncoef; r += ROWS) gcoef[cb + int64_t(r) * cl.rs] = tile[r * pitch + ln];
 }
 
 // eval_stream_kernel for the value form and the first derivative (up to degree
@@ -471,6 +560,26 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
     else return false;
     bool const line_major = pl.rs == 1;
     bool launched = false;
+    int64_t const cus = cu_count();
+    int const resident = int(kMaxLds / lds_of(pitch)); // 8-line tiles that a CU's LDS holds
+    // (the rules below: figures at the kernels)
+    int const lds2 = ncoef * 17 * int(sizeof(double));
+    if (!line_major && resident == 1 && nbatch >= 32 * cus && b.uniform && b.degree <= 3 && lds2 <= int(kMaxLds) &&
+        (4 * npts <= ncoef || (pl.rs % 8192 == 0 && npts <= ncoef))) {
+        dispatch_degree(b.degree, [&]<int D>() {
+            if constexpr (D <= 3) {
+                auto kern = eval_vjp_2pass_kernel<D, 16, 1024>;
+                hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds2),
+                          "hipFuncSetAttribute");
+                hipLaunchKernelGGL(kern, dim3(unsigned((nbatch + 15) / 16)), dim3(1024), lds2, stream, b, rules,
+                                   coords, w, gx, pl, npts, coef, gcoef, cl, nbatch, ncoef, 17);
+                hip_check(hipGetLastError(), "eval_vjp_2pass_kernel launch");
+                launched = true;
+            }
+        });
+        if (launched) return true;
+    }
     dispatch_degree(b.degree, [&]<int D>() {
         auto go = [&]<int NT>() {
             constexpr int LB = 8;
@@ -486,7 +595,8 @@ bool launch_eval_vjp_tiled(BSplinesPlan const& bs, Rules1D rules, const double* 
             hip_check(hipGetLastError(), "eval_vjp_tiled_kernel launch");
             launched = true;
         };
-        if (npts <= 384 && nbatch > 8 * int64_t(cu_count())) go.template operator()<256>();
+        if (nbatch >= 32 * cus && resident >= 4) go.template operator()<256>();
+        else if (nbatch > 8 * cus && resident >= 2) go.template operator()<512>();
         else go.template operator()<1024>();
     });
     return launched;
