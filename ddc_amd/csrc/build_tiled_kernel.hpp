@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     int const tid = threadIdx.x;
     int ln = tid % LB;
     int seg = tid / LB;
-    int64_t line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    int64_t line0 = tile_of<LB>(blockIdx.x, nbatch) * LB;
     if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int r0 = seg * L;
     int const nq = tv.nq;

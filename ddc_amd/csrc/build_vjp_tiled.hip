@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     int const tid = threadIdx.x;
     int const ln = tid % LB;
     int const seg = tid / LB;
-    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, nbatch) * LB;
     if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;

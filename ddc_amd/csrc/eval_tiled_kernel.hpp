@@ -162,7 +162,7 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
     int const tid = threadIdx.x;
     int const ln = line_major ? tid / ROWS : tid % LB;
     int const prow = line_major ? tid % ROWS : tid / LB;
-    int64_t const line0 = tile_of<LB>(blockIdx.x, gridDim.x) * LB;
+    int64_t const line0 = tile_of<LB>(blockIdx.x, nbatch) * LB;
     if (LB < 16 && line0 >= nbatch) return; // whole workgroup
     int64_t const line = line0 + ln;
     bool const active = line < nbatch;
