@@ -17,14 +17,22 @@
 //    198 -> 167, 600 x 60000 241 -> 166, 1024 x 65536 322 -> 290; non-uniform 700
 //    x 60001 369 -> 248; where two 8-line tiles do not fit a CU 4 lines: non-
 //    uniform 1024 x 65536 443 -> 421 (517 on 8 lines), 2000 x 20000 200 -> 168;
-//  - batch-contiguous, up to 512 points: 64 x 65536 122 -> 82, 256 x 65536 140 ->
-//    105, 512 x 65536 200 -> 191, non-uniform 266 -> 244.  Above, the streaming
-//    kernel is faster (1024 x 65536 357, here 500), unless the batch has too few
-//    tiles for it (600 x 12000 quartic 57 -> 48) or the rows do not start at
-//    128-byte lines, where 16-line runs straddle two (600 x 60001 451 -> 374, 1000
-//    x 60001 736 -> 699, non-uniform 751 -> 657);
-//  - except uniform bases with more than 400 points in batches of one 16-line
-//    tile per CU: 500 x 4000 11.8, here 14.4.
+//  - batch-contiguous, up to 512 points (128 where the streaming kernel takes a
+//    non-uniform basis): 64 x 65536 122 -> 82, 256 x 65536 140 -> 105, 512 x 65536
+//    200 -> 191; random mesh, 300 cells and 300 points x 65536 160, here 191.
+//    Above, the streaming kernel is faster (1024 x 65536 357, here 500), and with
+//    more cells than points already there (1000 cells, 300 points x 65536 201, here
+//    236; x 16384 54, here 49);
+//  - batch-contiguous, too few tiles for the streaming kernel: random mesh, 300
+//    cells, 1000 points x 5008 50 -> 39; uniform 33 -> 31, but x 8000 37, here 47;
+//  - rows that do not start at 128-byte lines, where 16-line runs straddle two, up
+//    to 1024 points (600 x 60001 451 -> 374, 1000 x 60001 736 -> 699, non-uniform 751
+//    -> 657; 3000 points of 1000 cells x 32769 1030, here 1123), and not for a few
+//    points of long lines (100 points of 1024 cells x 65541 270, here 317);
+//  - except uniform bases with more than 256 points in batches of one 16-line
+//    tile per CU (500 x 4000 11.8, here 14.4; 300 points of 1000 cells x 4096 16.1
+//    and 18.6), and 4 lines for many points of uniform bases (2000 cells, 6000
+//    points x 1024 60, here 65).
 #include "eval_tiled_kernel.hpp"
 
 namespace ddcx {
@@ -39,13 +47,21 @@ bool launch_eval_narrow(BSplinesPlan const& bs, Rules1D rules, int order, double
     // LDS of a tile with the given (odd) pitch
     auto lds = [&](int pitch) { return size_t(bs.size()) * pitch * sizeof(double) + extra; };
     int64_t const cus = cu_count();
+    bool const uniform = bs.view.uniform, rows = pl.rs == 1, aligned = pl.rs % 16 == 0;
     bool const two = lds(9) <= tiled::kMaxLds / 2;
+    // where not even an 8-line tile holds the line and its knots, a few lines
+    // are spread over all CUs by the per-point kernel
+    if (!uniform && lds(8) > tiled::kMaxLds && nbatch < 2 * cus) return false;
     int lines = 0;
-    if (nbatch <= 4 * cus) lines = 4;
-    else if (nbatch <= 8 * cus) lines = 8;
-    else if (pl.rs == 1) lines = two ? 8 : 4;
-    else if (bs.view.uniform && nbatch <= 16 * cus && npts > 400) lines = 0;
-    else if (pl.rs % 16 != 0 || (two && (npts <= 512 || nbatch < 32 * cus))) lines = 8;
+    if (nbatch <= 4 * cus) lines = rows || !uniform || npts <= 4096 ? 4 : 0;
+    else if (nbatch <= 8 * cus) lines = rows && !two ? 4 : 8;
+    else if (rows) lines = two ? 8 : 4;
+    else if (uniform && nbatch <= 16 * cus && npts > 256) lines = 0;
+    else if (!aligned) lines = npts <= 1024 && (two || 4 * npts >= bs.size()) ? 8 : 0;
+    else if (two && nbatch < 32 * cus) lines = !uniform || npts <= 512 || (npts <= 1024 && nbatch < 24 * cus) ? 8 : 0;
+    else if (two) // the streaming kernel, up to degree 3 for non-uniform bases, is the other choice
+        lines = uniform ? (npts <= 512 && (bs.size() <= 520 || nbatch < 128 * cus) ? 8 : 0)
+                        : npts <= (degree <= 3 ? 128 : 512) ? 8 : 0;
     if (lines == 0 || lds(lines + 1) > tiled::kMaxLds) return false;
     auto go = [&]<int D, int ORDER>() {
         if (lines == 4)
