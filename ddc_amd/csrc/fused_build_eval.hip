@@ -15,7 +15,7 @@ namespace {
 
 using namespace tiled;
 
-template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int D>
+template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int D, bool MLDS>
 __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv, BuildView bv, BSplinesView b,
                                                                 Rules1D rules, const double* __restrict__ vals,
                                                                 Layout vl, const double* __restrict__ dl,
@@ -31,14 +31,14 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     constexpr int NT = LB * K;
     constexpr int ROWS = NT / LB; // point rows per pass (= K)
     constexpr int U = 8;
-    constexpr bool MLDS = transfer_in_lds(LB);
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
     __shared__ double b2s[kNbMax][LB];
-    __shared__ double x2s[kNbMax][LB];
-    __shared__ BorderLds bl;
-    // row table and Q^-1 gamma blocks during the build, coefficient
-    // tile (size x LB) after
+    // the border's solution, in the space of the sweeps' exchange (over when it is
+    // written); K >= kNbMax
+    double(*const x2s)[LB] = ex[0];
+    // row table, Q^-1 gamma blocks, segment transfer products (MLDS) and border
+    // data during the build, coefficient tile (size x LB) after
     extern __shared__ double dyn[];
 
     int const tid = threadIdx.x;
@@ -79,7 +79,8 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
         b2 = rhs_src(bv, vals, vl, vb, dl, dr, dlay, lay(dlay, 0, lc), seg < tv.top ? seg : tv.nq + seg);
     SegBorder const sb = tv.seg[seg];
     double* const gpad = dyn + K * L * RS;
-    double* const mtr = gpad + tv.ngb * L * tv.nb; // segment transfer products (MLDS)
+    double* const mtr = gpad + tv.ngb * L * tv.nb;
+    BorderLds& bl = *reinterpret_cast<BorderLds*>(mtr + (MLDS ? K * (tv.wf * KF * KF + tv.wb * KB * KB) : 0));
     {
         stage_table<NT, K * L, RS>(tv.rt, dyn, tid);
         if constexpr (MLDS) stage_transfer<NT>(tv, mtr, tid);
@@ -175,7 +176,7 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     }
 }
 
-template <int K, int NT, int KF, int KB, bool FDIV, bool BDIVF, int D>
+template <int K, int NT, bool MLDS, int KF, int KB, bool FDIV, bool BDIVF, int D>
 void launch_one(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double* coef, Layout cl,
                 const double* vals, Layout vl, const double* dl, const double* dr, Layout dlay, double* out,
                 const double* coords, Layout pl, int64_t npts, int64_t nbatch, hipStream_t stream, size_t lds,
@@ -184,7 +185,7 @@ void launch_one(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, doub
     if (p.tiled_f.rs != KF + KB + 1 + (FDIV ? 1 : 0))
         throw Error(DDCX_ERR_INVALID, "row table record length does not match the band shape");
     constexpr int LB = NT / K, L = 16;
-    auto kern = fused_build_eval_kernel<LB, K, L, KF, KB, FDIV, BDIVF, D>;
+    auto kern = fused_build_eval_kernel<LB, K, L, KF, KB, FDIV, BDIVF, D, MLDS>;
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   int(lds)),
               "hipFuncSetAttribute");
@@ -193,7 +194,7 @@ void launch_one(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, doub
     hip_check(hipGetLastError(), "fused_build_eval_kernel launch");
 }
 
-template <int K, int NT = 1024>
+template <int K, int NT, bool MLDS>
 bool launch_K(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double* coef, Layout cl,
               const double* vals, Layout vl, const double* dl, const double* dr, Layout dlay, double* out,
               const double* coords, Layout pl, int64_t npts, int64_t nbatch, hipStream_t stream, size_t lds,
@@ -204,7 +205,7 @@ bool launch_K(BuilderPlan const& p, BSplinesView const& b, Rules1D rules, double
     bool done = false;
     auto go = [&]<int KF, int KB, bool FD, bool BD, int D>() {
         if (!done && deg == D) {
-            launch_one<K, NT, KF, KB, FD, BD, D>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl,
+            launch_one<K, NT, MLDS, KF, KB, FD, BD, D>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl,
                                             npts, nbatch, stream, lds, fpts, fshift);
             done = true;
         }
@@ -249,29 +250,40 @@ bool launch_build_eval_fused(BuilderPlan const& p, BSplinesPlan const& bs, Rules
     if (!offsets_fit(vl, int64_t(K) * L + p.tview_f.q0, nbatch)) return false;
     BSplinesView const b = bs.device_view();
     int const KE = std::max(t.kf, t.kb);
-    // LDS of a workgroup of LB lines: the row table and Q^-1 gamma blocks (and
-    // the transfer products) during the build, then the coefficient tile; 0
-    // when it does not fit
+    // LDS of a workgroup of LB lines: the tables of the build, then the
+    // coefficient tile; 0 when it does not fit
     auto lds_of = [&](int LB, bool transfer) {
         size_t const table = (size_t(K) * L * t.rs + gamma_lds_doubles(p.tview_f) +
                               (transfer ? transfer_doubles(p.tview_f) : 0)) *
-                             sizeof(double);
+                                 sizeof(double) +
+                             sizeof(BorderLds);
         size_t const lds = std::max(table, size_t(bs.size()) * LB * sizeof(double));
-        size_t const stat = size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+        size_t const stat = size_t(KE * K * LB + kLamMax * LB + kNbMax * LB) * sizeof(double);
         return lds + stat > size_t(160 * 1024) ? size_t(0) : lds;
     };
-    auto go = [&]<int KK, int NT>() {
-        size_t const lds = lds_of(NT / KK, transfer_in_lds(NT / KK));
-        return lds > 0 && launch_K<KK, NT>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl, npts,
-                                           nbatch, stream, lds, fpts, feet_shift);
+    auto go = [&]<int KK, int NT, bool MLDS>() {
+        size_t const lds = lds_of(NT / KK, MLDS);
+        return lds > 0 && launch_K<KK, NT, MLDS>(p, b, rules, coef, cl, vals, vl, dl, dr, dlay, out, coords, pl, npts,
+                                                 nbatch, stream, lds, fpts, feet_shift);
     };
+    // Bases whose widest tile does not fit (non-uniform quintic from 944 cells)
+    // take the two kernels where a build and an evaluation can follow each other:
+    // few lines of many points are evaluated faster there (1000 cells, 3000 points x
+    // 3 lines 30 us, 4-line tiles here 76).  Otherwise the narrower tiles do.
+    bool const widest = lds_of(1024 / K, false) > 0;
+    if (!widest && coef && !feet_shift) return false;
     // small batches (build_tiled_small.hip), 4 or 8 lines per workgroup: an
     // advection step of uniform cubic 512 cells x 1000 lines takes 15.5 us on 4
     // lines, 15.9 on 8 and 19.0 on 16; x 2000 lines 20.1, 16.3 and 18.9;
     // 1000 cells x 256 lines 18.2, 19.6 and 25.0
-    if (K == 64 && 2 * nbatch <= 8 * int64_t(cu_count()) && go.template operator()<64, 256>()) return true;
-    if (K == 64 && small_batch(nbatch, 1) && go.template operator()<64, 512>()) return true;
-    return K == 64 ? go.template operator()<64, 1024>() : go.template operator()<128, 1024>();
+    if (K == 64) {
+        bool const four = 2 * nbatch <= 8 * int64_t(cu_count()), eight = small_batch(nbatch, 1);
+        return (four && go.template operator()<64, 256, true>()) ||
+               ((eight || !widest) && go.template operator()<64, 512, true>()) ||
+               go.template operator()<64, 1024, false>() || (!widest && go.template operator()<64, 256, true>());
+    }
+    // the transfer products in LDS where they fit (not for non-uniform quartic splines)
+    return go.template operator()<128, 1024, true>() || go.template operator()<128, 1024, false>();
 }
 
 } // namespace ddcx
