@@ -53,7 +53,7 @@ __global__ void __launch_bounds__(LB* K) build_refine_kernel(RefineView rv, Buil
     __shared__ double e2s[kNbMax][LB]; // border correction of the current solve (scaled)
     __shared__ double x2s[kNbMax][LB]; // border solution
     __shared__ int lexp[LB];
-    extern __shared__ float rt32_lds[];
+    alignas(16) extern __shared__ float rt32_lds[];
 
     int const tid = threadIdx.x;
     int const ln = tid % LB;

@@ -47,7 +47,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
     __shared__ double b2s[kNbMax][LB];
     __shared__ double x2s[kNbMax][LB];
     __shared__ BorderLds bl;
-    extern __shared__ double rt_lds[];
+    alignas(16) extern __shared__ double rt_lds[];
 
     int const tid = threadIdx.x;
     int const ln = tid % LB;

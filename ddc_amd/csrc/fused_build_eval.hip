@@ -39,7 +39,7 @@ __global__ void __launch_bounds__(LB* K, 4) fused_build_eval_kernel(TiledView tv
     double(*const x2s)[LB] = ex[0];
     // row table, Q^-1 gamma blocks, segment transfer products (MLDS) and border
     // data during the build, coefficient tile (size x LB) after
-    extern __shared__ double dyn[];
+    alignas(16) extern __shared__ double dyn[];
 
     int const tid = threadIdx.x;
     int const ln = tid % LB;

@@ -25,8 +25,9 @@ __device__ __forceinline__ void chunk_fence(int i)
 // The border data that a workgroup reads after its sweeps, copied to LDS in
 // its prologue so that the border step waits on no global load: the lambda
 // couplings in their groups, the inverse of the Schur complement, and (in
-// dynamic LDS) the Q^-1 gamma blocks.
-struct BorderLds {
+// dynamic LDS) the Q^-1 gamma blocks.  16-byte aligned like the dynamic LDS behind
+// it: the row table is copied there two doubles at a time.
+struct alignas(16) BorderLds {
     int i[kLamMax];
     int p[kLamMax + 1];
     double v[kLamMax];
