@@ -40,10 +40,22 @@ using namespace tiled;
 // those keep a workgroup per tile.
 constexpr bool loops(int L, bool ic, int tmode) { return L == 32 && !ic && tmode == 1; }
 
+// Wavefronts per SIMD to allocate registers for.  The batch-contiguous kernel
+// of 129-256 rows in 1024 threads needs 64 to 66 registers up to three
+// multipliers: held to 64 (the degree-6 forms move 4-9 of them around the
+// border step), two workgroups share a CU.  At 66, one did: 224 x 28542 of
+// degree 6 took 86 us against 67, 203 x 65536 quartic 151 against 115.  All
+// others have 128 registers.
+constexpr int waves_per_simd(int lb, int k, int l, int kf, bool ic)
+{
+    return lb == 32 && k == 32 && l == 8 && kf <= 3 && !ic ? 8 : 4;
+}
+
 // TMODE: 0 row table read from global memory (L2), 1 staged in LDS whole,
 // 2 staged in LDS one sweep's fields at a time (tables too large for 1)
 template <int LB, int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int TMODE, bool IC>
-__global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, BuildView bv,
+__global__ void __launch_bounds__(LB* K, waves_per_simd(LB, K, L, KF, IC))
+                build_tiled_kernel(TiledView tv, BuildView bv,
                                                            const double* __restrict__ vals, Layout vl,
                                                            const double* __restrict__ dl,
                                                            const double* __restrict__ dr, Layout dlay,
@@ -59,7 +71,9 @@ __global__ void __launch_bounds__(LB* K, 4) build_tiled_kernel(TiledView tv, Bui
     __shared__ double ex[KE][K][LB];
     __shared__ double lamx[kLamMax][LB];
     __shared__ double b2s[kNbMax][LB];
-    __shared__ double x2s[kNbMax][LB];
+    // the border's solution, in the space of the sweeps' exchange (over when it is
+    // written, and begun again behind a barrier); K >= kNbMax
+    double(*const x2s)[LB] = ex[0];
     __shared__ BorderLds bl;
     alignas(16) extern __shared__ double rt_lds[];
 
@@ -305,7 +319,7 @@ bool launch_cfg(BuilderPlan const& p, TiledView const& tv, double* coef, Layout 
     constexpr int LB = NT / K;
     constexpr int KE = KF > KB ? KF : KB;
     constexpr size_t static_lds =
-        size_t(KE * K * LB + kLamMax * LB + 2 * kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
+        size_t(KE * K * LB + kLamMax * LB + kNbMax * LB) * sizeof(double) + sizeof(BorderLds);
     bool const ic = vl.rs == 1 && cl.rs == 1;
     size_t const stage = ic ? size_t(LB) * stage_pitch(K * L, LB) * sizeof(double) : 0;
     size_t const off = ic ? 2 * LB * sizeof(uint32_t) : 0;

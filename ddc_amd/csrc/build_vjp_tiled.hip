@@ -211,8 +211,7 @@ __global__ void __launch_bounds__(LB* K, 4) build_vjp_tiled_kernel(TiledView tv,
         for (int i = 0; i < L; ++i)
             if ((sb.mask >> i) & 1u) {
                 int const g = sb.slot0 + __popc(sb.mask & ((1u << i) - 1u));
-                int const z1 = bl.p[g + 1];
-                for (int z = bl.p[g]; z < z1; ++z) y[i] = fma(-bl.v[z], x2s[bl.i[z]][ln], y[i]);
+                for (int j = 0; j < nb; ++j) y[i] = fma(-bl.m[g * nb + j], x2s[j][ln], y[i]);
             }
     }
 

@@ -646,9 +646,8 @@ void BuilderPlan::upload()
     SolveView const& sv = view.sv;
     int const nb = prob.nb();
     size_t const at_points = pack.add(points);
-    size_t const slot = pack.add(border.slot), rowp = pack.add(border.rowp), val = pack.add(border.val),
-                 crow = pack.add(border.crow), colp = pack.add(border.colp), cval = pack.add(border.cval),
-                 sinv = pack.add(border.sinv), sinvt = pack.add(border.sinvt);
+    size_t const sinvlam = pack.add(border.sinvlam), lamt = pack.add(border.lamt), sinv = pack.add(border.sinv),
+                 sinvt = pack.add(border.sinvt);
     struct Places {
         size_t Mf, Mb, rt, seg, Gblk;
     };
@@ -688,11 +687,8 @@ void BuilderPlan::upload()
         tv.Mb = pack.at<double>(at.Mb);
         tv.seg = pack.at<SegBorder>(at.seg);
         tv.Gblk = pack.at<double>(at.Gblk);
-        tv.nnz = int(border.val.size());
-        tv.ngroup = transpose ? int(border.cols.size()) : nb;
-        tv.bi = pack.at<int>(transpose ? crow : slot);
-        tv.bv = pack.at<double>(transpose ? cval : val);
-        tv.bp = pack.at<int>(transpose ? colp : rowp);
+        tv.ncols = int(border.cols.size());
+        tv.bm = pack.at<double>(transpose ? lamt : sinvlam);
         tv.sinv = pack.at<double>(transpose ? sinvt : sinv);
     };
     view_of(tiled, p, false, tview);

@@ -264,14 +264,10 @@ struct TiledView {
     const double* Mb;
     const SegBorder* seg; // K
     const double* Gblk;
-    // the lambda couplings grouped for the border step: group g holds
-    // couplings bp[g] .. bp[g + 1] - 1.  The solve groups them by border row
-    // (ngroup = nb; bi = slot of the coupled column), the adjoint by coupled
-    // column (ngroup = number of slots; bi = border row).
-    int nnz, ngroup;
-    const int* bi;
-    const double* bv;
-    const int* bp;
+    // the border step's matrix: S^-1 lambda (nb x ncols, a column per slot) for
+    // the solve, lambda^T (ncols x nb) for the adjoint
+    int ncols;
+    const double* bm;
     const double* sinv; // inverse of the Schur complement (transposed for the adjoint), nb x nb
 };
 
@@ -327,13 +323,14 @@ struct RefineView {
 // The border data of the tiled kernels that does not depend on the tiling.
 // The Schur systems are nb x nb with nb <= 8: x2 = S^-1 b2 as a product with
 // the inverse (columns solved with the LU factors at plan creation) has no
-// serial chain and no division, unlike the substitutions.
+// serial chain and no division, unlike the substitutions.  Lambda is kept
+// dense over the coupled columns, times S^-1 for the build: a few more
+// products than nonzeros, and none of them waits for an index read.
 struct BorderHost {
-    std::vector<int> cols;              // distinct coupled columns of lambda, increasing
-    std::vector<int> slot, rowp;        // couplings by border row: slot of the column, row starts
-    std::vector<int> crow, colp;        // couplings by column: border row, column starts
-    std::vector<double> val, cval;      // values in either order
-    std::vector<double> sinv, sinvt;    // S^-1 and its transpose, row-major
+    std::vector<int> cols;           // distinct coupled columns of lambda, increasing
+    std::vector<double> sinvlam;     // S^-1 lambda, nb x cols
+    std::vector<double> lamt;        // lambda^T, cols x nb
+    std::vector<double> sinv, sinvt; // S^-1 and its transpose, row-major
 };
 
 struct BuilderPlan {

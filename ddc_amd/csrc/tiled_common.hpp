@@ -23,25 +23,19 @@ __device__ __forceinline__ void chunk_fence(int i)
 }
 
 // The border data that a workgroup reads after its sweeps, copied to LDS in
-// its prologue so that the border step waits on no global load: the lambda
-// couplings in their groups, the inverse of the Schur complement, and (in
-// dynamic LDS) the Q^-1 gamma blocks.  16-byte aligned like the dynamic LDS behind
-// it: the row table is copied there two doubles at a time.
+// its prologue so that the border step waits on no global load: the border
+// step's matrix, the inverse of the Schur complement, and (in dynamic LDS) the
+// Q^-1 gamma blocks.  16-byte aligned like the dynamic LDS behind it: the row table
+// is copied there two doubles at a time.
 struct alignas(16) BorderLds {
-    int i[kLamMax];
-    int p[kLamMax + 1];
-    double v[kLamMax];
+    double m[kLamMax];
     double sinv[kNbMax * kNbMax];
 };
 
 template <int NT, bool GAMMA>
 __device__ __forceinline__ void stage_border(TiledView const& tv, BorderLds& bl, double* gpad, int tid)
 {
-    for (int k = tid; k < tv.nnz; k += NT) {
-        bl.i[k] = tv.bi[k];
-        bl.v[k] = tv.bv[k];
-    }
-    for (int k = tid; k < tv.ngroup + 1; k += NT) bl.p[k] = tv.bp[k];
+    for (int k = tid; k < tv.nb * tv.ncols; k += NT) bl.m[k] = tv.bm[k];
     for (int k = tid; k < tv.nb * tv.nb; k += NT) bl.sinv[k] = tv.sinv[k];
     if constexpr (GAMMA) {
         int const n = tv.ngb * tv.L * tv.nb;
@@ -64,20 +58,20 @@ __device__ __forceinline__ void gather_coupled(double const (&y)[L], SegBorder c
     }
 }
 
-// Row k of x2 = S^-1 (b2 - lambda y) for one line: every border row's thread
-// computes the whole right-hand side (nb <= 8 rows of a few couplings, from
-// LDS) and its own row of the product, so the rows need no exchange.
+// Row k of x2 = S^-1 b2 - (S^-1 lambda) y for one line: two short products of
+// independent reads, so the rows need no exchange.  (As S^-1 (b2 - lambda y) with
+// the couplings in a list, every thread summed the whole right-hand side through
+// two dependent LDS reads per coupling, and with a border of 4 to 6 rows the
+// others waited: quartic Hermite 203 cells x 65536 139 -> 166 us.)
 template <int LB>
 __device__ __forceinline__ double border_row(TiledView const& tv, BorderLds const& bl, double const (*b2)[LB],
                                              double const (*lamx)[LB], int k, int ln)
 {
     double x = 0.0;
-    for (int j = 0; j < tv.nb; ++j) {
-        double v = b2[j][ln];
-        int const z1 = bl.p[j + 1];
-        for (int z = bl.p[j]; z < z1; ++z) v = fma(-bl.v[z], lamx[bl.i[z]][ln], v);
-        x = fma(bl.sinv[k * tv.nb + j], v, x);
-    }
+#pragma unroll 4
+    for (int j = 0; j < tv.nb; ++j) x = fma(bl.sinv[k * tv.nb + j], b2[j][ln], x);
+#pragma unroll 4
+    for (int s = 0; s < tv.ncols; ++s) x = fma(-bl.m[k * tv.ncols + s], lamx[s][ln], x);
     return x;
 }
 
@@ -87,17 +81,24 @@ __device__ __forceinline__ double border_row(TiledView const& tv, BorderLds cons
 // eight times the multiply-adds, in the segments that the whole workgroup
 // waits for; variants by column count made the compiler keep several copies
 // of y (164 to 179 registers instead of 109 to 125, and spills at 128).
+// Short segments have the registers to read four columns ahead.
 template <int LB, int L>
 __device__ __forceinline__ void apply_gamma(double (&y)[L], const double* G, int nb, double const (*x2s)[LB], int ln)
 {
-    for (int k = 0; k < nb; ++k) {
+    auto column = [&](int k) {
         double const x = x2s[k][ln];
         const double* g = G + k * L;
 #pragma unroll
         for (int i = 0; i < L; ++i) {
             y[i] = fma(-g[i], x, y[i]);
-            chunk_fence(i);
+            if constexpr (L >= 16) chunk_fence(i);
         }
+    };
+    if constexpr (L < 16) {
+#pragma unroll 4
+        for (int k = 0; k < nb; ++k) column(k);
+    } else {
+        for (int k = 0; k < nb; ++k) column(k);
     }
 }
 

@@ -81,7 +81,11 @@ const char* tiled_unsupported(HostProblem const& pr, int min_rows)
     if (nq < min_rows) return "main block too small";
     if (nq > 2048) return "main block larger than 2048 rows";
     if (pr.nb() > kMaxBorderTiled) return "border larger than 8";
-    if (int(pr.bl_v.size()) > kMaxLambda) return "too many border couplings";
+    // coupled columns: at most kMaxLambda entries in the border step's matrix
+    std::vector<int> cols = pr.bl_c;
+    std::sort(cols.begin(), cols.end());
+    cols.erase(std::unique(cols.begin(), cols.end()), cols.end());
+    if (int(pr.bl_v.size()) > kMaxLambda || int(cols.size()) * pr.nb() > kMaxLambda) return "too many border couplings";
     return nullptr;
 }
 
@@ -278,33 +282,28 @@ BorderHost make_border(HostProblem const& pr)
     b.cols = pr.bl_c;
     std::sort(b.cols.begin(), b.cols.end());
     b.cols.erase(std::unique(b.cols.begin(), b.cols.end()), b.cols.end());
-    b.rowp.assign(nb + 1, 0);
-    b.colp.assign(b.cols.size() + 1, 0);
-    // the COO copy is sorted by row; by column the rows stay in order
+    int const nc = int(b.cols.size());
+    b.lamt.assign(size_t(nc) * nb, 0.0);
     for (int z = 0; z < nnz; ++z) {
         int const s = int(std::lower_bound(b.cols.begin(), b.cols.end(), pr.bl_c[z]) - b.cols.begin());
-        b.slot.push_back(s);
-        b.val.push_back(pr.bl_v[z]);
-        ++b.rowp[pr.bl_r[z] + 1];
-        ++b.colp[s + 1];
-    }
-    for (int k = 0; k < nb; ++k) b.rowp[k + 1] += b.rowp[k];
-    for (size_t s = 0; s < b.cols.size(); ++s) b.colp[s + 1] += b.colp[s];
-    b.crow.resize(nnz);
-    b.cval.resize(nnz);
-    std::vector<int> next(b.colp.begin(), b.colp.end());
-    for (int z = 0; z < nnz; ++z) {
-        int const at = next[b.slot[z]]++;
-        b.crow[at] = pr.bl_r[z];
-        b.cval[at] = pr.bl_v[z];
+        b.lamt[size_t(s) * nb + pr.bl_r[z]] += pr.bl_v[z];
     }
     b.sinv.assign(size_t(nb) * nb, 0.0);
     b.sinvt.assign(size_t(nb) * nb, 0.0);
+    auto solve = [&](std::vector<double> e) {
+        if (nb > 0) pr.schur.solve(e.data(), 1, false);
+        return e;
+    };
     for (int j = 0; j < nb; ++j) {
         std::vector<double> e(nb, 0.0);
         e[j] = 1.0;
-        pr.schur.solve(e.data(), 1, false);
+        e = solve(e);
         for (int i = 0; i < nb; ++i) b.sinv[size_t(i) * nb + j] = b.sinvt[size_t(j) * nb + i] = e[i];
+    }
+    b.sinvlam.assign(size_t(nb) * nc, 0.0);
+    for (int s = 0; s < nc; ++s) {
+        auto const e = solve({b.lamt.begin() + size_t(s) * nb, b.lamt.begin() + size_t(s + 1) * nb});
+        for (int i = 0; i < nb; ++i) b.sinvlam[size_t(i) * nc + s] = e[i];
     }
     return b;
 }
