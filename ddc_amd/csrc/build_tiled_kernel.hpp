@@ -33,12 +33,25 @@ using namespace tiled;
 // Long lines in batch-contiguous arrays (the whole table in LDS): one workgroup
 // per resident place walks the tiles, so that the table and border data are
 // staged once, and each row of the next tile is requested as the current one's
-// row is stored.  us, a workgroup per tile -> this: uniform cubic 1024 x 65536
-// 247 -> 241, quintic 302 -> 281, non-uniform cubic 285 -> 271, cubic 300 x 100000
-// 226 -> 209, 512 x 8192 21.8 -> 19.4.  With the table staged in halves (quintic
-// Hermite 2048 x 32768) the staging waits behind the tile's loads: 383 -> 418, so
-// those keep a workgroup per tile.
+// row is stored.  us, a workgroup per tile -> this: cubic 300 x 100000 218 -> 207,
+// non-uniform quintic 1024 x 65536 335 -> 329, 513 x 65536 275 -> 261, 1024 x 20000
+// 135 -> 129, non-uniform cubic 1024 x 20000 86 -> 75.  With the table staged in
+// halves (quintic Hermite 2048 x 32768) the staging waits behind the tile's loads:
+// 383 -> 418, so those keep a workgroup per tile.
 constexpr bool loops(int L, bool ic, int tmode) { return L == 32 && !ic && tmode == 1; }
+
+// The exception, by grid size alone.  With rows a multiple of 8 KiB apart all
+// rows of a tile share few memory channels, and workgroups that walk in step
+// meet there; up to two multipliers that costs long lines more than the staging
+// saves, until there are more than about nq / 128 tiles for each place.  us,
+// walking -> a workgroup per tile: cubic 1024 x 16384 72 -> 61, x 65536 230 -> 220,
+// 2048 x 8192 72 -> 59, non-uniform 1024 x 16384 80 -> 65, quintic 1024 x 16384
+// 83 -> 70, cubic 512 x 16384 42 -> 37; but 1024 x 16400 56 -> 59, 300 x 16384
+// 36 -> 38, 513 x 65536 158 -> 161.
+inline bool walks(int kf, int nq, int64_t vrs, int64_t crs, int64_t tiles, int64_t places)
+{
+    return !(kf <= 2 && nq > 400 && vrs % 1024 == 0 && crs % 1024 == 0 && tiles * 128 <= places * nq);
+}
 
 // Wavefronts per SIMD to allocate registers for.  The batch-contiguous kernel
 // of 129-256 rows in 1024 threads needs 64 to 66 registers up to three
@@ -294,7 +307,7 @@ __global__ void __launch_bounds__(LB* K, waves_per_simd(LB, K, L, KF, IC))
 }
 
 template <int K, int L, int KF, int KB, bool FDIV, bool BDIVF, int TMODE, bool IC, int NT>
-void launch_one(BuilderPlan const& p, TiledView const& tv, size_t lds, double* coef, Layout cl, const double* vals, Layout vl,
+void launch_one(BuilderPlan const& p, TiledView const& tv, size_t static_lds, size_t lds, double* coef, Layout cl, const double* vals, Layout vl,
                 const double* dl, const double* dr, Layout dlay, int64_t nbatch, hipStream_t stream)
 {
     constexpr int LB = NT / K;
@@ -304,7 +317,13 @@ void launch_one(BuilderPlan const& p, TiledView const& tv, size_t lds, double* c
                                       int(lds)),
                   "hipFuncSetAttribute");
     unsigned grid = tile_grid<LB>(nbatch);
-    if (loops(L, IC, TMODE)) grid = std::min(grid, unsigned(cu_count()) * (1024 / NT)); // 128 registers: 1024 threads per CU
+    if (loops(L, IC, TMODE)) {
+        // resident places: 128 registers allow 1024 threads per CU, and the LDS must hold them
+        constexpr size_t cu_lds = 160 * 1024;
+        unsigned const per_cu = std::max<size_t>(1, std::min<size_t>(1024 / NT, cu_lds / (static_lds + lds)));
+        unsigned const places = unsigned(cu_count()) * per_cu;
+        if (walks(KF, tv.nq, vl.rs, cl.rs, grid, places)) grid = std::min(grid, places);
+    }
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NT), lds, stream, tv, p.view, vals, vl, dl, dr, dlay,
                        coef, cl, nbatch);
     hip_check(hipGetLastError(), "build_tiled_kernel launch");
@@ -332,7 +351,7 @@ bool launch_cfg(BuilderPlan const& p, TiledView const& tv, double* coef, Layout 
     int const mode = (static_lds + table <= budget && tv.rs <= 10) ? 1 : static_lds + half <= budget ? 2 : 0;
     size_t const lds = mode == 1 ? table : mode == 2 ? half : stage + off;
     auto go = [&]<int TM, bool I>() {
-        launch_one<K, L, KF, KB, FDIV, BDIVF, TM, I, NT>(p, tv, lds, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
+        launch_one<K, L, KF, KB, FDIV, BDIVF, TM, I, NT>(p, tv, static_lds, lds, coef, cl, vals, vl, dl, dr, dlay, nbatch, stream);
     };
     // the small-batch tiles exist with the whole table in LDS only
     if constexpr (transfer_in_lds(LB)) {
