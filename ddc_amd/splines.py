@@ -102,8 +102,10 @@ def n_boundary_equations(bc, degree):
 
 
 def _stream():
-    # torch.cuda.current_stream().cuda_stream without the Stream object
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    # torch.cuda.current_stream().cuda_stream, where torch has the private
+    # function without the Stream object
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return torch.cuda.current_stream().cuda_stream if raw is None else raw(torch.cuda.current_device())
 
 
 def _ptr(t):

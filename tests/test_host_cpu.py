@@ -279,3 +279,19 @@ def test_linear_problem_host_side():
     q = LP.make_new_dense(3)
     with pytest.raises(DDCXError, match="SINGULAR"):
         q.setup_solver()  # all zeros: dgetrf info > 0
+
+
+def test_stream_without_the_private_function(monkeypatch):
+    """The current stream's handle also where torch lacks the private accessor."""
+    import types
+
+    import torch
+
+    from ddc_amd import splines
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=42))
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert splines._stream() == 42
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 100 + device, raising=False)
+    assert splines._stream() == 103
