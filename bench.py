@@ -151,7 +151,8 @@ def pattern_ceiling(src, dst, lb, timed, n):
     """GB/s of a plain copy of src -> dst ((rows, lines) batch-contiguous
     FP64, same shape) in tiles of lb lines by all rows: the access pattern of
     the tiled kernels, measured by the probe library built beside libddcx
-    (None when it is not built)."""
+    (None when it is not built).  A yardstick: kernels that overlap their loads
+    and stores better than the copy can exceed it."""
     import ctypes
 
     import torch

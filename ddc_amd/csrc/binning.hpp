@@ -1,6 +1,6 @@
 // Binning of scattered evaluation points by cell tile, shared by the binned
 // 2D adjoint (eval2d_binned.hip) and the binned 3D evaluation
-// (eval_nd_binned.hip).  A caller's count pass gives each point a tile (16
+// (eval_nd.hip).  A caller's count pass gives each point a tile (16
 // bits, kNoBin for a point an extrapolation rule settles by itself) and per
 // batch entry and tile a count; then
 //   bin_scan_kernel    turns the counts into tile offsets (starts) and the

@@ -56,10 +56,11 @@ __device__ __forceinline__ void buffer_store(double v, __amdgpu_buffer_rsrc_t r,
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, int(off), 0, AUX);
 }
 
-// Persistent form of eval_tiled_kernel for values with plain batch-contiguous
-// arrays (element (row, line) at row * rs + line, 16-line tiles, NT threads:
-// 512 for uniform bases, 768 for non-uniform ones).  Each workgroup walks the tiles blockIdx.x, blockIdx.x +
-// gridDim.x, ...: while the points of one tile are evaluated, the coefficients
+// Persistent form of eval_tiled_kernel for values and first derivatives with
+// plain batch-contiguous arrays (element (row, line) at row * rs + line, 16-line
+// tiles, NT threads: 512 for uniform bases, 768 for non-uniform ones).  Each
+// workgroup walks the tiles blockIdx.x, blockIdx.x + gridDim.x, ...: while the
+// points of one tile are evaluated, the coefficients
 // of its next tile are loaded into registers (PR rows per thread, one slice per
 // stage of U points), and they go to LDS once the current tile has been read.
 // Coefficient loads, point loads and stores therefore overlap inside every CU

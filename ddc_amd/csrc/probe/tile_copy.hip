@@ -2,8 +2,10 @@
 // persistent copy of a (rows, lines) batch-contiguous FP64 array in tiles of
 // LB lines by all rows, lanes along lines (LB * 8-byte runs per row), rows
 // strided by ld * 8 bytes, non-temporal loads and stores, every element
-// read and written once.  This is the pattern of the tiled spline kernels
-// on batch-contiguous arrays, so its rate bounds theirs.
+// read and written once.  The tiled spline kernels touch batch-contiguous
+// arrays in this pattern; they can run a little faster than this copy, which
+// waits for each batch of rows before it stores them, so its rate is a
+// yardstick and no bound.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
