@@ -17,22 +17,27 @@
 //    198 -> 167, 600 x 60000 241 -> 166, 1024 x 65536 322 -> 290; non-uniform 700
 //    x 60001 369 -> 248; where two 8-line tiles do not fit a CU 4 lines: non-
 //    uniform 1024 x 65536 443 -> 421 (517 on 8 lines), 2000 x 20000 200 -> 168;
-//  - batch-contiguous, up to 512 points (128 where the streaming kernel takes a
-//    non-uniform basis): 64 x 65536 122 -> 82, 256 x 65536 140 -> 105, 512 x 65536
-//    200 -> 191; random mesh, 300 cells and 300 points x 65536 160, here 191.
-//    Above, the streaming kernel is faster (1024 x 65536 357, here 500), and with
-//    more cells than points already there (1000 cells, 300 points x 65536 201, here
-//    236; x 16384 54, here 49);
-//  - batch-contiguous, too few tiles for the streaming kernel: random mesh, 300
-//    cells, 1000 points x 5008 50 -> 39; uniform 33 -> 31, but x 8000 37, here 47;
-//  - rows that do not start at 128-byte lines, where 16-line runs straddle two, up
-//    to 1024 points (600 x 60001 451 -> 374, 1000 x 60001 736 -> 699, non-uniform 751
-//    -> 657; 3000 points of 1000 cells x 32769 1030, here 1123), and not for a few
-//    points of long lines (100 points of 1024 cells x 65541 270, here 317);
-//  - except uniform bases with more than 256 points in batches of one 16-line
-//    tile per CU (500 x 4000 11.8, here 14.4; 300 points of 1000 cells x 4096 16.1
-//    and 18.6), and 4 lines for many points of uniform bases (2000 cells, 6000
-//    points x 1024 60, here 65).
+//    where one 4-line tile fills a CU and there are a few points, 8 lines (uniform,
+//    2125 rows, 100 points x 16384 94 -> 68);
+//  - batch-contiguous, uniform, rows too long for two 8-line tiles: the wide kernel
+//    has 8 or 16 lines on the whole CU there (1757 rows, 200 points x 16384 116 ->
+//    68; 1579 rows, 100 points x 4010 25 -> 18);
+//  - batch-contiguous, uniform, up to 512 points: 64 x 65536 122 -> 82, 256 x 65536
+//    140 -> 105, 512 x 65536 200 -> 191.  Above, the streaming kernel is faster (1024
+//    x 65536 357, here 500), and with more cells than points already there (1000
+//    cells, 300 points x 65536 201, here 236; but 557 cells, 100 points x 32768 75 ->
+//    50).  Up to 1024 where the batch has too few tiles to stream (33 -> 31 for 300
+//    cells, 1000 points x 5008, but x 8000 37, here 47), 256 where it is one 16-line
+//    tile per CU (500 x 4000 11.8, here 14.4);
+//  - batch-contiguous, non-uniform: always above degree 3, which does not stream
+//    (5 to 18% at 512 points and more); up to 256 points below (200 points of as
+//    many cells 1.2 to 1.4 times; 300 points x 65536 160, here 191), and where the
+//    batch is too small to stream (300 cells, 1000 points x 5008 50 -> 39);
+//  - rows that do not start at 128-byte lines, where 16-line runs straddle two:
+//    up to 1024 points (600 x 60001 451 -> 374, 1000 x 60001 736 -> 699, non-uniform
+//    751 -> 657; 3000 points of 1000 cells x 32769 1030, here 1123) or 1.5 a row
+//    (1026 x 16389 207 -> 141), above that non-uniform where the wide kernel does not
+//    stream; not for a few points of long non-uniform lines in a large batch.
 #include "eval_tiled_kernel.hpp"
 
 namespace ddcx {
@@ -48,20 +53,29 @@ bool launch_eval_narrow(BSplinesPlan const& bs, Rules1D rules, int order, double
     auto lds = [&](int pitch) { return size_t(bs.size()) * pitch * sizeof(double) + extra; };
     int64_t const cus = cu_count();
     bool const uniform = bs.view.uniform, rows = pl.rs == 1, aligned = pl.rs % 16 == 0;
-    bool const two = lds(9) <= tiled::kMaxLds / 2;
-    // where not even an 8-line tile holds the line and its knots, a few lines
-    // are spread over all CUs by the per-point kernel
-    if (!uniform && lds(8) > tiled::kMaxLds && nbatch < 2 * cus) return false;
+    bool const two = lds(9) <= tiled::kMaxLds / 2;     // 8-line tiles, two per CU
+    bool const one4 = lds(5) > tiled::kMaxLds / 2;     // 4-line tiles, one per CU
+    bool const few = 4 * npts < bs.size();
+    // where not even an 8-line tile holds the line and its knots, the per-point
+    // kernel spreads a few lines over all CUs, and reads only what a few points need
+    if (!uniform && lds(8) > tiled::kMaxLds && (nbatch < 2 * cus || 16 * npts < bs.size())) return false;
+    auto narrow = [&] { // 8 lines, against the wider kernels
+        if (uniform) {
+            if (!two && lds(17) > tiled::kMaxLds) return true; // the wide kernel has no 16-line tile
+            if (aligned && nbatch <= 16 * cus) return npts <= 256;
+            if (!aligned) return npts <= 1024 || (2 * npts <= 3 * bs.size() && nbatch < 128 * cus);
+            if (nbatch < 32 * cus) return npts <= 512 || (npts <= 1024 && nbatch < 24 * cus);
+            return npts <= 512 && (bs.size() <= (few ? 800 : 520) || nbatch <= 128 * cus);
+        }
+        // the streaming kernel takes non-uniform bases up to degree 3
+        if (lds(16) > tiled::kMaxLds) return few || !aligned;
+        if (!aligned) return (npts <= 1024 || (degree > 3) == two) && (two || !few || nbatch < 128 * cus);
+        return two && (nbatch < 32 * cus || degree > 3 || npts <= 256);
+    };
     int lines = 0;
-    if (nbatch <= 4 * cus) lines = rows || !uniform || npts <= 4096 ? 4 : 0;
-    else if (nbatch <= 8 * cus) lines = rows && !two ? 4 : 8;
-    else if (rows) lines = two ? 8 : 4;
-    else if (uniform && nbatch <= 16 * cus && npts > 256) lines = 0;
-    else if (!aligned) lines = npts <= 1024 && (two || 4 * npts >= bs.size()) ? 8 : 0;
-    else if (two && nbatch < 32 * cus) lines = !uniform || npts <= 512 || (npts <= 1024 && nbatch < 24 * cus) ? 8 : 0;
-    else if (two) // the streaming kernel, up to degree 3 for non-uniform bases, is the other choice
-        lines = uniform ? (npts <= 512 && (bs.size() <= 520 || nbatch < 128 * cus) ? 8 : 0)
-                        : npts <= (degree <= 3 ? 128 : 512) ? 8 : 0;
+    if (nbatch <= 4 * cus) lines = 4;
+    else if (rows || nbatch <= 8 * cus) lines = two || (nbatch <= 8 * cus && !rows) || (few && one4) ? 8 : 4;
+    else if (narrow()) lines = 8;
     if (lines == 0 || lds(lines + 1) > tiled::kMaxLds) return false;
     auto go = [&]<int D, int ORDER>() {
         if (lines == 4)
