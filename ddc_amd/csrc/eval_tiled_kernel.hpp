@@ -99,15 +99,24 @@ __device__ __forceinline__ void point_values(BSplinesView const& b, const double
 
 // point_values in groups of G points, of which `live` (the same number in all
 // lanes of a wave) are points of the line: groups past them are left out, and
-// their y as it was.
+// their y as it was.  Of a first derivative's last group, the points one by one.
 template <int D, int ORDER, int KIND, int U, int G>
 __device__ __forceinline__ void live_values(BSplinesView const& b, const double* kn, Rules1D rules, double (&x)[U],
                                             int live, const double* tile, int pitch, double (&y)[U])
 {
     static_assert(U % G == 0);
 #pragma unroll
-    for (int u = 0; u < U; u += G)
+    for (int u = 0; u < U; u += G) {
+        if constexpr (ORDER == 1 && KIND != kUniformBasis && G > 1) {
+            if (u + G > live) {
+#pragma unroll
+                for (int k = u; k < u + G; ++k)
+                    if (k == 0 || k < live) point_values<D, ORDER, KIND, 1>(b, kn, rules, x + k, tile, pitch, y + k);
+                continue;
+            }
+        }
         if (u == 0 || u < live) point_values<D, ORDER, KIND, G>(b, kn, rules, x + u, tile, pitch, y + u);
+    }
 }
 
 // The coefficient tile of a workgroup's lines to LDS: thread (line ln, row
@@ -139,7 +148,8 @@ __device__ __forceinline__ void load_tile(double* tile, int pitch, const double*
     }
 }
 
-template <int D, int ORDER, int LB, int NT, int KIND>
+// UP: points per thread and stage (0: chosen here).
+template <int D, int ORDER, int LB, int NT, int KIND, int UP = 0>
 __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D rules, double* __restrict__ out,
                                                         const double* __restrict__ coords, Layout xl, Layout pl,
                                                         int64_t npts,
@@ -153,11 +163,13 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
     constexpr int ROWS = NT / LB;
     // points per pipeline stage per thread: as many as the registers hold
     // without spilling (derivative tables of non-uniform bases are the largest)
-    constexpr int U = LB < 16 && NT < 1024 ? 4
-                      : ORDER == 0 || (ORDER == 1 && KIND != kUniformBasis) ? 8
+    constexpr int U = UP > 0 ? UP
+                      : LB < 16 && NT < 1024 ? 4
+                      : ORDER == 0 ? 8
                       : KIND == kUniformBasis ? (D <= 4 ? 8 : 4)
                                               : (D <= 1 ? 8 : (D <= 3 ? 4 : 2));
-    constexpr int G = KIND == kUniformBasis ? U : ORDER == 0 ? 4 : 2; // points worked through together
+    // points worked through together
+    constexpr int G = KIND == kUniformBasis ? U : ORDER == 0 && KIND == kSafeNonUniform ? 4 : ORDER == 1 ? U : 2;
     constexpr int TC = 20;         // tile rows per thread per load chunk (one chunk up to 20 * ROWS rows)
     int const tid = threadIdx.x;
     int const ln = line_major ? tid / ROWS : tid % LB;
@@ -212,7 +224,7 @@ __global__ void __launch_bounds__(NT) eval_tiled_kernel(BSplinesView b, Rules1D 
         live_values<D, ORDER, KIND, U, G>(bl, knots, rules, xa, live, tl, pitch, y);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (G == U || u / G * G < live) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
+            if (KIND == kUniformBasis || (G == U && ORDER != 1) || (ORDER == 1 ? u == 0 || u < live : u / G * G < live)) __builtin_nontemporal_store(y[u], &op[at(i + u * ROWS)]);
 #pragma unroll
         for (int u = 0; u < U; ++u) xa[u] = xb[u];
     }
@@ -227,10 +239,24 @@ void launch_eval_tile(BSplinesPlan const& bs, Rules1D rules, double* out, const 
     int const nknots = bs.view.uniform ? 0 : int(bs.knots_host.size());
     BSplinesView const b = bs.device_view();
     size_t const lds = (size_t(ncoef) * pitch + nknots) * sizeof(double) + size_t(b.nbucket) * sizeof(uint32_t);
+    // First derivatives of non-uniform bases: one point per thread and stage where
+    // threads have only one or two points (64 points of 8192 quintic lines, us for 1
+    // / 2 / 4 points: 12.5 / 17.4 / 23.4), and in batch-contiguous arrays whose rows
+    // do not start at 128-byte lines: the fewer rows of points are in flight there,
+    // the fewer DRAM pages compete (cubic 173 cells, 800 points x 65541: 431 / 574 /
+    // 555), unless the lines are long, the workgroups on a CU few, and each waits
+    // for its own chain (1024 to 1448 rows 1.24, 1.08 of the best).  Otherwise four
+    // (rows contiguous 1024 x 65536 cubic 497 -> 419; 136 lines of 6144 points 54 ->
+    // 38), or two with 1024 threads, four of which would spill.
+    constexpr bool dnu = ORDER == 1;
+    constexpr int many = NT < 1024 ? 4 : 2;
+    bool const ahead = npts > 2 * (NT / LB) &&
+                       (pl.rs % 16 == 0 || pl.rs == 1 || (many == 4 && (ncoef > 700 || nbatch <= 8 * int64_t(cu_count()))));
     auto kern = b.uniform ? eval_tiled_kernel<D, ORDER, LB, NT, kUniformBasis>
                 : ORDER == 0 && bs.safe_products
                     ? eval_tiled_kernel<D, ORDER, LB, NT, ORDER == 0 ? kSafeNonUniform : kNonUniformBasis>
-                    : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis>;
+                : dnu && ahead ? eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis, dnu ? many : 0>
+                               : eval_tiled_kernel<D, ORDER, LB, NT, kNonUniformBasis, dnu ? 1 : 0>;
     hip_check(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                   int(lds)),
               "hipFuncSetAttribute");
