@@ -282,8 +282,13 @@ bool launch_build_eval_fused(BuilderPlan const& p, BSplinesPlan const& bs, Rules
                ((eight || !widest) && go.template operator()<64, 512, true>()) ||
                go.template operator()<64, 1024, false>() || (!widest && go.template operator()<64, 256, true>());
     }
-    // the transfer products in LDS where they fit (not for non-uniform quartic splines)
-    return go.template operator()<128, 1024, true>() || go.template operator()<128, 1024, false>();
+    // the transfer products in LDS where they fit; without them (non-uniform quartic
+    // splines) the two kernels are faster for large batches of many points, where
+    // they can follow each other: 2000 cells and points, us here / two kernels, x
+    // 2048 lines 75 / 79, x 8000 271 / 225; 100 points x 2048 34 / 61
+    if (go.template operator()<128, 1024, true>()) return true;
+    if (coef && !feet_shift && nbatch > 8 * int64_t(cu_count()) && 2 * npts >= bs.size()) return false;
+    return go.template operator()<128, 1024, false>();
 }
 
 } // namespace ddcx
